@@ -1,0 +1,397 @@
+// Projections of middling batches, Y_s[M, N_s] (+)= scale_s[n] X[M, K] W_s[N_s, K]^T for up to four
+// weights sharing X: from 17 rows of X to as many as the 256 x 256 tiles of gemm.hip leave part of
+// the chip idle for. int8 or bf16 W, fp32 or bf16 X, fp32 Y, on v_mfma_f32_16x16x32_bf16.
+//
+// What bounds it: at these sizes neither HBM (an 8192 x 2048 int8 weight is 17 MB, 3 us) nor the
+// matrix cores, but how much of the chip a tile split fills and what every workgroup pulls through
+// L2 (about 16 TB/s in all) and converts. So the tile varies: a workgroup is KG groups of NWN
+// waves; wave (kg, wn) owns 16 RT rows of W against 16 MT rows of X over every KG-th 64-k step, and
+// the groups' partial tiles are added in LDS in group order (deterministic, no workspace). W goes
+// from global memory straight to MFMA operands in registers (each weight byte is read and converted
+// once per workgroup, PD steps ahead); X goes through registers into LDS as bf16 hi (and, for fp32 X,
+// lo) parts, split once per workgroup instead of once per wave and W row tile, double-buffered with
+// one LDS-only barrier per step. 16-byte slots of a staged row are XOR-swizzled by the row.
+//
+// Measured against the kernels that served these sizes before (same box, us per launch):
+//   int8 W, fp32 X   300 x 8192 x 2048: 117 -> 36   300 x 2048 x 4096: 221 -> 25   1024 x 8192 x 2048: 119 -> 63
+//   bf16 W, bf16 X    64 x 2048 x 4096: 21 -> 9.6    300 x 2048 x 4096: 83 -> 25     300 x 8192 x 2048: 47 -> 33
+// Prefetching four steps instead of two, or accumulating in fewer, larger tiles at small M, gained
+// nothing: a step costs 0.1 to 0.2 us even in the smallest tile (the barrier, the LDS round trip and
+// the dependent products), which is why small tiles with K split over 8 waves win there.
+#include "common.h"
+
+#include <type_traits>
+
+using namespace aegist;
+
+namespace {
+
+typedef int int4v __attribute__((ext_vector_type(4)));
+
+constexpr int MKS = 64;                             // k per step
+constexpr int kMidBufWord3 = 0x00020000;            // buffer resource word 3 on gfx9: 32-bit data, no swizzle
+constexpr int kMidOob = 0x7ffffff0;                 // past every operand (< 2^31 - 16 bytes): loads return 0
+
+constexpr int MID_SEG = 4;
+struct MidSeg {
+    const void* W;
+    const uint16_t* scale;  // per-row scale or null
+    float* Y;
+    long long ldy;
+    int N, t0;              // rows; first N tile of the launch
+};
+struct MidArgs {
+    const void* X;
+    MidSeg seg[MID_SEG];
+    int nseg, ldx, M, K, accumulate, tiles_m, ntiles, per_xcd;
+};
+
+__device__ __forceinline__ int4v buf16(__amdgpu_buffer_rsrc_t rs, int off) {
+    return __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
+}
+
+// A lane's 16 weights of one row and step as two bf16x8 fragments; slot(h, g) is the 8-value slot
+// of the step that fragment h of lane group g holds. Each load instruction of a wave covers 64
+// contiguous bytes of 16 rows: int8 lanes take 16 consecutive values, bf16 lanes 8 of each half.
+template <typename TW> struct MidW;
+template <> struct MidW<int8_t> {
+    int4v r;
+    static __device__ __forceinline__ int slot(int h, int g) { return 2 * g + h; }
+    // k0: first k of the step; rows end at K (a multiple of 16)
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rs, int row, int k0, int g, int K) {
+        r = buf16(rs, k0 + 16 * g < K ? row + k0 + 16 * g : kMidOob);
+    }
+    __device__ __forceinline__ bf16x8 frag(int h) const {
+        // int8 -> fp32 is exact and keeps 8 significant bits, so its top half is the exact bf16
+        uint32_t p[4];
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const uint32_t d = (uint32_t)r[2 * h + i];
+            const float f0 = (float)(int8_t)d, f1 = (float)(int8_t)(d >> 8);
+            const float f2 = (float)(int8_t)(d >> 16), f3 = (float)(int8_t)(d >> 24);
+            p[2 * i] = __builtin_amdgcn_perm(__float_as_uint(f1), __float_as_uint(f0), 0x07060302u);
+            p[2 * i + 1] = __builtin_amdgcn_perm(__float_as_uint(f3), __float_as_uint(f2), 0x07060302u);
+        }
+        return __builtin_bit_cast(bf16x8, p);
+    }
+};
+template <> struct MidW<uint16_t> {
+    int4v r[2];
+    static __device__ __forceinline__ int slot(int h, int g) { return 4 * h + g; }
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rs, int row, int k0, int g, int K) {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int k = k0 + 32 * h + 8 * g;
+            r[h] = buf16(rs, k < K ? (row + k) * 2 : kMidOob);
+        }
+    }
+    __device__ __forceinline__ bf16x8 frag(int h) const { return __builtin_bit_cast(bf16x8, r[h]); }
+};
+
+// 8 consecutive activations of one row
+template <typename TX> struct MidX;
+template <> struct MidX<float> {
+    static constexpr int kParts = 2;
+    int4v r[2];
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rs, int off) {
+        r[0] = buf16(rs, off);
+        r[1] = buf16(rs, off + 16);
+    }
+    // x = hi + lo, hi = x truncated to bf16, lo = the rounded remainder: |x - hi - lo| <= 2^-16 |x|
+    __device__ __forceinline__ void store(unsigned char* dst, int part) const {
+        uint32_t h[4], l[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const uint32_t u0 = (uint32_t)r[e / 2][2 * (e % 2)], u1 = (uint32_t)r[e / 2][2 * (e % 2) + 1];
+            h[e] = __builtin_amdgcn_perm(u1, u0, 0x07060302u);
+            typedef float f2 __attribute__((ext_vector_type(2)));
+            typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+            const f2 lo = {__uint_as_float(u0) - __uint_as_float(u0 & 0xffff0000u),
+                           __uint_as_float(u1) - __uint_as_float(u1 & 0xffff0000u)};
+            l[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(lo, b2));
+        }
+        *(uint4*)dst = uint4{h[0], h[1], h[2], h[3]};
+        *(uint4*)(dst + part) = uint4{l[0], l[1], l[2], l[3]};
+    }
+};
+template <> struct MidX<uint16_t> {
+    static constexpr int kParts = 1;
+    int4v r;
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rs, int off) { r = buf16(rs, off); }
+    __device__ __forceinline__ void store(unsigned char* dst, int) const { *(int4v*)dst = r; }
+};
+
+template <typename TW, typename TX, int RT, int MT, int NWN, int KG, int PD>
+__global__ void __launch_bounds__(64 * NWN * KG) gemm_mid_kernel(const MidArgs ga) {
+    constexpr int BM = 16 * MT, BN = 16 * RT * NWN, TPG = 64 * NWN, SL = BM * 8 / TPG;
+    static_assert(SL >= 1 && SL * TPG == BM * 8, "the X stage must split evenly over the group's threads");
+    constexpr int kPart = BM * MKS * 2;                       // bytes of one part (hi or lo) of an X stage
+    constexpr int kStage = kPart * MidX<TX>::kParts;
+    constexpr int kRed = KG > 1 ? (KG - 1) * NWN * RT * MT * 1024 : 0;
+    constexpr int kLds = 2 * KG * kStage > kRed ? 2 * KG * kStage : kRed;
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[kLds];
+
+    // XCD x runs the logical tiles [x n / 8, (x + 1) n / 8), M tiles fastest: the workgroups that
+    // share W rows run on one XCD and read them through its L2
+    const int li = (blockIdx.x % 8) * ga.per_xcd + blockIdx.x / 8;
+    if (li >= ga.ntiles) return;
+    const int m0 = (li % ga.tiles_m) * BM, tn = li / ga.tiles_m;
+    int si = 0;
+#pragma unroll
+    for (int i = 1; i < MID_SEG; i++)
+        if (i < ga.nseg && tn >= ga.seg[i].t0) si = i;
+    const MidSeg sg = ga.seg[si];
+    const int n0 = (tn - sg.t0) * BN;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
+    const int kg = wave / NWN, wn = wave % NWN, r16 = lane % 16, g = lane / 16, tg = tid - kg * TPG;
+    const int M = ga.M, N = sg.N, K = ga.K;
+
+    const __amdgpu_buffer_rsrc_t wrs =
+        __builtin_amdgcn_make_buffer_rsrc((void*)sg.W, (short)0, (int)((long long)N * K * sizeof(TW)), kMidBufWord3);
+    const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)ga.X, (short)0, (int)(((long long)(M - 1) * ga.ldx + K) * sizeof(TX)), kMidBufWord3);
+    int wbase[RT];
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++) wbase[rt] = min(n0 + 16 * (RT * wn + rt) + r16, N - 1) * K;
+    int xbase[SL], xdst[SL];
+#pragma unroll
+    for (int i = 0; i < SL; i++) {
+        const int q = tg + TPG * i, row = q / 8, s = q % 8;
+        xbase[i] = min(m0 + row, M - 1) * ga.ldx + 8 * s;
+        xdst[i] = row * 128 + ((s ^ ((row >> 1) & 7)) * 16);
+    }
+    unsigned char* const buf = lds + kg * 2 * kStage;
+    const int xs8 = 8 * (tg % 8);  // this thread's k offset inside a step
+
+    MidX<TX> xr[PD][SL];
+    MidW<TW> wr[PD][RT];
+    // steps past K load zeros (both operands), so every K group runs the same number of steps
+    auto load_x = [&](int set, int t) {
+        const int k0 = (kg + KG * t) * MKS;
+        const bool ok = k0 + xs8 < K;
+#pragma unroll
+        for (int i = 0; i < SL; i++) xr[set][i].load(xrs, ok ? (xbase[i] + k0) * (int)sizeof(TX) : kMidOob);
+    };
+    auto load_w = [&](int slot, int t) {
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++) wr[slot][rt].load(wrs, wbase[rt], (kg + KG * t) * MKS, g, K);
+    };
+    auto store_x = [&](int set, int t) {
+#pragma unroll
+        for (int i = 0; i < SL; i++) xr[set][i].store(buf + (t & 1) * kStage + xdst[i], kPart);
+    };
+
+    f32x4 acc[RT][MT];
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) acc[rt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    // the row scales of the lane's 4 RT outputs, requested before the stream
+    const bool fin = kg == 0;
+    uint16_t sraw[RT][4];
+    if (fin && sg.scale) {
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) sraw[rt][j] = sg.scale[min(n0 + 16 * (RT * wn + rt) + 4 * g + j, N - 1)];
+    }
+
+    const int nt = (K + MKS * KG - 1) / (MKS * KG);
+    load_x(0, 0);
+#pragma unroll
+    for (int d = 0; d < PD; d++) load_w(d, d);
+    store_x(0, 0);
+#pragma unroll
+    for (int d = 0; d < PD; d++) load_x(d, 1 + d);
+    lds_barrier();
+    // step t (slot = t % PD): X of step t + 1 goes from registers to LDS and its registers take
+    // step t + 1 + PD; the products of step t; W registers refilled with step t + PD
+    auto step = [&](int t, int slot) {
+        store_x(slot, t + 1);
+        load_x(slot, t + 1 + PD);
+        const unsigned char* cur = buf + (slot & 1) * kStage;  // PD is even: slot and t agree
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++) {
+            bf16x8 a[RT];
+#pragma unroll
+            for (int rt = 0; rt < RT; rt++) a[rt] = wr[slot][rt].frag(ks);
+            if (ks == 1) load_w(slot, t + PD);
+#pragma unroll
+            for (int mt = 0; mt < MT; mt++) {
+                const int row = 16 * mt + r16;
+                const unsigned char* p = cur + row * 128 + ((MidW<TW>::slot(ks, g) ^ ((row >> 1) & 7)) * 16);
+                const bf16x8 bh = *(const bf16x8*)p;
+#pragma unroll
+                for (int rt = 0; rt < RT; rt++)
+                    acc[rt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rt], bh, acc[rt][mt], 0, 0, 0);
+                if constexpr (MidX<TX>::kParts == 2) {
+                    const bf16x8 bl = *(const bf16x8*)(p + kPart);
+#pragma unroll
+                    for (int rt = 0; rt < RT; rt++)
+                        acc[rt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rt], bl, acc[rt][mt], 0, 0, 0);
+                }
+            }
+        }
+        lds_barrier();
+    };
+    // whole rounds of PD steps: steps past K are products of zeros
+    for (int t = 0; t < nt; t += PD) {
+#pragma unroll
+        for (int d = 0; d < PD; d++) step(t + d, d);
+    }
+
+    if constexpr (KG > 1) {
+        // the K groups' partial tiles, added in group order
+        f32x4* red = (f32x4*)lds;
+        if (kg > 0) {
+#pragma unroll
+            for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++)
+                    red[((((kg - 1) * NWN + wn) * RT + rt) * MT + mt) * WAVE + lane] = acc[rt][mt];
+        }
+        lds_barrier();
+        if (!fin) return;
+#pragma unroll
+        for (int q = 0; q < KG - 1; q++)
+#pragma unroll
+            for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+                for (int mt = 0; mt < MT; mt++) acc[rt][mt] += red[(((q * NWN + wn) * RT + rt) * MT + mt) * WAVE + lane];
+    }
+    const bool vec = (sg.ldy % 4) == 0 && ((uintptr_t)sg.Y % 16) == 0;
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++) {
+        const int n = n0 + 16 * (RT * wn + rt) + 4 * g;
+        float sc[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) sc[j] = sg.scale ? bf2f(sraw[rt][j]) : 1.f;
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+            const int m = m0 + 16 * mt + r16;
+            if (m >= M) continue;
+            float* y = sg.Y + (size_t)m * sg.ldy + n;
+            if (vec && n + 3 < N) {
+                f32x4 v = acc[rt][mt];
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[j] *= sc[j];
+                if (ga.accumulate) v += *(const f32x4*)y;
+                *(f32x4*)y = v;
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    if (n + j < N) y[j] = (ga.accumulate ? y[j] : 0.f) + acc[rt][mt][j] * sc[j];
+            }
+        }
+    }
+}
+
+// One form of the kernel and its cost: us of one 64-k step of a round of workgroups (one per CU), the
+// median over a sweep of M 20 .. 1500 and N x K 512 .. 8192 x 2048 and 2048 x 4096 on one card; the
+// estimate ceil(tiles / 256) x steps x cost picked the fastest form or one within 10% of it at 50 of
+// the 56 swept sizes (at worst 20% slower, between neighbouring tile sizes).
+struct MidForm {
+    int rt, mt, nwn, kg;
+    float cost;
+};
+// fp32 X: staging and splitting X is the larger part of a step
+constexpr MidForm kFormsF32[] = {{1, 2, 1, 8, 0.156f}, {1, 2, 2, 8, 0.18f}, {2, 2, 2, 8, 0.265f}, {2, 2, 4, 4, 0.375f},
+                                 {2, 4, 4, 2, 0.60f},  {2, 4, 8, 1, 1.10f}, {4, 4, 8, 1, 1.70f}};
+constexpr MidForm kFormsBf16[] = {{1, 2, 1, 8, 0.100f}, {1, 2, 2, 8, 0.157f}, {1, 4, 2, 4, 0.205f}, {1, 4, 4, 2, 0.312f},
+                                  {2, 4, 4, 2, 0.548f}, {2, 8, 4, 1, 0.90f},  {2, 8, 8, 1, 1.21f}};
+constexpr int kForms = 7;
+// the 256 x 256 tiles of gemm.hip, in the same unit: int8 W with fp32 X, bf16 W with bf16 X
+constexpr float kTile256F32 = 3.7f, kTile256Bf16 = 1.5f;
+
+long long mid_tiles(const MidForm& f, const MidArgs& ga) {
+    long long t = 0;
+    for (int i = 0; i < ga.nseg; i++) t += (ga.seg[i].N + 16 * f.rt * f.nwn - 1) / (16 * f.rt * f.nwn);
+    return t * ((ga.M + 16 * f.mt - 1) / (16 * f.mt));
+}
+
+template <typename TW, typename TX, int RT, int MT, int NWN, int KG, int PD>
+int launch_mid(MidArgs ga, hipStream_t st) {
+    constexpr int BM = 16 * MT, BN = 16 * RT * NWN;
+    ga.tiles_m = (ga.M + BM - 1) / BM;
+    int t = 0;
+    for (int i = 0; i < ga.nseg; i++) {
+        ga.seg[i].t0 = t;
+        t += (ga.seg[i].N + BN - 1) / BN;
+    }
+    ga.ntiles = ga.tiles_m * t;
+    ga.per_xcd = (ga.ntiles + 7) / 8;
+    gemm_mid_kernel<TW, TX, RT, MT, NWN, KG, PD><<<8 * ga.per_xcd, 64 * NWN * KG, 0, st>>>(ga);
+    return after_launch("gemm_mid");
+}
+
+template <typename TW, typename TX>
+int run_mid(int form, const MidArgs& ga, hipStream_t st) {
+    constexpr bool f32 = std::is_same<TX, float>::value;
+#define AEG_MID(I)                                                                                              \
+    case I: {                                                                                                   \
+        constexpr MidForm f = f32 ? kFormsF32[I] : kFormsBf16[I];                                               \
+        return launch_mid<TW, TX, f.rt, f.mt, f.nwn, f.kg, 2>(ga, st);                                          \
+    }
+    switch (form) {
+        AEG_MID(0) AEG_MID(1) AEG_MID(2) AEG_MID(3) AEG_MID(4) AEG_MID(5) AEG_MID(6)
+    }
+#undef AEG_MID
+    return fail(AEGIST_ERR_SHAPE, "gemm_mid: no such form");
+}
+
+}  // namespace
+
+namespace aegist {
+
+// Whether this file's kernel takes the product (`tile256`: gemm.hip's 256 x 256 tiles could take it
+// too, as one launch of all weights), and the form it takes: 17 rows or more, operands below 2 GiB,
+// and an estimate no worse than that of the 256 x 256 tiles. -1 if not. The caller has checked
+// K % 16 == 0 and the 16-byte alignment of every row.
+int gemm_mid_form(int x_dtype, long long ldx, int w_dtype, int nseg, const int* N, int M, int K, bool tile256) {
+    if (M <= 16 || nseg < 1 || nseg > MID_SEG || K <= 0) return -1;
+    const long long lim = 0x7ffffff0LL, xs = x_dtype == AEGIST_F32 ? 4 : 2, wsz = w_dtype == AEGIST_I8 ? 1 : 2;
+    if (ldx > 0x7fffffffLL || (long long)M * ldx * xs >= lim) return -1;
+    MidArgs ga{};
+    ga.nseg = nseg;
+    ga.M = M;
+    long long t256 = 0;
+    for (int i = 0; i < nseg; i++) {
+        if ((long long)N[i] * K * wsz >= lim) return -1;
+        ga.seg[i].N = N[i];
+        t256 += N[i];
+    }
+    t256 = (t256 + 255) / 256 * ((M + 255) / 256);
+    const MidForm* forms = x_dtype == AEGIST_F32 ? kFormsF32 : kFormsBf16;
+    int best = -1;
+    float least = tile256 ? ((t256 + 255) / 256) * (x_dtype == AEGIST_F32 ? kTile256F32 : kTile256Bf16) : 3.4e38f;
+    for (int i = 0; i < kForms; i++) {
+        const long long t = mid_tiles(forms[i], ga);
+        if (t >= (1LL << 27)) continue;
+        const float est = ((t + 255) / 256) * forms[i].cost;
+        if (est <= least) {
+            least = est;
+            best = i;
+        }
+    }
+    return best;
+}
+
+int launch_gemm_mid(int form, const void* X, int x_dtype, long long ldx, int w_dtype, int nseg, const void* const* W,
+                    const uint16_t* const* scale, float* const* Y, const long long* ldy, const int* N, int M, int K,
+                    int accumulate, hipStream_t st) {
+    if (nseg < 1 || nseg > MID_SEG || form < 0) return fail(AEGIST_ERR_SHAPE, "gemm_mid: 1 to 4 weights per launch");
+    MidArgs ga{};
+    ga.X = X;
+    ga.nseg = nseg;
+    ga.ldx = (int)ldx;
+    ga.M = M;
+    ga.K = K;
+    ga.accumulate = accumulate;
+    for (int i = 0; i < nseg; i++) ga.seg[i] = MidSeg{W[i], scale[i], Y[i], ldy[i], N[i], 0};
+    if (w_dtype == AEGIST_I8)
+        return x_dtype == AEGIST_F32 ? run_mid<int8_t, float>(form, ga, st) : run_mid<int8_t, uint16_t>(form, ga, st);
+    return x_dtype == AEGIST_F32 ? run_mid<uint16_t, float>(form, ga, st) : run_mid<uint16_t, uint16_t>(form, ga, st);
+}
+
+}  // namespace aegist

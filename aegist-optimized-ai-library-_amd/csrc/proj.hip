@@ -5,8 +5,8 @@
 //     Y[m, n] (+)= scale[n] * sum_k X[m, k] W[n, k]
 // with fp32 accumulation. accumulate = 1 adds into Y (the residual add of the out-projections).
 //
-// At decode sizes (M = batch <= 64) the op streams the weight matrix once from HBM, so the
-// kernel is built around that stream: each wave owns RT 16-row tiles of W and a contiguous run
+// At decode sizes (M = batch <= 16; gemm_mid.hip takes larger batches, gemm.hip the largest) the op
+// streams the weight matrix once from HBM, so the kernel is built around that stream: each wave owns RT 16-row tiles of W and a contiguous run
 // of 64-wide k steps, loads 16 bytes of int8 weights (or 32 of bf16) per lane per step, and
 // feeds v_mfma_f32_16x16x32_bf16 with W as the A operand and X^T as the B operand, so every
 // weight byte is used by MT 16-row tiles of X at once. Four waves of a workgroup interleave
@@ -34,6 +34,10 @@ int launch_gemm_bf16(const uint16_t* X, long long ldx, const uint16_t* W, long l
 int launch_gemm_bf16_multi(const uint16_t* X, long long ldx, int nseg, const uint16_t* const* W, const long long* ldw,
                            float* const* Y, const long long* ldy, const int* N, int M, int K, int accumulate,
                            hipStream_t st);
+int gemm_mid_form(int x_dtype, long long ldx, int w_dtype, int nseg, const int* N, int M, int K, bool tile256);
+int launch_gemm_mid(int form, const void* X, int x_dtype, long long ldx, int w_dtype, int nseg, const void* const* W,
+                    const uint16_t* const* scale, float* const* Y, const long long* ldy, const int* N, int M, int K,
+                    int accumulate, hipStream_t st);
 }  // namespace aegist
 
 namespace {
@@ -332,9 +336,9 @@ __global__ __launch_bounds__(64 * NWAVE) void proj_skinny_kernel(const TX* __res
 // each lane is permuted, the 1 KB it covers is not), so the 16 rows a fragment read touches
 // hit 16 different bank groups.
 constexpr int SKC = 256;  // k per chunk
-template <typename TX, int NW, int NS, int MT = 1>
+template <typename TX, int NW, int NS>
 struct StreamSmem {
-    static constexpr int XB = 16 * MT * SKC * sizeof(TX);  // X bytes per stage (16 MT rows)
+    static constexpr int XB = 16 * SKC * sizeof(TX);  // X bytes per stage (16 rows)
     __attribute__((aligned(16))) unsigned char w[NS][16 * NW][SKC * 2];
     __attribute__((aligned(16))) unsigned char x[NS][XB];
 };
@@ -365,16 +369,15 @@ __device__ __forceinline__ void wait_vm(int n) {
     }
 }
 
-template <typename TX, int NW, int NS, int MT = 1>
+template <typename TX, int NW, int NS>
 __global__ __launch_bounds__(64 * NW) void proj_stream_kernel(const TX* __restrict__ X, long long ldx,
                                                                const ProjSegs segs, int M, int K, int accumulate,
                                                                float* __restrict__ part) {
-    static_assert(MT == 1 || sizeof(TX) == 2, "several m tiles take bf16 X only");
-    __shared__ StreamSmem<TX, NW, NS, MT> sm;
+    __shared__ StreamSmem<TX, NW, NS> sm;
     constexpr int RW = 16 * NW;                       // W rows per workgroup
     constexpr int WI = RW / 2 / NW;                   // W load instructions per wave per stage (= 8)
-    constexpr int XI = StreamSmem<TX, NW, NS, MT>::XB / 1024 / NW;  // X load instructions per wave per stage
-    static_assert(XI * NW * 1024 == StreamSmem<TX, NW, NS, MT>::XB, "X stage must split evenly over the waves");
+    constexpr int XI = StreamSmem<TX, NW, NS>::XB / 1024 / NW;  // X load instructions per wave per stage
+    static_assert(XI * NW * 1024 == StreamSmem<TX, NW, NS>::XB, "X stage must split evenly over the waves");
     constexpr int PER = WI + XI;                      // loads per wave per stage
     const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
     const int r16 = lane % 16, g = lane / 16;
@@ -414,9 +417,7 @@ __global__ __launch_bounds__(64 * NW) void proj_stream_kernel(const TX* __restri
         }
     };
 
-    f32x4 acc[MT];
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++) acc[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    f32x4 acc{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int c = 0; c < NS - 1; c++)
         if (c < nch) issue(c);
@@ -433,11 +434,8 @@ __global__ __launch_bounds__(64 * NW) void proj_stream_kernel(const TX* __restri
             // k block i of the chunk: lane (row, g) takes slot 4 i + g of its row (swizzled)
             const bf16x8 a = *(const bf16x8*)&sm.w[st][row][((4 * i + g) ^ (row & 15)) * 16];
             if constexpr (sizeof(TX) == 2) {
-#pragma unroll
-                for (int mt = 0; mt < MT; mt++) {
-                    const bf16x8 b = *(const bf16x8*)&sm.x[st][((16 * mt + r16) * SKC + 32 * i + 8 * g) * 2];
-                    acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[mt], 0, 0, 0);
-                }
+                const bf16x8 b = *(const bf16x8*)&sm.x[st][(r16 * SKC + 32 * i + 8 * g) * 2];
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
             } else {
                 const float* xp = (const float*)&sm.x[st][(r16 * SKC + 32 * i + 8 * g) * 4];
                 const f32x4 x0 = *(const f32x4*)xp, x1 = *(const f32x4*)(xp + 4);
@@ -452,63 +450,38 @@ __global__ __launch_bounds__(64 * NW) void proj_stream_kernel(const TX* __restri
                                    v1 - __uint_as_float(__float_as_uint(v1) & 0xffff0000u)};
                     l[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(lo, b2));
                 }
-                acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf16x8, h), acc[0], 0, 0, 0);
-                acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf16x8, l), acc[0], 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf16x8, h), acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf16x8, l), acc, 0, 0, 0);
             }
         }
     }
-    // lane (m = 16 mt + r16, g) of tile mt holds Y[m][n0 + 16 wave + 4 g .. +3]
-    const int nb = n0 + 16 * wave + 4 * g;
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++) {
-        const int m = 16 * mt + r16;
-        if (m >= M || nb >= N) continue;
-        if (part) {
-            float* pp = part + ((size_t)ks * M + m) * N + nb;
-            if (nb + 3 < N && (N % 4) == 0) {
-                *(f32x4*)pp = acc[mt];
-            } else {
-#pragma unroll
-                for (int j = 0; j < 4; j++)
-                    if (nb + j < N) pp[j] = acc[mt][j];
-            }
-            continue;
-        }
-        float* yp = Y + (size_t)m * ldy + nb;
-        if (nb + 3 < N && ((uintptr_t)yp % 16) == 0) {
-            f32x4 v = acc[mt];
-            if (accumulate) v += *(const f32x4*)yp;
-            *(f32x4*)yp = v;
+    // lane (m = r16, g) holds Y[m][n0 + 16 wave + 4 g .. +3]
+    const int nb = n0 + 16 * wave + 4 * g, m = r16;
+    if (m >= M || nb >= N) return;
+    if (part) {
+        float* pp = part + ((size_t)ks * M + m) * N + nb;
+        if (nb + 3 < N && (N % 4) == 0) {
+            *(f32x4*)pp = acc;
         } else {
 #pragma unroll
             for (int j = 0; j < 4; j++)
-                if (nb + j < N) yp[j] = (accumulate ? yp[j] : 0.f) + acc[mt][j];
+                if (nb + j < N) pp[j] = acc[j];
         }
+        return;
     }
-}
-
-// Y[m][n] (+)= sum over ks = 0 .. nks - 1, in that order, of part[ks][m][n] (the split-K slices
-// of proj_stream_kernel); 4 columns per thread, N % 4 == 0.
-__global__ void proj_splitk_reduce_kernel(const float* __restrict__ part, int nks, int M, int N, float* __restrict__ Y,
-                                          long long ldy, int accumulate) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x, n4 = N / 4;
-    if (i >= M * n4) return;
-    const int m = i / n4, n = 4 * (i % n4);
-    const size_t slice = (size_t)M * N;
-    const float* p = part + (size_t)m * N + n;
-    f32x4 v = *(const f32x4*)p;
-    for (int k = 1; k < nks; k++) v += *(const f32x4*)(p + k * slice);
-    float* y = Y + (size_t)m * ldy + n;
-    if (((uintptr_t)y % 16) == 0) {
-        if (accumulate) v = *(const f32x4*)y + v;
-        *(f32x4*)y = v;
+    float* yp = Y + (size_t)m * ldy + nb;
+    if (nb + 3 < N && ((uintptr_t)yp % 16) == 0) {
+        f32x4 v = acc;
+        if (accumulate) v += *(const f32x4*)yp;
+        *(f32x4*)yp = v;
     } else {
 #pragma unroll
-        for (int j = 0; j < 4; j++) y[j] = (accumulate ? y[j] : 0.f) + v[j];
+        for (int j = 0; j < 4; j++)
+            if (nb + j < N) yp[j] = (accumulate ? yp[j] : 0.f) + acc[j];
     }
 }
 
-template <typename TX, int NW, int NS, int MT = 1>
+template <typename TX, int NW, int NS>
 int launch_stream(const TX* X, long long ldx, ProjSegs segs, int M, int K, int accumulate, hipStream_t st,
                   float* part = nullptr, int nks = 1) {
     int t = 0;
@@ -517,7 +490,7 @@ int launch_stream(const TX* X, long long ldx, ProjSegs segs, int M, int K, int a
         t += (segs.s[i].N + 16 * NW - 1) / (16 * NW);
     }
     segs.tile0[segs.n] = t;
-    proj_stream_kernel<TX, NW, NS, MT><<<dim3(t, nks), 64 * NW, 0, st>>>(X, ldx, segs, M, K, accumulate, part);
+    proj_stream_kernel<TX, NW, NS><<<dim3(t, nks), 64 * NW, 0, st>>>(X, ldx, segs, M, K, accumulate, part);
     return 0;
 }
 
@@ -562,48 +535,55 @@ void launch_mt(const TX* X, long long ldx, const ProjSegs& segs, int M, int K, i
 
 template <typename TW, typename TX>
 int run_proj(const TX* X, long long ldx, const ProjSegs& segs, int M, int K, int accumulate, hipStream_t st) {
-    // int8 weights with fp32 activations past 64 rows (the engine's gemm_i8): the tiled GEMM
-    if constexpr (std::is_same<TW, int8_t>::value && std::is_same<TX, float>::value) {
-        bool ok = M > 64;
-        for (int i = 0; i < segs.n && ok; i++) ok = gemm_i8f32_fits(X, ldx, segs.s[i].W, K, M, segs.s[i].N, K);
-        if (ok) {
-            for (int i = 0; i < segs.n; i++) {
-                int rc = launch_gemm_i8f32(X, ldx, (const int8_t*)segs.s[i].W, K, segs.s[i].scale, segs.s[i].Y,
-                                           segs.s[i].ldy, M, segs.s[i].N, K, accumulate, st);
-                if (rc) return rc;
-            }
-            return 0;
+    constexpr bool i8 = std::is_same<TW, int8_t>::value, f32 = std::is_same<TX, float>::value;
+    if (M > 16) {
+        const void* W[MAX_SEG];
+        const uint16_t* scale[MAX_SEG];
+        float* Y[MAX_SEG];
+        long long ldw[MAX_SEG], ldy[MAX_SEG];
+        int N[MAX_SEG];
+        // past 64 rows the 256 x 256 MFMA tiles take int8 weights with fp32 activations (the engine's
+        // gemm_i8, one launch per weight) and unscaled bf16 weights with bf16 activations (all weights
+        // in one launch, stacked along N, when each but the last has a multiple of 8 rows)
+        bool tile256 = M > 64 && i8 == f32, stack8 = segs.n <= 3;
+        for (int i = 0; i < segs.n; i++) {
+            const ProjSeg& sg = segs.s[i];
+            W[i] = sg.W;
+            scale[i] = sg.scale;
+            Y[i] = sg.Y;
+            ldw[i] = K;
+            ldy[i] = sg.ldy;
+            N[i] = sg.N;
+            if (i8) tile256 = tile256 && gemm_i8f32_fits(X, ldx, sg.W, K, M, sg.N, K);
+            else tile256 = tile256 && !sg.scale && gemm_bf16_fits(X, ldx, sg.W, K, M, sg.N, K);
+            if (i + 1 < segs.n && sg.N % 8) stack8 = false;
         }
-    }
-    // bf16 weights and activations past 64 rows: the tiled MFMA GEMM, all weights in one launch
-    // (stacked along N) when each but the last has a multiple of 8 rows, else one launch each
-    if constexpr (std::is_same<TW, uint16_t>::value && std::is_same<TX, uint16_t>::value) {
-        bool ok = M > 64, stack8 = segs.n <= 3;
-        for (int i = 0; i < segs.n && ok; i++) {
-            ok = segs.s[i].scale == nullptr && gemm_bf16_fits(X, ldx, segs.s[i].W, K, M, segs.s[i].N, K);
-            if (i + 1 < segs.n && segs.s[i].N % 8) stack8 = false;
-        }
-        if (ok && stack8) {
-            const uint16_t* W[MAX_SEG];
-            float* Y[MAX_SEG];
-            long long ldw[MAX_SEG], ldy[MAX_SEG];
-            int N[MAX_SEG];
-            for (int i = 0; i < segs.n; i++) {
-                W[i] = (const uint16_t*)segs.s[i].W;
-                Y[i] = segs.s[i].Y;
-                ldw[i] = K;
-                ldy[i] = segs.s[i].ldy;
-                N[i] = segs.s[i].N;
+        const int form = gemm_mid_form(f32 ? AEGIST_F32 : AEGIST_BF16, ldx, i8 ? AEGIST_I8 : AEGIST_BF16, segs.n, N, M, K,
+                                       tile256);
+        if (form >= 0)
+            return launch_gemm_mid(form, X, f32 ? AEGIST_F32 : AEGIST_BF16, ldx, i8 ? AEGIST_I8 : AEGIST_BF16, segs.n, W,
+                                   scale, Y, ldy, N, M, K, accumulate, st);
+        if constexpr (i8 && f32) {
+            if (tile256) {
+                for (int i = 0; i < segs.n; i++) {
+                    int rc = launch_gemm_i8f32(X, ldx, (const int8_t*)W[i], K, scale[i], Y[i], ldy[i], M, N[i], K,
+                                               accumulate, st);
+                    if (rc) return rc;
+                }
+                return 0;
             }
-            return launch_gemm_bf16_multi(X, ldx, segs.n, W, ldw, Y, ldy, N, M, K, accumulate, st);
         }
-        if (ok) {
-            for (int i = 0; i < segs.n; i++) {
-                int rc = launch_gemm_bf16(X, ldx, (const uint16_t*)segs.s[i].W, K, segs.s[i].Y, segs.s[i].ldy, M,
-                                          segs.s[i].N, K, accumulate, st);
-                if (rc) return rc;
+        if constexpr (!i8 && !f32) {
+            if (tile256 && stack8)
+                return launch_gemm_bf16_multi(X, ldx, segs.n, (const uint16_t* const*)W, ldw, Y, ldy, N, M, K, accumulate,
+                                              st);
+            if (tile256) {
+                for (int i = 0; i < segs.n; i++) {
+                    int rc = launch_gemm_bf16(X, ldx, (const uint16_t*)W[i], K, Y[i], ldy[i], M, N[i], K, accumulate, st);
+                    if (rc) return rc;
+                }
+                return 0;
             }
-            return 0;
         }
     }
     // bf16 weights at M <= 16 with K a multiple of the chunk, no row scales: the LDS-staged stream
@@ -621,46 +601,11 @@ int run_proj(const TX* X, long long ldx, const ProjSegs& segs, int M, int K, int
             launch_stream<TX, 2, 2>(X, ldx, segs, M, K, accumulate, st);
             return after_launch("proj_stream");
         }
-        // 17..64 rows of bf16 X and one weight whose rows give too few workgroups (2048 x 4096:
-        // 64 workgroups of 32 rows): the same stream with all the rows' X staged once per chunk,
-        // split over K into ~256 workgroups when the calling thread has bound a workspace for
-        // the fp32 partials, which a second launch adds in slice order (deterministic). Measured
-        // at M = 64: 2048 x 4096 21.2 -> 13.7 us; with enough rows (8192 x 2048 and the stack's
-        // grouped input projections) the row-tile kernel below is as fast, so it keeps them.
-        if constexpr (std::is_same<TX, uint16_t>::value) {
-            const long long t = (segs.s[0].N + 31) / 32;
-            if (M > 16 && M <= 64 && K % SKC == 0 && !scaled && segs.n == 1 && t < 192 && segs.s[0].N % 4 == 0 &&
-                stream_enabled()) {
-                const int nks = (int)std::min<long long>(K / SKC, (256 + t - 1) / t);
-                size_t bound = 0;
-                void* ws = bound_workspace(&bound);
-                if (nks > 1 && ws && bound >= (size_t)nks * M * segs.s[0].N * 4) {
-                    float* part = (float*)ws;
-                    if (M <= 32) launch_stream<TX, 2, 2, 2>(X, ldx, segs, M, K, accumulate, st, part, nks);
-                    else launch_stream<TX, 2, 2, 4>(X, ldx, segs, M, K, accumulate, st, part, nks);
-                    int rc = after_launch("proj_stream64");
-                    if (rc) return rc;
-                    const ProjSeg& sg = segs.s[0];
-                    const int nthr = M * (sg.N / 4);
-                    proj_splitk_reduce_kernel<<<(nthr + 255) / 256, 256, 0, st>>>(part, nks, M, sg.N, sg.Y, sg.ldy,
-                                                                                 accumulate);
-                    return after_launch("proj_splitk_reduce");
-                }
-            }
-        }
     }
-    // m tiles per workgroup: the whole batch up to 64 rows of bf16 X (32 of fp32 X, whose hi/lo
-    // operands take twice the registers), so the weights are read once; larger M is covered by
-    // a grid of row groups
-    if (M <= 16) {
-        launch_mt<TW, TX, 1>(X, ldx, segs, M, K, accumulate, st);
-    } else if constexpr (XLoad<TX>::kLo) {
-        launch_mt<TW, TX, 2>(X, ldx, segs, M, K, accumulate, st);
-    } else {
-        if (M <= 32) launch_mt<TW, TX, 2>(X, ldx, segs, M, K, accumulate, st);
-        else if (M <= 48) launch_mt<TW, TX, 3>(X, ldx, segs, M, K, accumulate, st);
-        else launch_mt<TW, TX, 4>(X, ldx, segs, M, K, accumulate, st);
-    }
+    // past 16 rows only operands that gemm_mid.hip cannot address (2 GiB and more) come here: a grid
+    // of groups of 32 rows
+    if (M <= 16) launch_mt<TW, TX, 1>(X, ldx, segs, M, K, accumulate, st);
+    else launch_mt<TW, TX, 2>(X, ldx, segs, M, K, accumulate, st);
     return after_launch("proj_skinny");
 }
 

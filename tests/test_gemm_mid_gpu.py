@@ -1,0 +1,57 @@
+"""GPU parity of the middling-batch projections (17 rows and more, csrc/gemm_mid.hip) against fp64 dot
+products of the exact operands, at the edges of their tiles (16 to 128 rows of X, 16 to 256 of W, 64 k
+split over 1 to 8 wave groups). bf16 products are exact and summed in fp32: every output is within
+K 2^-24 sum |x w s| of the exact one; fp32 X enters as bf16 hi + lo, within another 2^-16 sum |x w s|."""
+import pytest
+import torch
+
+from aegist_mixer import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _operands(M, N, K, w8, xf, seed, dev):
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(M, K, generator=g).to(torch.float32 if xf else torch.bfloat16)
+    w = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8) if w8 else \
+        (torch.randn(N, K, generator=g) * 0.02).to(torch.bfloat16)
+    s = (torch.rand(N, generator=g) * 1e-2).to(torch.bfloat16) if w8 else None
+    return x.to(dev), w.to(dev), None if s is None else s.to(dev)
+
+
+def _check(out, y0, x, w, s, K):
+    xd, wd = x.double(), w.double() * (1 if s is None else s.double()[:, None])
+    ref, mag = xd @ wd.t(), xd.abs() @ wd.abs().t()
+    if y0 is not None:
+        ref, mag = ref + y0.double(), mag + y0.double().abs()
+    bound = ((2.0 ** -16 if x.dtype == torch.float32 else 0) + (K + 2) * 2.0 ** -24) * mag + 1e-30
+    worst = ((out.double() - ref).abs() / bound).max().item()
+    print(f"  worst error / bound {worst:.3f}", flush=True)
+    assert worst <= 1
+
+
+@pytest.mark.parametrize("w8,xf", [(True, True), (False, False), (False, True), (True, False)])
+@pytest.mark.parametrize("M,N,K", [(17, 16, 16), (31, 33, 48), (32, 100, 80), (33, 2048, 512), (64, 2048, 4096),
+                                   (65, 1000, 144), (129, 4096, 2048), (300, 8192, 128), (300, 2048, 2064),
+                                   (600, 4100, 320), (1030, 8192, 192)])
+def test_mid_batch_matches_exact(dev, M, N, K, w8, xf):
+    print(f"mid M={M} N={N} K={K} w8={w8} xf={xf}", flush=True)
+    x, w, s = _operands(M, N, K, w8, xf, M + N + K, dev)
+    _check(ops.linear(x, w, s), None, x, w, s, K)
+    y0 = torch.randn(M, N, generator=torch.Generator().manual_seed(1)).to(dev)
+    out = ops.linear(x, w, s, out=y0.clone(), accumulate=True)
+    _check(out, y0, x, w, s, K)
+
+
+@pytest.mark.parametrize("w8,xf", [(True, True), (False, False)])
+def test_mid_batch_segments_and_strides(dev, w8, xf):
+    """Four weights in one launch (sizes that end inside a tile), X rows inside wider rows and
+    outputs whose rows are not 16-byte aligned."""
+    M, K, Ns = 50, 256, (300, 32, 7, 130)
+    ws = [_operands(M, N, K, w8, xf, N, dev) for N in Ns]
+    x = _operands(M, 1, K + 64, w8, xf, 3, dev)[0][:, :K]
+    outs = [torch.full((M, N + 3), 7.0, device=dev)[:, :N] for N in Ns]
+    ops.linear_multi(x, [w[1] for w in ws], [w[2] for w in ws] if w8 else None, outs=outs)
+    for (_, w, s), o in zip(ws, outs):
+        _check(o, None, x, w, s, K)
+        assert (o.as_strided((M, 3), (o.stride(0), 1), o.shape[1]) == 7).all()
