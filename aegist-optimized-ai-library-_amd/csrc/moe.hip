@@ -26,10 +26,15 @@
 #include "common.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace aegist {
 int launch_proj(const void* X, int x_dtype, long long ldx, const void* W, int w_dtype, const uint16_t* scale, float* Y,
                 long long ldy, int M, int N, int K, int accumulate, hipStream_t st);
+bool moe_decode_fits(int T, int D, int I, int E, int K);
+int launch_moe_decode(const float* h, const unsigned long long* eptr, const int* idx, const float* wts, int T, int D,
+                      int I, int E, int K, long long gu_s, long long gu_m, long long dn_q, long long dn_s,
+                      long long dn_m, float* act, float* ypick, hipStream_t st);
 }  // namespace aegist
 
 using namespace aegist;
@@ -69,6 +74,23 @@ __device__ __forceinline__ T ld_global(const void* p) {
     return *(const __attribute__((address_space(1))) T*)p;
 }
 
+// Maximum over the wave by DPP moves (row shifts, then row broadcasts) instead of LDS permutes, whose
+// round trips made up most of the router's rounds; the total is the last lane's. No NaN inputs.
+__device__ __forceinline__ float wave_max_dpp(float v) {
+    auto step = [](float x, auto ctrl, auto rows) {
+        return fmaxf(x, __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(x), __float_as_int(x),
+                                                                   decltype(ctrl)::value, decltype(rows)::value, 0xF, false)));
+    };
+    using std::integral_constant;
+    v = step(v, integral_constant<int, 0x111>{}, integral_constant<int, 0xF>{});  // row_shr:1
+    v = step(v, integral_constant<int, 0x112>{}, integral_constant<int, 0xF>{});
+    v = step(v, integral_constant<int, 0x114>{}, integral_constant<int, 0xF>{});
+    v = step(v, integral_constant<int, 0x118>{}, integral_constant<int, 0xF>{});
+    v = step(v, integral_constant<int, 0x142>{}, integral_constant<int, 0xA>{});  // row_bcast:15 to rows 1, 3
+    v = step(v, integral_constant<int, 0x143>{}, integral_constant<int, 0xC>{});  // row_bcast:31 to rows 2, 3
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), WAVE - 1));
+}
+
 // ---------------------------------------------------------------------------------------------
 // Router top-K over precomputed logits [T, E] (the projection kernel computes h W^T): one wave
 // per token, lane holds the probabilities of experts lane + 64 i in registers; softmax in fp32;
@@ -101,21 +123,18 @@ __global__ void __launch_bounds__(256) router_topk_kernel(const float* __restric
     float myv = 0.f;  // lane k keeps pick k
     int mye = 0;
     for (int k = 0; k < K; k++) {
-        float bv = -1.f;
+        // the largest probability of the wave, then the lowest expert that has it (experts lane + 64 i:
+        // the first i with a holder, its lowest lane); NaN and taken entries never compare greater
+        float lv = -1.f;
+#pragma unroll
+        for (int i = 0; i < NPER; i++) lv = p[i] > lv ? p[i] : lv;
+        const float bv = wave_max_dpp(lv);
         int bi = 0x7fffffff;
+        if (bv > -1.f) {
 #pragma unroll
-        for (int i = 0; i < NPER; i++)  // experts in increasing order: the first of equals wins
-            if (p[i] > bv) {
-                bv = p[i];
-                bi = lane + WAVE * i;
-            }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            const float v2 = __shfl_xor(bv, o, WAVE);
-            const int i2 = __shfl_xor(bi, o, WAVE);
-            if (v2 > bv || (v2 == bv && i2 < bi)) {
-                bv = v2;
-                bi = i2;
+            for (int i = 0; i < NPER; i++) {
+                const unsigned long long m = __ballot(p[i] == bv);
+                if (m != 0 && bi == 0x7fffffff) bi = WAVE * i + __builtin_ctzll(m);
             }
         }
 #pragma unroll
@@ -841,7 +860,20 @@ __global__ void __launch_bounds__(256) moe_combine_kernel(float* __restrict__ x,
                                                           const float* __restrict__ ysh, const float* __restrict__ h,
                                                           const uint16_t* __restrict__ wg, int D, int K) {
     __shared__ float red[8];
-    const int t = blockIdx.x, i = blockIdx.y * blockDim.x + threadIdx.x;
+    const int t = blockIdx.x, i = blockIdx.y * blockDim.x + threadIdx.x, ii = min(i, D - 1);
+    // every load is issued before the gate's reduction (a workgroup is a chain of round trips at
+    // decode sizes); dropped picks read a row that is not added
+    float v[16];
+    bool ok[16];
+#pragma unroll
+    for (int k = 0; k < 16; k++) {
+        if (k < K) {
+            const int e = idx[(size_t)t * K + k];
+            ok[k] = e >= 0 && e < E;
+            v[k] = ypick[((size_t)t * K + k) * D + ii];
+        }
+    }
+    const float x0 = x[(size_t)t * D + ii], y0 = ysh ? ysh[(size_t)t * D + ii] : 0.f;
     float gate = 0.f;
     if (ysh) {
         float a = 0.f;
@@ -849,20 +881,12 @@ __global__ void __launch_bounds__(256) moe_combine_kernel(float* __restrict__ x,
         gate = sigmoid_f(block_sum(a, red));
     }
     if (i >= D) return;
-    float v[16];
-#pragma unroll
-    for (int k = 0; k < 16; k++) {
-        if (k < K) {
-            const int e = idx[(size_t)t * K + k];
-            v[k] = (e >= 0 && e < E) ? ypick[((size_t)t * K + k) * D + i] : 0.f;
-        }
-    }
     float s = 0.f;
 #pragma unroll
     for (int k = 0; k < 16; k++)
-        if (k < K) s += v[k];
-    float r = x[(size_t)t * D + i] + s;
-    if (ysh) r += gate * ysh[(size_t)t * D + i];
+        if (k < K) s += ok[k] ? v[k] : 0.f;
+    float r = x0 + s;
+    if (ysh) r += gate * y0;
     x[(size_t)t * D + i] = r;
 }
 
@@ -1001,6 +1025,14 @@ int aegist_moe_experts(const float* h, const unsigned long long* eptr, const int
     float* as = (float*)(w + p.as);
     float* yp = (float*)(w + p.yp);
 
+    if (moe_decode_fits(T, D, I, E, K)) {
+        // fp32 activations in the place of the hi / lo parts
+        int rc = launch_moe_decode(h, eptr, idx, wts, T, D, I, E, K, off.gu_s, off.gu_m, off.dn_q, off.dn_s, off.dn_m,
+                                   (float*)ah, yp, st);
+        if (rc) return rc;
+        moe_combine_kernel<<<dim3(T, (D + 255) / 256), 256, 0, st>>>(x, yp, idx, E, ysh, h, wg, D, K);
+        return after_launch("moe_combine");
+    }
     // experts with more than 32 picks take the big-tile kernels where the shapes allow, once the
     // batch is large enough for such experts to be common (16 picks per expert on average)
     const bool big = (long long)N >= 16LL * E && D % UB == 0 && I % UB == 0 && D / 64 <= 32 && I / 64 <= 32 &&

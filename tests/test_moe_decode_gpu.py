@@ -1,0 +1,49 @@
+"""GPU parity of the experts' decode path (csrc/moe_decode.hip: up to 512 picks, at most two per expert
+on average, row lengths 512 / 1024 / 2048) against the fp64 oracle: one pick to the path's largest
+batch, experts shared by 1 to 9 picks (workgroups of 1 to 4), out-of-range ids, every row length.
+The activations enter as bf16 hi + lo and sums are fp32, as in the larger batches' tiles: bar 5e-5."""
+import pytest
+import torch
+
+from conftest import rel_err
+from oracle import mixer_ref as R
+from test_moe_gpu import _experts
+
+from aegist_mixer import ops
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T,D,I,E,K,hot,bad", [(1, 2048, 512, 1, 1, 1, False), (1, 2048, 512, 256, 8, 256, False),
+                                               (9, 2048, 512, 64, 8, 8, False), (8, 1024, 512, 32, 8, 9, True),
+                                               (9, 512, 1024, 40, 8, 12, True), (5, 512, 2048, 24, 3, 24, False),
+                                               (16, 2048, 512, 256, 8, 256, True), (64, 512, 512, 256, 8, 200, False),
+                                               (32, 1024, 1024, 256, 16, 16, False)])
+def test_moe_decode_matches_oracle(dev, T, D, I, E, K, hot, bad):
+    print(f"moe decode T={T} D={D} I={I} E={E} K={K} hot={hot} bad={bad}", flush=True)
+    g = torch.Generator().manual_seed(T * 31 + D + I)
+    rows, h = _experts(E, D, I, T + E), torch.randn(T, D, generator=g)
+    idx = torch.stack([torch.randperm(hot, generator=g)[:K] for _ in range(T)]).int()
+    if bad:
+        idx[::3, 0], idx[1::4, -1] = E + 5, -1
+    wts, x0 = torch.rand(T, K, generator=g), torch.randn(T, D, generator=g)
+    ysh, wg = torch.randn(T, D, generator=g), (torch.randn(D, generator=g) * 0.05).bfloat16()
+    x, hd, rd = x0.to(dev), h.to(dev), rows.to(dev)
+    ops.moe_experts(hd, rd, idx.to(dev), wts.to(dev), x, I, ysh=ysh.to(dev), wg=wg.to(dev))
+    torch.cuda.synchronize()
+    ref = R.moe_experts(h, rows, idx.long(), wts, D, I) + torch.sigmoid(h.double() @ wg.double())[:, None] * ysh.double()
+    err = rel_err(x.cpu().double() - x0.double(), ref)
+    print(f"  rel err {err:.2e}", flush=True)
+    assert err < 5e-5
+
+
+@pytest.mark.parametrize("T,E,K", [(3, 16, 4), (2, 64, 8), (5, 65, 16), (4, 1000, 8), (2, 2000, 3)])
+def test_router_rounds_take_the_lowest_of_equals(dev, T, E, K):
+    """Equal probabilities in lanes and registers of every distance: groups of experts share one weight
+    row, so the K picks are the lowest ids of the best groups, in order."""
+    g = torch.Generator().manual_seed(E)
+    base = torch.randn(5, 256, generator=g).bfloat16()
+    W, h = base[torch.randint(0, 5, (E,), generator=g)], torch.randn(T, 256, generator=g)
+    idx, _ = ops.router_topk(h.to(dev), W.to(dev), K)
+    ref = torch.sort(-(h.double() @ W.double().t()), dim=-1, stable=True).indices[:, :K]
+    assert torch.equal(idx.cpu().long(), ref)
