@@ -1,5 +1,5 @@
 // Projections of middling batches, Y_s[M, N_s] (+)= scale_s[n] X[M, K] W_s[N_s, K]^T for up to four
-// weights sharing X: from 17 rows of X to as many as the 256 x 256 tiles of gemm.hip leave part of
+// weights sharing X: from 3 rows of X to as many as the 256 x 256 tiles of gemm.hip leave part of
 // the chip idle for. int8 or bf16 W, fp32 or bf16 X, fp32 Y, on v_mfma_f32_16x16x32_bf16.
 //
 // What bounds it: at these sizes neither HBM (an 8192 x 2048 int8 weight is 17 MB, 3 us) nor the
@@ -301,6 +301,22 @@ constexpr MidForm kFormsF32[] = {{1, 2, 1, 8, 0.156f}, {1, 2, 2, 8, 0.18f}, {2, 
 constexpr MidForm kFormsBf16[] = {{1, 2, 1, 8, 0.100f}, {1, 2, 2, 8, 0.157f}, {1, 4, 2, 4, 0.205f}, {1, 4, 4, 2, 0.312f},
                                   {2, 4, 4, 2, 0.548f}, {2, 8, 4, 1, 0.90f},  {2, 8, 8, 1, 1.21f}};
 constexpr int kForms = 7;
+// Up to 16 rows (one 16-row tile of X), after the sized forms; chosen by rows of W and K, see small_form
+constexpr MidForm kFormsSmall[] = {{1, 1, 1, 8, 0.f}, {1, 1, 1, 4, 0.f}, {1, 1, 2, 4, 0.f}, {2, 1, 2, 4, 0.f}};
+constexpr int kSmall = 4;
+
+// Measured (us, 16 rows, weights from HBM; fp32 X with int8 W, then bf16 both), row-tile kernel -> here:
+//   8192 x 2048 9.5 -> 7.6, 10.1 -> 8.8    4096 x 2048 8.4 -> 7.0, 7.0 -> 6.1
+//   2048 x 4096 13.4 -> 9.3, 10.3 -> 7.9   512 x 2048 8.0 -> 5.5, 6.1 -> 4.9
+// 4 K groups instead of 8 where the rows alone give the chip enough waves or K is short; wider tiles
+// (X staged for more rows) from 6144 rows of W for fp32 X, whose stage costs most, and where even
+// these are more than two workgroups per CU (bf16 W, fp32 X 32768 x 2048: 36.2 -> 33.0).
+int small_form(bool f32, long long rows, int K) {
+    if (rows > 16384) return kForms + 3;
+    if (f32 ? rows >= 6144 : rows > 8192) return kForms + 2;
+    if (K <= 1024 || (!f32 && rows >= 6144)) return kForms + 1;
+    return kForms;
+}
 // the 256 x 256 tiles of gemm.hip, in the same unit: int8 W with fp32 X, bf16 W with bf16 X
 constexpr float kTile256F32 = 3.7f, kTile256Bf16 = 1.5f;
 
@@ -333,10 +349,14 @@ int run_mid(int form, const MidArgs& ga, hipStream_t st) {
         constexpr MidForm f = f32 ? kFormsF32[I] : kFormsBf16[I];                                               \
         return launch_mid<TW, TX, f.rt, f.mt, f.nwn, f.kg, 2>(ga, st);                                          \
     }
+#define AEG_MID_SMALL(I)                                                                                        \
+    case kForms + I: return launch_mid<TW, TX, kFormsSmall[I].rt, 1, kFormsSmall[I].nwn, kFormsSmall[I].kg, 2>(ga, st);
     switch (form) {
+        AEG_MID_SMALL(0) AEG_MID_SMALL(1) AEG_MID_SMALL(2) AEG_MID_SMALL(3)
         AEG_MID(0) AEG_MID(1) AEG_MID(2) AEG_MID(3) AEG_MID(4) AEG_MID(5) AEG_MID(6)
     }
 #undef AEG_MID
+#undef AEG_MID_SMALL
     return fail(AEGIST_ERR_SHAPE, "gemm_mid: no such form");
 }
 
@@ -344,20 +364,20 @@ int run_mid(int form, const MidArgs& ga, hipStream_t st) {
 
 namespace aegist {
 
-// Whether this file's kernel takes the product (`tile256`: gemm.hip's 256 x 256 tiles could take it
-// too, as one launch of all weights), and the form it takes: 17 rows or more, operands below 2 GiB,
-// and an estimate no worse than that of the 256 x 256 tiles. -1 if not. The caller has checked
-// K % 16 == 0 and the 16-byte alignment of every row.
-int gemm_mid_form(int x_dtype, long long ldx, int w_dtype, int nseg, const int* N, int M, int K, bool tile256) {
-    if (M <= 16 || nseg < 1 || nseg > MID_SEG || K <= 0) return -1;
-    const long long lim = 0x7ffffff0LL, xs = x_dtype == AEGIST_F32 ? 4 : 2, wsz = w_dtype == AEGIST_I8 ? 1 : 2;
-    if (ldx > 0x7fffffffLL || (long long)M * ldx * xs >= lim) return -1;
+// The form this file's kernel would take the product in, or -1 if the 256 x 256 tiles of gemm.hip are
+// estimated faster (`tile256`: they could take it, as one launch of all weights). Every operand is
+// below 2^31 - 16 bytes (the caller splits larger ones), K % 16 == 0, rows 16-byte aligned.
+int gemm_mid_form(int x_dtype, int nseg, const int* N, int M, int K, bool tile256) {
+    if (M <= 16) {
+        long long rows = 0;
+        for (int i = 0; i < nseg; i++) rows += N[i];
+        return small_form(x_dtype == AEGIST_F32, rows, K);
+    }
     MidArgs ga{};
     ga.nseg = nseg;
     ga.M = M;
     long long t256 = 0;
     for (int i = 0; i < nseg; i++) {
-        if ((long long)N[i] * K * wsz >= lim) return -1;
         ga.seg[i].N = N[i];
         t256 += N[i];
     }
@@ -367,7 +387,6 @@ int gemm_mid_form(int x_dtype, long long ldx, int w_dtype, int nseg, const int* 
     float least = tile256 ? ((t256 + 255) / 256) * (x_dtype == AEGIST_F32 ? kTile256F32 : kTile256Bf16) : 3.4e38f;
     for (int i = 0; i < kForms; i++) {
         const long long t = mid_tiles(forms[i], ga);
-        if (t >= (1LL << 27)) continue;
         const float est = ((t + 255) / 256) * forms[i].cost;
         if (est <= least) {
             least = est;

@@ -5,22 +5,16 @@
 //     Y[m, n] (+)= scale[n] * sum_k X[m, k] W[n, k]
 // with fp32 accumulation. accumulate = 1 adds into Y (the residual add of the out-projections).
 //
-// At decode sizes (M = batch <= 16; gemm_mid.hip takes larger batches, gemm.hip the largest) the op
-// streams the weight matrix once from HBM, so the kernel is built around that stream: each wave owns RT 16-row tiles of W and a contiguous run
-// of 64-wide k steps, loads 16 bytes of int8 weights (or 32 of bf16) per lane per step, and
-// feeds v_mfma_f32_16x16x32_bf16 with W as the A operand and X^T as the B operand, so every
-// weight byte is used by MT 16-row tiles of X at once. Four waves of a workgroup interleave
-// their k steps (neighbouring waves read neighbouring 64-byte runs of the same rows) and add
-// their partial tiles through LDS at the end, where the row scale and the accumulate are fused
-// into the store.
+// This file picks the kernel by size and holds the weight stream of decode batches. One or two rows
+// run in gemv.hip, the rest up to a few thousand in gemm_mid.hip, the largest in gemm.hip.
 //
 // int8 and bf16 weights are exact in bf16. An fp32 X is split into bf16 hi + lo
 // (x = hi + lo + O(2^-17 |x|)) and both halves go through the MFMA, so the result matches an
 // fp32 dot product to ~1e-5 relative; a bf16 X needs only the hi half.
 #include "common.h"
 
+#include <algorithm>
 #include <cstdlib>
-#include <type_traits>
 
 using namespace aegist;
 
@@ -34,7 +28,10 @@ int launch_gemm_bf16(const uint16_t* X, long long ldx, const uint16_t* W, long l
 int launch_gemm_bf16_multi(const uint16_t* X, long long ldx, int nseg, const uint16_t* const* W, const long long* ldw,
                            float* const* Y, const long long* ldy, const int* N, int M, int K, int accumulate,
                            hipStream_t st);
-int gemm_mid_form(int x_dtype, long long ldx, int w_dtype, int nseg, const int* N, int M, int K, bool tile256);
+int gemm_mid_form(int x_dtype, int nseg, const int* N, int M, int K, bool tile256);
+int launch_gemv(const void* X, int x_dtype, long long ldx, int w_dtype, int nseg, const void* const* W,
+                const uint16_t* const* scale, float* const* Y, const long long* ldy, const int* N, int M, int K,
+                int accumulate, hipStream_t st);
 int launch_gemm_mid(int form, const void* X, int x_dtype, long long ldx, int w_dtype, int nseg, const void* const* W,
                     const uint16_t* const* scale, float* const* Y, const long long* ldy, const int* N, int M, int K,
                     int accumulate, hipStream_t st);
@@ -49,109 +46,6 @@ bool stream_enabled() {
     }();
     return on;
 }
-
-constexpr int KSTEP = 64;  // k per wave step: 16 bytes of int8 (two MFMA k-blocks of 32) per lane
-#ifndef PROJ_TARGET_WAVES
-#define PROJ_TARGET_WAVES 2048  // waves per launch the shape heuristic aims for
-#endif
-
-typedef int int4v __attribute__((ext_vector_type(4)));
-
-// 16 consecutive weights of one row starting at k (zero outside the row), as two bf16x8
-// operands: lo = k .. k+7, hi = k+8 .. k+15.
-template <typename TW> struct WLoad;
-template <> struct WLoad<int8_t> {
-    int4v raw;
-    __device__ __forceinline__ void load(const int8_t* row, int k, int K, bool ok) {
-        raw = (ok && k < K) ? *(const int4v*)(row + k) : int4v{0, 0, 0, 0};
-    }
-    __device__ __forceinline__ void cvt(bf16x8& a, bf16x8& b) const {
-        // int8 -> fp32 is exact (one sign-extending byte conversion each) and |q| <= 128 keeps
-        // 8 significant bits, so the top half of the fp32 pattern is the exact bf16; one byte
-        // permute packs two of them
-        uint32_t pa[4], pb[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const uint32_t d = (uint32_t)raw[i];
-            const float f0 = (float)(int8_t)d, f1 = (float)(int8_t)(d >> 8);
-            const float f2 = (float)(int8_t)(d >> 16), f3 = (float)(int8_t)(d >> 24);
-            const uint32_t p01 = __builtin_amdgcn_perm(__float_as_uint(f1), __float_as_uint(f0), 0x07060302u);
-            const uint32_t p23 = __builtin_amdgcn_perm(__float_as_uint(f3), __float_as_uint(f2), 0x07060302u);
-            if (i < 2) {
-                pa[2 * i] = p01;
-                pa[2 * i + 1] = p23;
-            } else {
-                pb[2 * (i - 2)] = p01;
-                pb[2 * (i - 2) + 1] = p23;
-            }
-        }
-        a = __builtin_bit_cast(bf16x8, pa);
-        b = __builtin_bit_cast(bf16x8, pb);
-    }
-};
-template <> struct WLoad<uint16_t> {
-    bf16x8 r0, r1;
-    __device__ __forceinline__ void load(const uint16_t* row, int k, int K, bool ok) {
-        if (ok && k < K) {
-            r0 = *(const bf16x8*)(row + k);
-            r1 = *(const bf16x8*)(row + k + 8);
-        } else {
-            r0 = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-            r1 = r0;
-        }
-    }
-    __device__ __forceinline__ void cvt(bf16x8& a, bf16x8& b) const {
-        a = r0;
-        b = r1;
-    }
-};
-
-// 16 consecutive activations of one row of X starting at k, as bf16 hi (and lo for fp32 X).
-template <typename TX> struct XLoad;
-template <> struct XLoad<float> {
-    static constexpr bool kLo = true;
-    f32x4 r[4];
-    __device__ __forceinline__ void load(const float* row, int k, int K, bool ok) {
-#pragma unroll
-        for (int i = 0; i < 4; i++) r[i] = (ok && k < K) ? *(const f32x4*)(row + k + 4 * i) : f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-    // x = hi + lo with hi = x truncated to bf16 (exact difference) and lo rounded to bf16:
-    // |x - hi - lo| <= 2^-16 |x|
-    __device__ __forceinline__ void cvt(bf16x8& ha, bf16x8& hb, bf16x8& la, bf16x8& lb) const {
-        uint32_t h[8], l[8];
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const float x0 = r[i / 2][2 * (i % 2)], x1 = r[i / 2][2 * (i % 2) + 1];
-            h[i] = __builtin_amdgcn_perm(__float_as_uint(x1), __float_as_uint(x0), 0x07060302u);
-            typedef float f2 __attribute__((ext_vector_type(2)));
-            typedef __bf16 b2 __attribute__((ext_vector_type(2)));
-            const f2 lo = {x0 - __uint_as_float(__float_as_uint(x0) & 0xffff0000u),
-                           x1 - __uint_as_float(__float_as_uint(x1) & 0xffff0000u)};
-            l[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(lo, b2));
-        }
-        ha = __builtin_bit_cast(bf16x8, *(uint32_t(*)[4])h);
-        hb = __builtin_bit_cast(bf16x8, *(uint32_t(*)[4])(h + 4));
-        la = __builtin_bit_cast(bf16x8, *(uint32_t(*)[4])l);
-        lb = __builtin_bit_cast(bf16x8, *(uint32_t(*)[4])(l + 4));
-    }
-};
-template <> struct XLoad<uint16_t> {
-    static constexpr bool kLo = false;
-    bf16x8 r0, r1;
-    __device__ __forceinline__ void load(const uint16_t* row, int k, int K, bool ok) {
-        if (ok && k < K) {
-            r0 = *(const bf16x8*)(row + k);
-            r1 = *(const bf16x8*)(row + k + 8);
-        } else {
-            r0 = bf16x8{0, 0, 0, 0, 0, 0, 0, 0};
-            r1 = r0;
-        }
-    }
-    __device__ __forceinline__ void cvt(bf16x8& ha, bf16x8& hb, bf16x8&, bf16x8&) const {
-        ha = r0;
-        hb = r1;
-    }
-};
 
 // Up to four weight matrices that share X (a layer's input projections) go in one launch;
 // segment i owns workgroups [tile0[i], tile0[i+1]) along grid x.
@@ -169,162 +63,9 @@ struct ProjSegs {
     int n;
 };
 
-// One workgroup: rows [n0, n0 + 16 RT) of one segment's W against rows [m0, m0 + 16 MT) of X,
-// all of K. grid = (total row tiles of all segments, ceil(M / 16MT)); NWAVE waves split the k
-// steps.
-template <typename TW, typename TX, int MT, int RT, int NWAVE>
-__global__ __launch_bounds__(64 * NWAVE) void proj_skinny_kernel(const TX* __restrict__ X, long long ldx,
-                                                                 const ProjSegs segs, int M, int K, int accumulate) {
-    __shared__ f32x4 red[NWAVE][RT * MT][WAVE];
-    const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
-    const int r16 = lane % 16, g = lane / 16;
-    int si = 0;
-#pragma unroll
-    for (int i = 1; i < MAX_SEG; i++)
-        if (i < segs.n && (int)blockIdx.x >= segs.tile0[i]) si = i;
-    const TW* __restrict__ W = (const TW*)segs.s[si].W;
-    const uint16_t* __restrict__ scale = segs.s[si].scale;
-    float* __restrict__ Y = segs.s[si].Y;
-    const long long ldy = segs.s[si].ldy;
-    const int N = segs.s[si].N;
-    const int n0 = ((int)blockIdx.x - segs.tile0[si]) * 16 * RT, m0 = blockIdx.y * 16 * MT;
-
-    const TW* wrow[RT];
-    bool wok[RT];
-#pragma unroll
-    for (int rt = 0; rt < RT; rt++) {
-        const int n = n0 + 16 * rt + r16;
-        wok[rt] = n < N;
-        wrow[rt] = W + (size_t)(wok[rt] ? n : 0) * K;
-    }
-    const TX* xrow[MT];
-    bool xok[MT];
-#pragma unroll
-    for (int mt = 0; mt < MT; mt++) {
-        const int m = m0 + 16 * mt + r16;
-        xok[mt] = m < M;
-        xrow[mt] = X + (size_t)(xok[mt] ? m : 0) * ldx;
-    }
-
-    f32x4 acc[RT][MT];
-#pragma unroll
-    for (int rt = 0; rt < RT; rt++)
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++) acc[rt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    // The epilogue's row scales (and, when accumulating, the old Y values) of the tiles this
-    // wave finishes (tile t by wave t % NWAVE) are requested now, so they arrive with the
-    // weights instead of costing a round trip at the end.
-    // int8 weights (always with row scales): the loads are unconditional and their values are
-    // only used in the epilogue (a guarded load whose value is used inside its branch waits for
-    // it there, before the weight stream starts; measured 6% at M = 1). Without row scales or
-    // accumulation every lane reads one word that the epilogue ignores (one cache line). bf16
-    // weights (normally without scales) keep guarded loads, which then issue nothing.
-    constexpr bool kEarly = std::is_same<TW, int8_t>::value;
-    constexpr int NFIN = (RT * MT + NWAVE - 1) / NWAVE;  // tiles finished per wave, at most
-    uint16_t sraw[NFIN][4];
-    float fsc[NFIN][4], fy[NFIN][4];
-#pragma unroll
-    for (int u = 0; u < NFIN; u++) {
-        const int t = wave + NWAVE * u, rt = t / MT, mt = t % MT;
-        const int m = m0 + 16 * mt + r16;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int n = n0 + 16 * rt + 4 * g + j;
-            const bool ok = t < RT * MT && n < N && m < M;
-            if constexpr (kEarly) {
-                const int nn = ok ? n : 0, mm = ok ? m : 0;
-                sraw[u][j] = *(scale ? scale + nn : (const uint16_t*)W);
-                fy[u][j] = *(accumulate ? Y + (size_t)mm * ldy + nn : Y);
-            } else {
-                fsc[u][j] = (ok && scale) ? bf2f(scale[n]) : 1.f;
-                fy[u][j] = (ok && accumulate) ? Y[(size_t)m * ldy + n] : 0.f;
-            }
-        }
-    }
-
-    // loads of DEPTH steps are issued together, then consumed: with ~4 steps per wave that is
-    // every load of the wave in flight at once
-    constexpr int DEPTH = (XLoad<TX>::kLo ? MT * 16 : MT * 8) + RT * 8 <= 32 ? 4 : 2;
-    WLoad<TW> wl[DEPTH][RT];
-    XLoad<TX> xl[DEPTH][MT];
-    auto fetch = [&](int buf, int step) {
-        const int k = step * KSTEP + 16 * g;
-#pragma unroll
-        for (int rt = 0; rt < RT; rt++) wl[buf][rt].load(wrow[rt], k, K, wok[rt]);
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++) xl[buf][mt].load(xrow[mt], k, K, xok[mt]);
-    };
-    auto compute = [&](int buf) {
-        bf16x8 xa[MT], xb[MT], la[MT], lb[MT];
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++) xl[buf][mt].cvt(xa[mt], xb[mt], la[mt], lb[mt]);
-#pragma unroll
-        for (int rt = 0; rt < RT; rt++) {
-            bf16x8 wa, wb;
-            wl[buf][rt].cvt(wa, wb);
-#pragma unroll
-            for (int mt = 0; mt < MT; mt++) {
-                acc[rt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa, xa[mt], acc[rt][mt], 0, 0, 0);
-                acc[rt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb, xb[mt], acc[rt][mt], 0, 0, 0);
-                if (XLoad<TX>::kLo) {
-                    acc[rt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa, la[mt], acc[rt][mt], 0, 0, 0);
-                    acc[rt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb, lb[mt], acc[rt][mt], 0, 0, 0);
-                }
-            }
-        }
-    };
-
-    // wave w takes steps w, w + NWAVE, ... (neighbouring waves read neighbouring runs of a row);
-    // steps past the end load zeros and are skipped
-    // rolling prefetch: a buffer is refilled with the step DEPTH rounds ahead as soon as it has
-    // been consumed, so the next round's loads are in flight during this round's MFMAs
-    const int nsteps = (K + KSTEP - 1) / KSTEP;
-#pragma unroll
-    for (int d = 0; d < DEPTH; d++) fetch(d, wave + d * NWAVE);
-    for (int s0 = wave; s0 < nsteps; s0 += DEPTH * NWAVE) {
-#pragma unroll
-        for (int d = 0; d < DEPTH; d++) {
-            const int st = s0 + d * NWAVE;
-            if (st < nsteps) compute(d);
-            const int nx = st + DEPTH * NWAVE;
-            if (s0 + DEPTH * NWAVE < nsteps) fetch(d, nx);  // uniform: the next round exists
-        }
-    }
-
-#pragma unroll
-    for (int rt = 0; rt < RT; rt++)
-#pragma unroll
-        for (int mt = 0; mt < MT; mt++) red[wave][rt * MT + mt][lane] = acc[rt][mt];
-    __syncthreads();
-    // tile t is finished by wave t % NWAVE: lane holds column m = m0 + 16 mt + r16, rows
-    // n 4g .. 4g+3
-#pragma unroll
-    for (int u = 0; u < NFIN; u++) {
-        const int t = wave + NWAVE * u;
-        if (t >= RT * MT) break;
-        f32x4 v = red[0][t][lane];
-#pragma unroll
-        for (int w = 1; w < NWAVE; w++) v += red[w][t][lane];
-        const int rt = t / MT, mt = t % MT;
-        const int m = m0 + 16 * mt + r16;
-        if (m >= M) continue;
-        float* yrow = Y + (size_t)m * ldy;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int n = n0 + 16 * rt + 4 * g + j;
-            if (n >= N) continue;
-            if constexpr (kEarly)
-                yrow[n] = (accumulate ? fy[u][j] : 0.f) + v[j] * (scale ? bf2f(sraw[u][j]) : 1.f);
-            else
-                yrow[n] = fy[u][j] + v[j] * fsc[u][j];
-        }
-    }
-}
-
 // ---------------------------------------------------------------------------------------------
-// Decode-size bf16 projections (M <= 16) with W staged through LDS. The row-tile pattern above
-// (lane = (row, 32-byte run)) reads 16 rows x 128 bytes per pair of load instructions, and the
+// Decode-size bf16 projections (M <= 16) with W staged through LDS. Lanes that hold (row, run)
+// fragments straight from global memory read 16 rows x 64 or 128 bytes per instruction, and the
 // DRAM side serves that at ~half the rate of contiguous reads (same box: a read-only kernel
 // with that pattern 51% of HBM on 50 MB, 1 KB-contiguous reads 67%). Here every load
 // instruction is a direct global -> LDS copy of 1 KB of one pair of W rows (512 bytes each) and
@@ -336,9 +77,9 @@ __global__ __launch_bounds__(64 * NWAVE) void proj_skinny_kernel(const TX* __res
 // each lane is permuted, the 1 KB it covers is not), so the 16 rows a fragment read touches
 // hit 16 different bank groups.
 constexpr int SKC = 256;  // k per chunk
-template <typename TX, int NW, int NS>
+template <int NW, int NS>
 struct StreamSmem {
-    static constexpr int XB = 16 * SKC * sizeof(TX);  // X bytes per stage (16 rows)
+    static constexpr int XB = 16 * SKC * 2;  // X bytes per stage (16 rows)
     __attribute__((aligned(16))) unsigned char w[NS][16 * NW][SKC * 2];
     __attribute__((aligned(16))) unsigned char x[NS][XB];
 };
@@ -351,7 +92,6 @@ __device__ __forceinline__ void g2lds16(const void* src, void* lds) {
 }
 // The same copy with the nontemporal hint (cache-policy bit 1): the weight stream is read once
 // per launch, and kept out of L2 / MALL it runs faster (config 4 decode step 1.637 -> 1.583 ms).
-// The row-tile kernel's register loads measured slower with the hint, so they keep plain loads.
 __device__ __forceinline__ void g2lds16_nt(const void* src, void* lds) {
     __builtin_amdgcn_global_load_lds(src, (__attribute__((address_space(3))) void*)lds, 16, 0, 2);
 }
@@ -369,15 +109,15 @@ __device__ __forceinline__ void wait_vm(int n) {
     }
 }
 
-template <typename TX, int NW, int NS>
-__global__ __launch_bounds__(64 * NW) void proj_stream_kernel(const TX* __restrict__ X, long long ldx,
+template <int NW, int NS>
+__global__ __launch_bounds__(64 * NW) void proj_stream_kernel(const uint16_t* __restrict__ X, long long ldx,
                                                                const ProjSegs segs, int M, int K, int accumulate,
                                                                float* __restrict__ part) {
-    __shared__ StreamSmem<TX, NW, NS> sm;
+    __shared__ StreamSmem<NW, NS> sm;
     constexpr int RW = 16 * NW;                       // W rows per workgroup
     constexpr int WI = RW / 2 / NW;                   // W load instructions per wave per stage (= 8)
-    constexpr int XI = StreamSmem<TX, NW, NS>::XB / 1024 / NW;  // X load instructions per wave per stage
-    static_assert(XI * NW * 1024 == StreamSmem<TX, NW, NS>::XB, "X stage must split evenly over the waves");
+    constexpr int XI = StreamSmem<NW, NS>::XB / 1024 / NW;  // X load instructions per wave per stage
+    static_assert(XI * NW * 1024 == StreamSmem<NW, NS>::XB, "X stage must split evenly over the waves");
     constexpr int PER = WI + XI;                      // loads per wave per stage
     const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
     const int r16 = lane % 16, g = lane / 16;
@@ -406,7 +146,7 @@ __global__ __launch_bounds__(64 * NW) void proj_stream_kernel(const TX* __restri
             const uint16_t* src = W + (size_t)n * K + (size_t)c * SKC + slot * 8;
             g2lds16_nt(src, &sm.w[st][2 * pr][0]);
         }
-        constexpr int XROWB = SKC * (int)sizeof(TX);   // bytes of one X row per chunk
+        constexpr int XROWB = SKC * 2;   // bytes of one X row per chunk
 #pragma unroll
         for (int i = 0; i < XI; i++) {
             const int off = (wave * XI + i) * 1024 + lane * 16;  // byte offset in the stage's X block
@@ -433,26 +173,8 @@ __global__ __launch_bounds__(64 * NW) void proj_stream_kernel(const TX* __restri
         for (int i = 0; i < SKC / 32; i++) {
             // k block i of the chunk: lane (row, g) takes slot 4 i + g of its row (swizzled)
             const bf16x8 a = *(const bf16x8*)&sm.w[st][row][((4 * i + g) ^ (row & 15)) * 16];
-            if constexpr (sizeof(TX) == 2) {
-                const bf16x8 b = *(const bf16x8*)&sm.x[st][(r16 * SKC + 32 * i + 8 * g) * 2];
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
-            } else {
-                const float* xp = (const float*)&sm.x[st][(r16 * SKC + 32 * i + 8 * g) * 4];
-                const f32x4 x0 = *(const f32x4*)xp, x1 = *(const f32x4*)(xp + 4);
-                uint32_t h[4], l[4];
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const float v0 = e < 2 ? x0[2 * e] : x1[2 * e - 4], v1 = e < 2 ? x0[2 * e + 1] : x1[2 * e - 3];
-                    h[e] = __builtin_amdgcn_perm(__float_as_uint(v1), __float_as_uint(v0), 0x07060302u);
-                    typedef float f2 __attribute__((ext_vector_type(2)));
-                    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
-                    const f2 lo = {v0 - __uint_as_float(__float_as_uint(v0) & 0xffff0000u),
-                                   v1 - __uint_as_float(__float_as_uint(v1) & 0xffff0000u)};
-                    l[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector(lo, b2));
-                }
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf16x8, h), acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf16x8, l), acc, 0, 0, 0);
-            }
+            const bf16x8 b = *(const bf16x8*)&sm.x[st][(r16 * SKC + 32 * i + 8 * g) * 2];
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
         }
     }
     // lane (m = r16, g) holds Y[m][n0 + 16 wave + 4 g .. +3]
@@ -481,8 +203,8 @@ __global__ __launch_bounds__(64 * NW) void proj_stream_kernel(const TX* __restri
     }
 }
 
-template <typename TX, int NW, int NS>
-int launch_stream(const TX* X, long long ldx, ProjSegs segs, int M, int K, int accumulate, hipStream_t st,
+template <int NW, int NS>
+int launch_stream(const uint16_t* X, long long ldx, ProjSegs segs, int M, int K, int accumulate, hipStream_t st,
                   float* part = nullptr, int nks = 1) {
     int t = 0;
     for (int i = 0; i < segs.n; i++) {
@@ -490,123 +212,70 @@ int launch_stream(const TX* X, long long ldx, ProjSegs segs, int M, int K, int a
         t += (segs.s[i].N + 16 * NW - 1) / (16 * NW);
     }
     segs.tile0[segs.n] = t;
-    proj_stream_kernel<TX, NW, NS><<<dim3(t, nks), 64 * NW, 0, st>>>(X, ldx, segs, M, K, accumulate, part);
+    proj_stream_kernel<NW, NS><<<dim3(t, nks), 64 * NW, 0, st>>>(X, ldx, segs, M, K, accumulate, part);
     return 0;
 }
 
-template <typename TW, typename TX, int MT, int RT, int NW>
-void launch_k(const TX* X, long long ldx, ProjSegs segs, int M, int K, int accumulate, hipStream_t st) {
-    int t = 0;
+// The kernel of a product whose operands are all below 2^31 - 16 bytes.
+int run_proj(const void* X, int xd, long long ldx, int wd, const ProjSegs& segs, int M, int K, int accumulate,
+             hipStream_t st) {
+    const bool i8 = wd == AEGIST_I8, f32 = xd == AEGIST_F32;
+    const void* W[MAX_SEG];
+    const uint16_t* scale[MAX_SEG];
+    float* Y[MAX_SEG];
+    long long ldw[MAX_SEG], ldy[MAX_SEG], rows = 0, tiles = 0;
+    int N[MAX_SEG];
+    // past 64 rows the 256 x 256 MFMA tiles take int8 weights with fp32 activations (the engine's
+    // gemm_i8, one launch per weight) and unscaled bf16 weights with bf16 activations (all weights
+    // in one launch, stacked along N, when each but the last has a multiple of 8 rows)
+    bool tile256 = M > 64 && i8 == f32, stack8 = segs.n <= 3, scaled = false;
     for (int i = 0; i < segs.n; i++) {
-        segs.tile0[i] = t;
-        t += (segs.s[i].N + 16 * RT - 1) / (16 * RT);
+        const ProjSeg& sg = segs.s[i];
+        W[i] = sg.W;
+        scale[i] = sg.scale;
+        Y[i] = sg.Y;
+        ldw[i] = K;
+        ldy[i] = sg.ldy;
+        N[i] = sg.N;
+        rows += sg.N;
+        tiles += (sg.N + 31) / 32;
+        scaled |= sg.scale != nullptr;
+        if (i8) tile256 = tile256 && gemm_i8f32_fits(X, ldx, sg.W, K, M, sg.N, K);
+        else tile256 = tile256 && !sg.scale && gemm_bf16_fits(X, ldx, sg.W, K, M, sg.N, K);
+        if (i + 1 < segs.n && sg.N % 8) stack8 = false;
     }
-    segs.tile0[segs.n] = t;
-    const dim3 grid(t, (M + 16 * MT - 1) / (16 * MT));
-    proj_skinny_kernel<TW, TX, MT, RT, NW><<<grid, 64 * NW, 0, st>>>(X, ldx, segs, M, K, accumulate);
-}
-
-// Shape of the launch: about 2048 waves in all (8 per CU, enough loads in flight to cover HBM
-// latency) with at least two k steps per wave; two row tiles per wave where that is reachable
-// (each activation load then feeds twice the weights), else one.
-template <typename TW, typename TX, int MT>
-void launch_mt(const TX* X, long long ldx, const ProjSegs& segs, int M, int K, int accumulate, hipStream_t st) {
-    const long long gy = (M + 16 * MT - 1) / (16 * MT);
-    const int nsteps = (K + KSTEP - 1) / KSTEP;
-    long long t2 = 0, t1 = 0;
-    for (int i = 0; i < segs.n; i++) {
-        t2 += (segs.s[i].N + 31) / 32 * gy;
-        t1 += (segs.s[i].N + 15) / 16 * gy;
+    // one or two rows: whole-row loads on the VALU; two rows on int8 weights of 8192 and more rows stay
+    // with the MFMA form (131072 x 2048: 63 against 78 us, 8192 x 2048 7.4 against 7.7)
+    if (M == 1 || (M == 2 && !(i8 && rows >= 8192)))
+        return launch_gemv(X, xd, ldx, wd, segs.n, W, scale, Y, ldy, N, M, K, accumulate, st);
+    // bf16 weights and activations at 3 to 16 rows, no row scales, K a multiple of the chunk: the
+    // LDS-staged stream when it takes more than one workgroup per CU (9216 x 2048, 16 rows: 11.3
+    // against 12.8 us on the MFMA form, 12352 x 2048 13.0 against 14.4; below, the K split over
+    // the waves of a workgroup keeps more loads in flight: 8192 x 2048 11.7 against 8.8 us)
+    if (M <= 16 && !i8 && !f32 && K % SKC == 0 && !scaled && tiles > 256 && stream_enabled()) {
+        launch_stream<2, 2>((const uint16_t*)X, ldx, segs, M, K, accumulate, st);
+        return after_launch("proj_stream");
     }
-    constexpr int kTarget = PROJ_TARGET_WAVES;
-#define AEG_PROJ(RT, NW) return launch_k<TW, TX, MT, RT, NW>(X, ldx, segs, M, K, accumulate, st)
-    if (t2 * 4 >= kTarget) AEG_PROJ(2, 4);
-    if (t2 * 8 >= kTarget && nsteps >= 16) AEG_PROJ(2, 8);
-    if (t1 * 4 >= kTarget) AEG_PROJ(1, 4);
-    if (t1 * 8 >= kTarget || nsteps < 32) {
-        if (nsteps >= 16) AEG_PROJ(1, 8);
-        AEG_PROJ(1, 4);
-    }
-    // sixteen waves per workgroup leave 128 registers per lane: one m tile only
-    if constexpr (MT == 1) AEG_PROJ(1, 16);
-    else AEG_PROJ(1, 8);
-#undef AEG_PROJ
-}
-
-template <typename TW, typename TX>
-int run_proj(const TX* X, long long ldx, const ProjSegs& segs, int M, int K, int accumulate, hipStream_t st) {
-    constexpr bool i8 = std::is_same<TW, int8_t>::value, f32 = std::is_same<TX, float>::value;
-    if (M > 16) {
-        const void* W[MAX_SEG];
-        const uint16_t* scale[MAX_SEG];
-        float* Y[MAX_SEG];
-        long long ldw[MAX_SEG], ldy[MAX_SEG];
-        int N[MAX_SEG];
-        // past 64 rows the 256 x 256 MFMA tiles take int8 weights with fp32 activations (the engine's
-        // gemm_i8, one launch per weight) and unscaled bf16 weights with bf16 activations (all weights
-        // in one launch, stacked along N, when each but the last has a multiple of 8 rows)
-        bool tile256 = M > 64 && i8 == f32, stack8 = segs.n <= 3;
+    const int form = gemm_mid_form(xd, segs.n, N, M, K, tile256);
+    if (form >= 0)
+        return launch_gemm_mid(form, X, xd, ldx, wd, segs.n, W, scale, Y, ldy, N, M, K, accumulate, st);
+    if (i8) {
         for (int i = 0; i < segs.n; i++) {
-            const ProjSeg& sg = segs.s[i];
-            W[i] = sg.W;
-            scale[i] = sg.scale;
-            Y[i] = sg.Y;
-            ldw[i] = K;
-            ldy[i] = sg.ldy;
-            N[i] = sg.N;
-            if (i8) tile256 = tile256 && gemm_i8f32_fits(X, ldx, sg.W, K, M, sg.N, K);
-            else tile256 = tile256 && !sg.scale && gemm_bf16_fits(X, ldx, sg.W, K, M, sg.N, K);
-            if (i + 1 < segs.n && sg.N % 8) stack8 = false;
+            int rc = launch_gemm_i8f32((const float*)X, ldx, (const int8_t*)W[i], K, scale[i], Y[i], ldy[i], M, N[i], K,
+                                       accumulate, st);
+            if (rc) return rc;
         }
-        const int form = gemm_mid_form(f32 ? AEGIST_F32 : AEGIST_BF16, ldx, i8 ? AEGIST_I8 : AEGIST_BF16, segs.n, N, M, K,
-                                       tile256);
-        if (form >= 0)
-            return launch_gemm_mid(form, X, f32 ? AEGIST_F32 : AEGIST_BF16, ldx, i8 ? AEGIST_I8 : AEGIST_BF16, segs.n, W,
-                                   scale, Y, ldy, N, M, K, accumulate, st);
-        if constexpr (i8 && f32) {
-            if (tile256) {
-                for (int i = 0; i < segs.n; i++) {
-                    int rc = launch_gemm_i8f32(X, ldx, (const int8_t*)W[i], K, scale[i], Y[i], ldy[i], M, N[i], K,
-                                               accumulate, st);
-                    if (rc) return rc;
-                }
-                return 0;
-            }
-        }
-        if constexpr (!i8 && !f32) {
-            if (tile256 && stack8)
-                return launch_gemm_bf16_multi(X, ldx, segs.n, (const uint16_t* const*)W, ldw, Y, ldy, N, M, K, accumulate,
-                                              st);
-            if (tile256) {
-                for (int i = 0; i < segs.n; i++) {
-                    int rc = launch_gemm_bf16(X, ldx, (const uint16_t*)W[i], K, Y[i], ldy[i], M, N[i], K, accumulate, st);
-                    if (rc) return rc;
-                }
-                return 0;
-            }
-        }
+        return 0;
     }
-    // bf16 weights at M <= 16 with K a multiple of the chunk, no row scales: the LDS-staged stream
-    if constexpr (std::is_same<TW, uint16_t>::value) {
-        bool scaled = false;
-        for (int i = 0; i < segs.n; i++) scaled |= segs.s[i].scale != nullptr;
-        // ... when it takes more than one workgroup per CU: at <= 256 workgroups (N <= 8192) the
-        // row-tile kernel below, with its K split over the waves of a workgroup, keeps more loads
-        // in flight (8192 x 2048: 10.9 against 11.7 us; 2048 x 4096: 10.5 against 14.9 us), and
-        // above it the row-tile kernel's 8-wave workgroups need a second round on part of the
-        // CUs (9216 x 2048: 16.3 against 12.8 us; 12352 x 2048: 16.9 against 13.3 us)
-        long long tiles = 0;
-        for (int i = 0; i < segs.n; i++) tiles += (segs.s[i].N + 31) / 32;
-        if (M <= 16 && K % SKC == 0 && !scaled && tiles > 256 && stream_enabled()) {
-            launch_stream<TX, 2, 2>(X, ldx, segs, M, K, accumulate, st);
-            return after_launch("proj_stream");
-        }
+    if (stack8)
+        return launch_gemm_bf16_multi((const uint16_t*)X, ldx, segs.n, (const uint16_t* const*)W, ldw, Y, ldy, N, M, K,
+                                      accumulate, st);
+    for (int i = 0; i < segs.n; i++) {
+        int rc = launch_gemm_bf16((const uint16_t*)X, ldx, (const uint16_t*)W[i], K, Y[i], ldy[i], M, N[i], K, accumulate,
+                                  st);
+        if (rc) return rc;
     }
-    // past 16 rows only operands that gemm_mid.hip cannot address (2 GiB and more) come here: a grid
-    // of groups of 32 rows
-    if (M <= 16) launch_mt<TW, TX, 1>(X, ldx, segs, M, K, accumulate, st);
-    else launch_mt<TW, TX, 2>(X, ldx, segs, M, K, accumulate, st);
-    return after_launch("proj_skinny");
+    return 0;
 }
 
 }  // namespace
@@ -632,14 +301,32 @@ int launch_proj_multi(const void* X, int x_dtype, long long ldx, int w_dtype, in
         segs.s[segs.n++] = ProjSeg{W[i], scale ? scale[i] : nullptr, Y[i], ldy[i], N[i]};
     }
     if (M == 0 || segs.n == 0) return 0;
-    if (w_dtype == AEGIST_I8 && x_dtype == AEGIST_F32) return run_proj<int8_t, float>((const float*)X, ldx, segs, M, K, accumulate, st);
-    if (w_dtype == AEGIST_I8 && x_dtype == AEGIST_BF16)
-        return run_proj<int8_t, uint16_t>((const uint16_t*)X, ldx, segs, M, K, accumulate, st);
-    if (w_dtype == AEGIST_BF16 && x_dtype == AEGIST_F32)
-        return run_proj<uint16_t, float>((const float*)X, ldx, segs, M, K, accumulate, st);
-    if (w_dtype == AEGIST_BF16 && x_dtype == AEGIST_BF16)
-        return run_proj<uint16_t, uint16_t>((const uint16_t*)X, ldx, segs, M, K, accumulate, st);
-    return fail(AEGIST_ERR_DTYPE, "proj: W must be AEGIST_I8 or AEGIST_BF16, X AEGIST_F32 or AEGIST_BF16");
+    if ((w_dtype != AEGIST_I8 && w_dtype != AEGIST_BF16) || (x_dtype != AEGIST_F32 && x_dtype != AEGIST_BF16))
+        return fail(AEGIST_ERR_DTYPE, "proj: W must be AEGIST_I8 or AEGIST_BF16, X AEGIST_F32 or AEGIST_BF16");
+    // the kernels address operands through 31-bit byte offsets: larger ones go in blocks of rows
+    const long long lim = 0x7ffffff0LL, ws = w_dtype == AEGIST_I8 ? 1 : 2;
+    // (rows so long that 8 of W or 3 of X pass the limit: one row of X at a time, whose kernel does not)
+    const bool huge = 8LL * K * ws >= lim || 3 * ldx * xs >= lim;
+    const long long mb = huge ? 1 : (lim - 1) / std::max(1LL, ldx * xs);
+    const long long nb = huge ? 0x7fffffffLL : std::max(8LL, (lim - 1) / std::max(1LL, K * ws) / 256 * 256);
+    if (M <= mb) {
+        bool whole = true;
+        for (int i = 0; i < segs.n; i++) whole &= segs.s[i].N <= nb;
+        if (whole) return run_proj(X, x_dtype, ldx, w_dtype, segs, M, K, accumulate, st);
+    }
+    for (long long m = 0; m < M; m += mb)
+        for (int i = 0; i < segs.n; i++)
+            for (long long n = 0; n < segs.s[i].N; n += nb) {
+                const ProjSeg& sg = segs.s[i];
+                ProjSegs one{};
+                one.n = 1;
+                one.s[0] = ProjSeg{(const char*)sg.W + n * K * ws, sg.scale ? sg.scale + n : nullptr, sg.Y + m * sg.ldy + n,
+                                   sg.ldy, (int)std::min<long long>(nb, sg.N - n)};
+                int rc = run_proj((const char*)X + m * ldx * xs, x_dtype, ldx, w_dtype, one,
+                                  (int)std::min<long long>(mb, M - m), K, accumulate, st);
+                if (rc) return rc;
+            }
+    return 0;
 }
 
 // Split-K form for decode sizes: part[ks][m][n] = sum over the ks-th of nks slices of K of
@@ -653,7 +340,7 @@ int launch_proj_splitk(const uint16_t* X, long long ldx, const uint16_t* W, floa
     ProjSegs segs{};
     segs.s[0] = ProjSeg{W, nullptr, part, N, N};
     segs.n = 1;
-    launch_stream<uint16_t, 2, 2>(X, ldx, segs, M, K, 0, st, part, nks);
+    launch_stream<2, 2>(X, ldx, segs, M, K, 0, st, part, nks);
     return after_launch("proj_stream_splitk");
 }
 

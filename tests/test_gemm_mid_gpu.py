@@ -55,3 +55,30 @@ def test_mid_batch_segments_and_strides(dev, w8, xf):
     for (_, w, s), o in zip(ws, outs):
         _check(o, None, x, w, s, K)
         assert (o.as_strided((M, 3), (o.stride(0), 1), o.shape[1]) == 7).all()
+
+
+@pytest.mark.parametrize("w8,xf", [(True, True), (False, False), (False, True), (True, False)])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 16), (1, 5, 48), (2, 515, 1040), (1, 1030, 2064), (2, 2049, 512), (1, 4099, 528),
+                                   (2, 8200, 32), (1, 8192, 2048), (3, 33, 16), (5, 100, 1040), (16, 2048, 2064),
+                                   (7, 6150, 64), (16, 8192, 512), (11, 9000, 256), (9, 16500, 80)])
+def test_small_batch_matches_exact(dev, M, N, K, w8, xf):
+    """One and two rows (csrc/gemv.hip: rows and pieces that end inside a wave's) and 3 to 16 (the small
+    forms of gemm_mid.hip, the streamed weights)."""
+    print(f"small M={M} N={N} K={K} w8={w8} xf={xf}", flush=True)
+    x, w, s = _operands(M, N, K, w8, xf, M + N + K, dev)
+    _check(ops.linear(x, w, s), None, x, w, s, K)
+    y0 = torch.randn(M, N, generator=torch.Generator().manual_seed(1)).to(dev)
+    _check(ops.linear(x, w, s, out=y0.clone(), accumulate=True), y0, x, w, s, K)
+
+
+@pytest.mark.parametrize("M", [1, 2, 6])
+@pytest.mark.parametrize("w8,xf", [(True, True), (False, False)])
+def test_small_batch_segments_and_strides(dev, M, w8, xf):
+    K, Ns = 272, (300, 32, 7, 130)
+    ws = [_operands(M, N, K, w8, xf, N, dev) for N in Ns]
+    x = _operands(M, 1, K + 64, w8, xf, 3, dev)[0][:, :K]
+    outs = [torch.full((M, N + 3), 7.0, device=dev)[:, :N] for N in Ns]
+    ops.linear_multi(x, [w[1] for w in ws], [w[2] for w in ws] if w8 else None, outs=outs)
+    for (_, w, s), o in zip(ws, outs):
+        _check(o, None, x, w, s, K)
+        assert (o.as_strided((M, 3), (o.stride(0), 1), o.shape[1]) == 7).all()
