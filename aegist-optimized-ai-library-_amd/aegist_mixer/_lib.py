@@ -139,10 +139,16 @@ def lib():
     return _lib
 
 
+_fns: dict = {}  # bound entry points by name (an attribute lookup per call costs about a microsecond)
+
+
 def call(name: str, *args) -> None:
-    fn = getattr(lib(), name, None)
+    fn = _fns.get(name)
     if fn is None:
-        raise AegistError(name, -99, "symbol not exported by this build of libaegist_mixer.so")
+        fn = getattr(lib(), name, None)
+        if fn is None:
+            raise AegistError(name, -99, "symbol not exported by this build of libaegist_mixer.so")
+        _fns[name] = fn
     rc = fn(*args)
     if rc != 0:
         raise AegistError(name, rc, lib().aegist_last_error().decode(errors="replace"))

@@ -38,8 +38,11 @@ def _need_contig(*ts):
             raise AegistError("layout", -1, "tensor must be contiguous")
 
 
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+def _stream(device=None) -> int:
+    """Raw handle of the current stream of `device` (of the current device if None), without building
+    a torch.cuda.Stream object per launch (batch-1 calls are bound by such host work)."""
+    index = torch.cuda.current_device() if device is None or device.index is None else device.index
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 _ws_cache: dict[tuple, torch.Tensor] = {}
@@ -51,7 +54,7 @@ def _workspace(nbytes: int, device) -> torch.Tensor:
     One buffer per (device, current stream), so calls on different streams never share scratch
     bytes, and reuse on one stream is ordered by that stream; a replaced buffer is released
     through torch's stream-ordered caching allocator."""
-    key = (str(device), torch.cuda.current_stream(device).cuda_stream)
+    key = (device, _stream(device))
     ws = _ws_cache.get(key)
     if ws is None or ws.numel() < nbytes:
         ws = torch.empty(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
@@ -441,7 +444,8 @@ def expert_pointers(experts):
     """Device array of expert-row addresses for a contiguous uint8 [E, row_bytes] expert tensor."""
     E, rb = experts.shape
     base = experts.data_ptr()
-    return torch.tensor([base + e * rb for e in range(E)], dtype=torch.int64, device=experts.device)
+    # filled on the device: a host list would be copied over, and the caller would wait for the copy
+    return torch.arange(base, base + E * rb, rb, dtype=torch.int64, device=experts.device)
 
 
 def moe_experts(h, experts, idx, wts, x, I: int, ysh=None, wg=None, eptr=None):
@@ -490,8 +494,10 @@ def moe_forward(h, x, router_w, experts, I: int, K: int, shared=None, shared_gat
     ysh = None
     if shared is not None:
         (wgt, sg), (wup, su), (wdn, sd) = shared
-        g = linear(h, wgt, sg)
-        u = linear(h, wup, su)
+        if wgt.dtype == wup.dtype and (sg is None) == (su is None):  # one launch for both
+            g, u = linear_multi(h, [wgt, wup], None if sg is None else [sg, su])
+        else:
+            g, u = linear(h, wgt, sg), linear(h, wup, su)
         ysh = linear(silu_mul(g, u), wdn, sd)
     moe_experts(h, experts, idx, wts, x, I, ysh=ysh, wg=shared_gate if shared is not None else None)
     return idx, wts
