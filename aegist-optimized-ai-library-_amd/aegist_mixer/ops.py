@@ -441,10 +441,18 @@ def router_topk(h, W, K: int):
 
 
 def expert_pointers(experts):
-    """Device array of expert-row addresses for a contiguous uint8 [E, row_bytes] expert tensor."""
+    """Device array of expert-row addresses for a contiguous uint8 [E, row_bytes] expert tensor,
+    complete on return (usable from any stream): a table that a program makes once and keeps."""
     E, rb = experts.shape
     base = experts.data_ptr()
-    # filled on the device: a host list would be copied over, and the caller would wait for the copy
+    return torch.tensor([base + e * rb for e in range(E)], dtype=torch.int64, device=experts.device)
+
+
+def _expert_pointers_here(experts):
+    """The same table for use on the current stream: filled by a kernel, so a call that makes its own
+    table does not wait for a transfer."""
+    E, rb = experts.shape
+    base = experts.data_ptr()
     return torch.arange(base, base + E * rb, rb, dtype=torch.int64, device=experts.device)
 
 
@@ -458,7 +466,7 @@ def moe_experts(h, experts, idx, wts, x, I: int, ysh=None, wg=None, eptr=None):
     T, D = h.shape
     K = idx.shape[1]
     if eptr is None:
-        eptr = expert_pointers(experts)
+        eptr = _expert_pointers_here(experts)
     E = eptr.numel()
     need = lib().aegist_moe_workspace_bytes(T, K, D, I, E)
     ws = torch.empty(need, dtype=torch.uint8, device=h.device)

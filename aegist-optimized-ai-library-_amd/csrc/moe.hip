@@ -153,13 +153,17 @@ __global__ void __launch_bounds__(256) router_topk_kernel(const float* __restric
 }
 
 // ---------------------------------------------------------------------------------------------
-// Grouping (one workgroup of 1024 threads): picks i = t K + k with expert idx[i]; out of range
-// experts are dropped and counted. eoff[E + 1]: exclusive prefix of the counts; ptok / psrc:
-// token and pick index of each grouped position. An expert's positions are cut into blocks
-// (moe_group_kernel): blocks of <= 16 positions go to tiles1 (meta[0] of them), of 17..32 to
-// tiles2 (meta[2]), of up to 64 to tiles3 (meta[3]), as (expert, p0, p1). meta[1] = dropped
-// picks. The order of positions inside an expert is unspecified (atomics); no result depends on
-// it (every pick's sums run in the same order whatever tile it lands in with whom).
+// Grouping: picks i = t K + k with expert idx[i]; out of range experts are dropped and counted.
+// eoff[E + 1]: exclusive prefix of the counts; ptok / psrc: token and pick index of each grouped
+// position. Two launches, each over blocks of `per` picks: moe_count_kernel counts the block's picks per
+// expert in LDS (its other workgroups split the activations), moe_place_kernel adds the blocks'
+// counts up, scans them over the experts and places its block's picks. (One workgroup doing all of it
+// took 32 us for 16384 picks, twice through LDS atomics; 8 us each in blocks of 1024, the activation
+// split's 8 us included.)
+// An expert's positions are cut into tiles: in big mode all into ceil(c / 64) balanced ones (tiles3,
+// meta[3] of them), else into blocks of 17..32 (tiles2, meta[2]) and a last one of <= 16 (tiles1,
+// meta[0]). meta[1] = dropped picks. The order of positions inside an expert is unspecified (atomics);
+// no result depends on it (every pick's sums run in the same order whatever tile it lands in with whom).
 __device__ __forceinline__ int block_excl_scan(int v, int* wsum, int* total) {
     const int lane = threadIdx.x % WAVE, w = threadIdx.x / WAVE, nw = blockDim.x / WAVE;
     int x = v;
@@ -180,54 +184,77 @@ __device__ __forceinline__ int block_excl_scan(int v, int* wsum, int* total) {
     return off + x - v;
 }
 
-// Tiles: with `big3` set, an expert with more than 32 picks has them all in ceil(c / 64) blocks
-// of balanced size (tiles3, 33..64 picks each but for c = 65..95: 32..48); otherwise blocks of
-// PB = 32 (tiles2) and a last one of <= 16 (tiles1).
-__global__ void __launch_bounds__(1024) moe_group_kernel(const int* __restrict__ idx, int N, int K, int E,
+__device__ __forceinline__ void xprep_chunk(long long q, long long nq, const float* __restrict__ h,
+                                            uint16_t* __restrict__ xh, uint16_t* __restrict__ xl, float* __restrict__ xs);
+
+__global__ void __launch_bounds__(256) moe_count_kernel(const int* __restrict__ idx, int N, int E, int per, int nb,
+                                                        int* __restrict__ cnt, const float* __restrict__ h, int T, int D,
+                                                        uint16_t* __restrict__ xh, uint16_t* __restrict__ xl,
+                                                        float* __restrict__ xs) {
+    __shared__ int c[MAX_E];
+    const int b = blockIdx.x;
+    if (b >= nb) {
+        xprep_chunk((long long)(b - nb) * blockDim.x + threadIdx.x, (long long)T * (D / 8), h, xh, xl, xs);
+        return;
+    }
+    for (int e = threadIdx.x; e < E; e += blockDim.x) c[e] = 0;
+    __syncthreads();
+    for (int i = b * per + threadIdx.x; i < min(N, (b + 1) * per); i += blockDim.x) {
+        const int e = idx[i];
+        if (e >= 0 && e < E) atomicAdd(&c[e], 1);
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < E; e += blockDim.x) cnt[(size_t)b * E + e] = c[e];
+}
+
+__global__ void __launch_bounds__(1024) moe_place_kernel(const int* __restrict__ idx, int N, int K, int E, int per, int nb,
+                                                         const int* __restrict__ cnt,
                                                          const unsigned long long* __restrict__ eptr,
                                                          int* __restrict__ eoff, int* __restrict__ ptok,
                                                          int* __restrict__ psrc, MoeTile* __restrict__ tiles1,
                                                          MoeTile* __restrict__ tiles2, MoeTile* __restrict__ tiles3,
                                                          int big3, int* __restrict__ meta) {
-    __shared__ int cnt[MAX_E], cur[MAX_E], wsum[16], bad;
-    const int tid = threadIdx.x;
-    for (int e = tid; e < MAX_E; e += blockDim.x) cnt[e] = 0;
-    if (tid == 0) bad = 0;
-    __syncthreads();
-    for (int i = tid; i < N; i += blockDim.x) {
-        const int e = idx[i];
-        if (e >= 0 && e < E) atomicAdd(&cnt[e], 1);
-        else atomicAdd(&bad, 1);
-    }
-    __syncthreads();
-    const int c = tid < E ? cnt[tid] : 0;
-    const int n3 = big3 && c > 32 ? (c + PBB - 1) / PBB : 0;
-    const int c3 = n3 > 0 ? c : 0, cr = c - c3, rem = cr % PB;
-    const int small = rem > 0 && rem <= 16 ? 1 : 0;      // the last block, if it is small
-    const int big = cr / PB + (rem > 16 ? 1 : 0);        // full blocks and a large last block
-    int tot_c, tot_1, tot_2, tot_3;
-    const int off = block_excl_scan(c, wsum, &tot_c);
-    const int off1 = block_excl_scan(small, wsum, &tot_1);
-    const int off2 = block_excl_scan(big, wsum, &tot_2);
-    const int off3 = block_excl_scan(n3, wsum, &tot_3);
+    __shared__ int cur[MAX_E], wsum[16];
+    const int tid = threadIdx.x, b = blockIdx.x;
+    int c = 0, mine = 0;  // the expert's picks; those of the blocks before this one
     if (tid < E) {
-        eoff[tid] = off;
-        cur[tid] = off;
-        const unsigned long long base = c > 0 ? eptr[tid] : 0ull;
-        for (int j = 0; j < n3; j++) tiles3[off3 + j] = MoeTile{base, off + c3 * j / n3, off + c3 * (j + 1) / n3};
-        for (int j = 0; j < big; j++)
-            tiles2[off2 + j] = MoeTile{base, off + c3 + j * PB, off + c3 + min(cr, (j + 1) * PB)};
-        if (small) tiles1[off1] = MoeTile{base, off + c - rem, off + c};
+#pragma unroll 8
+        for (int k = 0; k < nb; k++) {
+            const int v = cnt[(size_t)k * E + tid];
+            mine += k < b ? v : 0;
+            c += v;
+        }
     }
-    if (tid == 0) {
-        eoff[E] = tot_c;
-        meta[0] = tot_1;
-        meta[1] = bad;
-        meta[2] = tot_2;
-        meta[3] = tot_3;
+    int tot_c;
+    const int off = block_excl_scan(c, wsum, &tot_c);
+    if (tid < E) cur[tid] = off + mine;
+    if (b == 0) {
+        const int n3 = big3 ? (c + PBB - 1) / PBB : 0;
+        const int c3 = n3 > 0 ? c : 0, cr = c - c3, rem = cr % PB;
+        const int small = rem > 0 && rem <= 16 ? 1 : 0;      // the last block, if it is small
+        const int big = cr / PB + (rem > 16 ? 1 : 0);        // full blocks and a large last block
+        int tot_1, tot_2, tot_3;
+        const int off1 = block_excl_scan(small, wsum, &tot_1);
+        const int off2 = block_excl_scan(big, wsum, &tot_2);
+        const int off3 = block_excl_scan(n3, wsum, &tot_3);
+        if (tid < E) {
+            eoff[tid] = off;
+            const unsigned long long base = c > 0 ? eptr[tid] : 0ull;
+            for (int j = 0; j < n3; j++) tiles3[off3 + j] = MoeTile{base, off + c3 * j / n3, off + c3 * (j + 1) / n3};
+            for (int j = 0; j < big; j++)
+                tiles2[off2 + j] = MoeTile{base, off + c3 + j * PB, off + c3 + min(cr, (j + 1) * PB)};
+            if (small) tiles1[off1] = MoeTile{base, off + c - rem, off + c};
+        }
+        if (tid == 0) {
+            eoff[E] = tot_c;
+            meta[0] = tot_1;
+            meta[1] = N - tot_c;
+            meta[2] = tot_2;
+            meta[3] = tot_3;
+        }
     }
     __syncthreads();
-    for (int i = tid; i < N; i += blockDim.x) {
+    for (int i = b * per + tid; i < min(N, (b + 1) * per); i += blockDim.x) {
         const int e = idx[i];
         if (e < 0 || e >= E) continue;
         const int pos = atomicAdd(&cur[e], 1);
@@ -260,11 +287,8 @@ __device__ __forceinline__ void split8(const float* v, uint4& hi, uint4& lo, flo
     lo = uint4{L[0], L[1], L[2], L[3]};
 }
 
-__global__ void __launch_bounds__(256) moe_xprep_kernel(const float* __restrict__ h, int T, int D,
-                                                        uint16_t* __restrict__ xh, uint16_t* __restrict__ xl,
-                                                        float* __restrict__ xs) {
-    const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;  // chunk index
-    const long long nq = (long long)T * (D / 8);
+__device__ __forceinline__ void xprep_chunk(long long q, long long nq, const float* __restrict__ h,
+                                            uint16_t* __restrict__ xh, uint16_t* __restrict__ xl, float* __restrict__ xs) {
     const bool ok = q < nq;
     const long long qq = ok ? q : nq - 1;
     const float* src = h + qq * 8;
@@ -587,96 +611,216 @@ __global__ void __launch_bounds__(256, 2) moe_down_kernel(const MoeTile* __restr
 }
 
 // ---------------------------------------------------------------------------------------------
-// Prefill-sized tiles (up to 64 picks of an expert with more than 32): a workgroup of 4 waves covers UB = 128 rows
-// of the output (gate / up: 128 units, i.e. 128 gate and 128 up rows; down: 128 output rows) for
-// all the tile's picks. Each wave owns 32 rows of every matrix (RT 16-row tiles in all) and walks
-// the 64-groups in order; the picks' activations of one group (hi and lo, 64 picks x 64 values)
-// are staged once per workgroup in LDS by direct global -> LDS loads (double-buffered, 16-byte
-// slots XOR-swizzled by the pick row), so each activation byte is fetched once per workgroup and
-// each code byte once per tile, against once per 32 picks and once per 16 rows in the kernels
-// above. Per group and row tile the 4 x 2 x 2 products on the group's codes give P, and the lane
-// adds s P + (m - 128 s) X into its accumulators, the same fp32 formula as expert_block.
-constexpr int NWB = 4;         // waves per big workgroup (two workgroups per CU)
-constexpr int UB = 32 * NWB;   // rows per matrix per big workgroup
+// Prefill-sized batches: every expert's picks in tiles of up to 64. A workgroup of 8 waves covers 512
+// code rows for a tile's picks (gate / up: 256 units, i.e. 256 gate and 256 up rows; down: 512 output
+// rows), each wave 64 rows as 4 row tiles, walking the 64-groups in order; the picks' activations of a
+// group (hi and lo, 64 picks x 64 values) are staged once per workgroup in LDS (double-buffered, 16-byte
+// slots XOR-swizzled by the pick row), so an activation byte is fetched once per workgroup and a
+// code byte once per tile.
+//
+// Bound by the VALU beside the products (batch 2048: matrix cores busy 28% and vector units 42% of the
+// cycles in the earlier form, which spent 6 vector instructions per product). Kept out of the loop:
+//   - the min's term sum_g m X, which is itself a matrix product over the groups: it starts the
+//     accumulators, m as two bf16 parts and the fp32 group sums X as three (both exact), 6 products
+//     per tile instead of 4 FMAs per group and tile;
+//   - the 128 of the codes: a group's products start from -128 X (one splat per pick tile and group, the
+//     C operand of every row tile's first product), so what leaves them is sum c x, and the scale is
+//     applied by one mixed-precision FMA per value with the fp16 scale as it stands;
+//   - column tiles without picks: NT = 1 .. 4 by the tile's count.
+// The codes stay two groups ahead over an LDS-only barrier per pair of groups.
+// Measured, batch 2048 (gate / up + down, profiled): 331 + 205 us before, 265 + 175 us now; with neither
+// codes, activations nor LDS reads in the loop the whole op still takes 380 of its 415 us: the products
+// and the vector work of the two waves of a SIMD overlap poorly (28% and 25% busy), and a workgroup's
+// start is 8 us of its 40 (down) to 100 (gate / up).
+constexpr int NWB = 8;         // waves per big workgroup (one workgroup per CU)
+constexpr int RTB = 4;         // row tiles per wave
+constexpr int UB = 32 * NWB;   // units per gate / up workgroup
+constexpr int OB = 64 * NWB;   // output rows per down workgroup
 
-// Rows of sc and gs are padded by one word so that the rows one read touches (4 apart in sc, 1
-// apart in gs) fall in different banks.
-struct BigSmem {
-    uint32_t sc[2 * UB * 33];                // (s | m << 16) fp16 pairs, [matrix row][group], G <= 32
-    float gs[PBB * 33];                      // activation group sums [pick][group], G <= 32
-};
+// Scales and group sums lie group-major: a lane's 4 rows of scales are one 8-byte read, the picks' sums
+// 16 consecutive words, and every offset is a constant.
+constexpr int BSR = 64 * NWB + 4, BGR = PBB;
 constexpr int kActBytes = 2 * PBB * 128;     // one group's activations: hi, lo x 64 picks x 128 B
+struct BigSmem {
+    __attribute__((aligned(1024))) unsigned char act[2][2][kActBytes];  // two pairs of groups
+    __attribute__((aligned(16))) uint16_t sc[32 * BSR];  // fp16 scales [group][wave's row], G <= 32
+    float gs[32 * BGR];                      // activation group sums [group][pick]
+    float red[NWB][PBB];
+};
 
-// Stage (s, m) pairs of nrow rows (row0 .. row0 + nrow) x G groups as packed fp16 pairs, rows
-// G + 1 words apart.
-__device__ __forceinline__ void stage_sc_packed(uint32_t* sc, const uint16_t* __restrict__ s,
-                                                const uint16_t* __restrict__ mn, long long row0, int nrow, int G) {
-    const uint16_t* s0 = s + (size_t)row0 * G;
-    const uint16_t* m0 = mn + (size_t)row0 * G;
-    const int n8 = nrow * G / 8;
-    typedef uint32_t u4v __attribute__((ext_vector_type(4)));
-    for (int i = threadIdx.x; i < n8; i += blockDim.x) {
-        const u4v sv = ld_global<u4v>(s0 + 8 * i), mv = ld_global<u4v>(m0 + 8 * i);
-        const uint32_t sw[4] = {sv.x, sv.y, sv.z, sv.w}, mw[4] = {mv.x, mv.y, mv.z, mv.w};
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-            const int k = 8 * i + e;  // row k / G, group k % G
-            sc[k + k / G] = ((sw[e / 2] >> (16 * (e & 1))) & 0xffffu) | (((mw[e / 2] >> (16 * (e & 1))) & 0xffffu) << 16);
-        }
-    }
-}
-
-// The big-tile block: RT row tiles per wave (codes of row tile rt at code row qrow[rt] + lane n,
-// scales at LDS row srow[rt] + .. of sc), activations of pick rows xrow(p) (element offset of the
-// pick's row in xh / xl), groups [0, G). acc[rt][t]: lane (n, g) holds rows 4 g + j, pick 16 t + n.
-template <int RT>
-__device__ __forceinline__ void big_block(const unsigned char* __restrict__ qbase, const long long (&qrow)[RT],
-                                          const int (&srow)[RT], int Kdim, const uint16_t* __restrict__ xh,
-                                          const uint16_t* __restrict__ xl, const long long* __restrict__ xrow8,
-                                          const uint32_t* sc, const float* gs, int G, unsigned char* act0,
-                                          unsigned char* act1, f32x4 (&acc)[RT][4]) {
+// The tile's sums: acc[rt][t] of lane (n, g) = rows qrow[rt] + 4 g + j, pick 16 t + n, over the G groups of
+// Kdim codes. row_of(pick): its row in xh / xl; sc_row(r): the code row of LDS scale row r (the wave's rows
+// are 64 wave + 16 rt + ..); gs_of(pick, group): its group sum. A workgroup's start is a chain of round
+// trips that its few groups have to pay for (down: 8), so every load of the start is issued before the
+// first is used, and one barrier publishes all that is staged.
+template <int NT, typename RowOf, typename ScRow, typename GsOf>
+__device__ __forceinline__ void big_block(BigSmem& sm, RowOf row_of, ScRow sc_row, GsOf gs_of,
+                                          const unsigned char* __restrict__ qbase, const unsigned char* __restrict__ sbase,
+                                          const unsigned char* __restrict__ mbase, const int (&qrow)[RTB], int Kdim,
+                                          const uint16_t* __restrict__ xh, const uint16_t* __restrict__ xl, int G,
+                                          f32x4 (&acc)[RTB][4]) {
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / WAVE), lane = tid % WAVE;
     const int n = lane % 16, g = lane / 16;
-#pragma unroll
-    for (int rt = 0; rt < RT; rt++)
-#pragma unroll
-        for (int t = 0; t < 4; t++) acc[rt][t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const size_t rowbytes = Kdim / 2;
-    const unsigned char* arow[RT];
-#pragma unroll
-    for (int rt = 0; rt < RT; rt++) arow[rt] = qbase + (size_t)(qrow[rt] + n) * rowbytes + 8 * g;
     typedef uint32_t u2v __attribute__((ext_vector_type(2)));
-    // activation pieces: 16 per group (8 per array, 8 picks x 128 B each), 16 / NWB per wave;
-    // lane L of piece q (pick 8 (q % 8) + L / 8) fetches the global 16-byte slot (L % 8) ^ sw(pick)
-    // so that LDS slot L % 8 of the pick's row holds it
+    typedef uint32_t u4w __attribute__((ext_vector_type(4)));
+    unsigned arow[RTB];
+#pragma unroll
+    for (int rt = 0; rt < RTB; rt++) arow[rt] = (unsigned)(qrow[rt] + n) * (Kdim / 2) + 8 * g;
+    // activation pieces: 16 per group (8 per part, 8 picks x 128 B each), 16 / NWB per wave (pieces of
+    // picks past the tile's column tiles are skipped: uniform); lane L of piece q holds slot L % 8 of pick
+    // 8 (q % 8) + L / 8, which goes to LDS slot (L % 8) ^ sw(pick). Through registers: with direct
+    // global -> LDS copies the compiler drains every load in flight, the codes' prefetch too, at each
+    // group's barrier
     constexpr int PPW = 16 / NWB;
-    const uint16_t* src[PPW];
+    unsigned src[PPW];
+    int dst[PPW];
 #pragma unroll
     for (int u = 0; u < PPW; u++) {
         const int q = PPW * wave + u, pk = 8 * (q % 8) + lane / 8;
-        src[u] = (q < 8 ? xh : xl) + xrow8[pk] + ((lane % 8) ^ ((pk >> 1) & 7)) * 8;
+        src[u] = (unsigned)row_of(pk) * (2 * Kdim) + (lane % 8) * 16;
+        dst[u] = (q / 8 * PBB + pk) * 128 + ((lane % 8) ^ ((pk >> 1) & 7)) * 16;
     }
-    typedef __attribute__((address_space(3))) void lds_void;
-    auto stage = [&](unsigned char* buf, int grp) {
+    u4w st[2][PPW];  // a pair of groups in flight
+    auto fetch = [&](int set, int grp) {
+#pragma unroll
+        for (int u = 0; u < PPW; u++) {
+            const int q = PPW * wave + u;
+            if ((q % 8) < 2 * NT)
+                st[set][u] = ld_global<u4w>((const unsigned char*)(q < 8 ? xh : xl) + (src[u] + 128 * min(grp, G - 1)));
+        }
+    };
+    auto store = [&](int set, unsigned char* buf) {
 #pragma unroll
         for (int u = 0; u < PPW; u++)
-            __builtin_amdgcn_global_load_lds(src[u] + 64 * grp, (lds_void*)(buf + (PPW * wave + u) * 1024), 16, 0, 0);
+            if (((PPW * wave + u) % 8) < 2 * NT) *(u4w*)(buf + dst[u]) = st[set][u];
     };
     // codes of group grp for every row tile (ring of 2 groups)
-    u2v ar[2][RT];
+    u2v ar[2][RTB];
+    fetch(0, 0);
+    fetch(1, 1);
 #pragma unroll
     for (int u = 0; u < 2; u++)
 #pragma unroll
-        for (int rt = 0; rt < RT; rt++) ar[u][rt] = ld_global<u2v>(arow[rt] + 32 * min(u, G - 1));
-    stage(act0, 0);
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-    auto group = [&](const unsigned char* cur, unsigned char* nxt, int grp, int slot) {
-        if (grp + 1 < G) stage(nxt, grp + 1);
-        // this group's activation fragments: pick tile t, k step ks: LDS slot (2 g + ks) ^ sw(row)
-        bf16x8 bh[4][2], bl[4][2];
+        for (int rt = 0; rt < RTB; rt++) ar[u][rt] = ld_global<u2v>(qbase + (arow[rt] + 32 * min(u, G - 1)));
+    // the row mins of groups 8 g .. 8 g + 7, all requested at once (clamped: a guarded load waits in its branch)
+    u4w mraw[RTB];
+    if (G % 8 == 0) {
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
+        for (int rt = 0; rt < RTB; rt++)
+            mraw[rt] = ld_global<u4w>(mbase + ((unsigned)(qrow[rt] + n) * G + min(8 * g, G - 8)) * 2);
+    } else {
+#pragma unroll
+        for (int rt = 0; rt < RTB; rt++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const unsigned row = (unsigned)(qrow[rt] + n) * G;
+                const uint32_t a = ld_global<uint16_t>(mbase + (row + min(8 * g + 2 * e, G - 1)) * 2);
+                const uint32_t b = ld_global<uint16_t>(mbase + (row + min(8 * g + 2 * e + 1, G - 1)) * 2);
+                mraw[rt][e] = a | (b << 16);
+            }
+    }
+    // scales: 8 halves of a row per piece, G / 8 (rounded up) pieces a row; group sums: 64 picks a group
+    constexpr int NTH = 64 * NWB, SMAX = 64 * NWB * 32 / 8 / NTH, GMAX = PBB * 32 / NTH;
+    u4w sv[SMAX];
+    float gv[GMAX];
+    const int npc = 64 * NWB * G / 8;
+#pragma unroll
+    for (int u = 0; u < SMAX; u++) {
+        const int i = min(tid + NTH * u, npc - 1), r = 8 * i / G;  // a piece may end in the next row: the same run
+        if (NTH * u < npc) sv[u] = ld_global<u4w>(sbase + ((unsigned)sc_row(r / 32 * 32) * G + (8 * i - r / 32 * 32 * G)) * 2);
+    }
+#pragma unroll
+    for (int u = 0; u < GMAX; u++) {
+        const int i = tid + NTH * u;
+        if (NTH * u < PBB * G) gv[u] = gs_of(i % PBB, min(i / PBB, G - 1));
+    }
+    store(0, sm.act[0][0]);
+    store(1, sm.act[0][1]);
+#pragma unroll
+    for (int u = 0; u < SMAX; u++) {
+        const int i = tid + NTH * u;
+        if (i < npc) {
+#pragma unroll
+            for (int e = 0; e < 8; e++)
+                sm.sc[(8 * i + e) % G * BSR + (8 * i + e) / G] = (uint16_t)(sv[u][e / 2] >> (16 * (e & 1)));
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < GMAX; u++) {
+        const int i = tid + NTH * u;
+        if (i < PBB * G) sm.gs[i / PBB * BGR + i % PBB] = gv[u];
+    }
+    fetch(0, 2);
+    fetch(1, 3);
+    lds_barrier();
+    // acc = sum over groups of m X: A = m [row][8 g .. 8 g + 7], B = X [pick][same groups], zeros past G
+    {
+        bf16x8 xb[3][NT];
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+            uint32_t p1[4], p2[4], p3[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                float x[2], r[2], q[2];
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const int k = 8 * g + 2 * e + h;
+                    const float xk = sm.gs[min(k, G - 1) * BGR + 16 * t + n];
+                    x[h] = k < G ? xk : 0.f;
+                    r[h] = x[h] - __uint_as_float(__float_as_uint(x[h]) & 0xffff0000u);
+                    q[h] = r[h] - __uint_as_float(__float_as_uint(r[h]) & 0xffff0000u);
+                }
+                p1[e] = __builtin_amdgcn_perm(__float_as_uint(x[1]), __float_as_uint(x[0]), 0x07060302u);
+                p2[e] = __builtin_amdgcn_perm(__float_as_uint(r[1]), __float_as_uint(r[0]), 0x07060302u);
+                p3[e] = f2bf2(q[0], q[1]);
+            }
+            xb[0][t] = __builtin_bit_cast(bf16x8, p1);
+            xb[1][t] = __builtin_bit_cast(bf16x8, p2);
+            xb[2][t] = __builtin_bit_cast(bf16x8, p3);
+        }
+#pragma unroll
+        for (int rt = 0; rt < RTB; rt++) {
+            uint32_t hi[4], lo[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                float m[2], l[2];
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    m[h] = 8 * g + 2 * e + h < G ? h2f((uint16_t)(mraw[rt][e] >> (16 * h))) : 0.f;
+                    l[h] = m[h] - __uint_as_float(__float_as_uint(m[h]) & 0xffff0000u);
+                }
+                hi[e] = __builtin_amdgcn_perm(__float_as_uint(m[1]), __float_as_uint(m[0]), 0x07060302u);
+                lo[e] = __builtin_amdgcn_perm(__float_as_uint(l[1]), __float_as_uint(l[0]), 0x07060302u);
+            }
+            const bf16x8 ah = __builtin_bit_cast(bf16x8, hi), al = __builtin_bit_cast(bf16x8, lo);
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                f32x4 v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int p = 2; p >= 0; p--) {  // smallest parts first
+                    v = mfma_bf(al, xb[p][t], v);
+                    v = mfma_bf(ah, xb[p][t], v);
+                }
+                acc[rt][t] = v;
+            }
+#pragma unroll
+            for (int t = 0; t < NT; t++) asm volatile("" : "+v"(acc[rt][t]));
+        }
+    }
+    uint32_t mask = 0x000F000Fu, magic = 0x43004300u;
+    asm volatile("" : "+s"(mask), "+v"(magic));  // in registers: one and-or per pair of codes
+    auto codes = [&](uint32_t p) {
+        u4w d;
+#pragma unroll
+        for (int j = 0; j < 4; j++) d[j] = ((p >> (4 * j)) & mask) | magic;
+        return __builtin_bit_cast(bf16x8, d);
+    };
+    auto group = [&](int grp, int slot, const unsigned char* cur) {
+        // this group's activation fragments: pick tile t, k step ks: LDS slot (2 g + ks) ^ sw(row)
+        bf16x8 bh[NT][2], bl[NT][2];
+        f32x4 c0[NT];  // -128 X of the pick in all four rows
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
             const int row = 16 * t + n;
 #pragma unroll
             for (int ks = 0; ks < 2; ks++) {
@@ -684,95 +828,87 @@ __device__ __forceinline__ void big_block(const unsigned char* __restrict__ qbas
                 bh[t][ks] = *(const bf16x8*)(cur + off);
                 bl[t][ks] = *(const bf16x8*)(cur + PBB * 128 + off);
             }
+            const float x = -128.f * sm.gs[grp * BGR + row];
+            c0[t] = f32x4{x, x, x, x};
         }
-        float X[4];
 #pragma unroll
-        for (int t = 0; t < 4; t++) X[t] = gs[(16 * t + n) * (G + 1) + grp];
-#pragma unroll
-        for (int rt = 0; rt < RT; rt++) {
+        for (int rt = 0; rt < RTB; rt++) {
             const u2v a2 = ar[slot][rt];
-            f32x4 P[4];
+            const uint2 sv = *(const uint2*)&sm.sc[grp * BSR + 64 * wave + 16 * rt + 4 * g];
+            const bf16x8 a0 = codes(a2.x), a1 = codes(a2.y);
+            f32x4 P[NT];
 #pragma unroll
-            for (int t = 0; t < 4; t++) P[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int t = 0; t < NT; t++) P[t] = mfma_bf(a0, bh[t][0], c0[t]);
 #pragma unroll
-            for (int ks = 0; ks < 2; ks++) {
-                const bf16x8 a = codes_bf16(ks ? a2.y : a2.x);
+            for (int t = 0; t < NT; t++) P[t] = mfma_bf(a0, bl[t][0], P[t]);
 #pragma unroll
-                for (int t = 0; t < 4; t++) {
-                    P[t] = mfma_bf(a, bh[t][ks], P[t]);
-                    P[t] = mfma_bf(a, bl[t][ks], P[t]);
-                }
-            }
+            for (int t = 0; t < NT; t++) P[t] = mfma_bf(a1, bh[t][1], P[t]);
+#pragma unroll
+            for (int t = 0; t < NT; t++) P[t] = mfma_bf(a1, bl[t][1], P[t]);
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const uint32_t pr = sc[(srow[rt] + 4 * g + j) * (G + 1) + grp];
-                const float sv = h2f((uint16_t)(pr & 0xffffu)), mv = h2f((uint16_t)(pr >> 16));
-                const float mp = mv - 128.f * sv;
+                const float s = h2f((uint16_t)((j < 2 ? sv.x : sv.y) >> (16 * (j & 1))));
 #pragma unroll
-                for (int t = 0; t < 4; t++) acc[rt][t][j] = fmaf(sv, P[t][j], fmaf(mp, X[t], acc[rt][t][j]));
+                for (int t = 0; t < NT; t++) acc[rt][t][j] = fmaf(s, P[t][j], acc[rt][t][j]);
             }
-        }
-        // refill this ring slot with the codes two groups ahead (clamped: static wait counts)
+            // this row tile is done: without the fence its sums drift past the store and the barrier,
+            // with every row tile's products alive (340 spilled registers)
 #pragma unroll
-        for (int rt = 0; rt < RT; rt++) ar[slot][rt] = ld_global<u2v>(arow[rt] + 32 * min(grp + 2, G - 1));
-        // the next group's direct loads are older than the RT code loads just issued
-        __builtin_amdgcn_s_waitcnt((RT & 15) | (7 << 4) | (15 << 8));
-        __syncthreads();
+            for (int t = 0; t < NT; t++) asm volatile("" : "+v"(acc[rt][t]));
+        }
+        // refill this ring slot with the codes two groups ahead (past the end: the last group's)
+#pragma unroll
+        for (int rt = 0; rt < RTB; rt++) ar[slot][rt] = ld_global<u2v>(qbase + (arow[rt] + 32 * min(grp + 2, G - 1)));
     };
-    int grp = 0;
-    for (; grp + 2 <= G; grp += 2) {
-        group(act0, act1, grp, 0);
-        group(act1, act0, grp + 1, 1);
+    // G is even (rows of 128 codes): one barrier per pair of groups; the next pair's activations, in
+    // flight during this one, go to the other half of the buffer
+    int buf = 0;
+#pragma unroll 1
+    for (int grp = 0; grp < G; grp += 2) {
+#pragma unroll
+        for (int u = 0; u < 2; u++) group(grp + u, u, sm.act[buf][u]);
+        buf ^= 1;
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            store(u, sm.act[buf][u]);
+            fetch(u, grp + 4 + u);
+        }
+        lds_barrier();
     }
-    if (grp < G) group(act0, act1, grp, 0);
 }
 
-// Gate / up for big tiles: units [256 ub, 256 ub + 256) x one tile of <= 64 picks. act as in
+// Gate / up for big tiles: units [UB ub, UB ub + UB) x one tile of <= 64 picks. act as in
 // moe_gate_up_kernel (bf16 hi / lo in chunk order, group sums over 64 units).
-__global__ void __launch_bounds__(64 * NWB, 2) moe_gate_up_big_kernel(const MoeTile* __restrict__ tiles,
-                                                              const int* __restrict__ ntiles,
-                                                              const int* __restrict__ ptok,
-                                                              const uint16_t* __restrict__ xh,
-                                                              const uint16_t* __restrict__ xl,
-                                                              const float* __restrict__ xs, int D, int I,
-                                                              ExpertOffsets off, uint16_t* __restrict__ ah,
-                                                              uint16_t* __restrict__ al, float* __restrict__ as) {
-    __shared__ BigSmem sm;
-    __shared__ __attribute__((aligned(1024))) unsigned char act0[kActBytes];
-    __shared__ __attribute__((aligned(1024))) unsigned char act1[kActBytes];
-    __shared__ float red[NWB][PBB];
-    __shared__ long long xrow8[PBB];
-    const int ub = blockIdx.x, tile = blockIdx.y;
-    const MoeTile tl = tiles[tile];
-    if (tile >= *ntiles) return;
-    const int G = D / 64, u0 = ub * UB;
-    const int p0 = tl.p0, np = tl.p1 - tl.p0;
-    const unsigned char* base = (const unsigned char*)tl.base;
+template <int NT>
+__device__ __forceinline__ void big_gate_up(BigSmem& sm, const unsigned char* base, const ExpertOffsets& off, int p0, int np,
+                                            const int* __restrict__ ptok, const float* __restrict__ xs,
+                                            const uint16_t* __restrict__ xh, const uint16_t* __restrict__ xl, int D, int I,
+                                            uint16_t* __restrict__ ah, uint16_t* __restrict__ al, float* __restrict__ as) {
     const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE, n = lane % 16, g = lane / 16;
-    // picks past the tile repeat its last one (their results are not stored)
-    if (tid < PBB) xrow8[tid] = (long long)ptok[p0 + min(tid, np - 1)] * D;
-    stage_sc_packed(sm.sc, (const uint16_t*)(base + off.gu_s), (const uint16_t*)(base + off.gu_m), u0, UB, G);
-    stage_sc_packed(sm.sc + UB * (G + 1), (const uint16_t*)(base + off.gu_s), (const uint16_t*)(base + off.gu_m),
-                    I + u0, UB, G);
-    for (int i = tid; i < PBB * G; i += blockDim.x) {
-        const int pr = i / G, c = i % G;
-        sm.gs[pr * (G + 1) + c] = xs[(size_t)ptok[p0 + min(pr, np - 1)] * G + c];
-    }
-    __syncthreads();
+    const int ub = blockIdx.x, u0 = ub * UB;
     // wave w: units u0 + 32 w .. + 32: gate row tiles 0, 1 and up row tiles 2, 3
-    const int wu = u0 + 32 * wave;
-    const long long qrow[4] = {wu, wu + 16, I + wu, I + wu + 16};
-    const int srow[4] = {32 * wave, 32 * wave + 16, UB + 32 * wave, UB + 32 * wave + 16};
-    f32x4 acc[4][4];
-    big_block<4>(base, qrow, srow, D, xh, xl, xrow8, sm.sc, sm.gs, G, act0, act1, acc);
+    // (I is a multiple of 128: waves past it repeat the last units, unstored)
+    const bool mine = u0 + 32 * wave < I;
+    const int wu = mine ? u0 + 32 * wave : I - 32;
+    const int qrow[RTB] = {wu, wu + 16, I + wu, I + wu + 16};
+    f32x4 acc[RTB][4];
+    // picks past the tile repeat its last one (their results are not stored); LDS scale row
+    // 64 w + 32 m + r is matrix m's row u0 + 32 w + r
+    const int G = D / 64;
+    auto row_of = [&](int pk) { return ptok[p0 + min(pk, np - 1)]; };
+    auto sc_row = [&](int r) { return r / 32 % 2 * I + min(u0 + r / 64 * 32, I - 32) + r % 32; };
+    auto gs_of = [&](int pk, int k) { return xs[(size_t)row_of(pk) * G + k]; };
+    big_block<NT>(sm, row_of, sc_row, gs_of, base, base + off.gu_s, base + off.gu_m, qrow, D, xh, xl, G, acc);
     // act = silu(gate) * up; lane (n, g) of tile (rt, t) holds units wu + 16 rt + 4 g + j of pick
     // 16 t + n. A chunk of 8 units lies in lanes g = 2c and 2c + 1: the even lane takes the odd
     // lane's 4 values and writes the chunk (hi, lo in chunk order) and its sum.
-    float wsum[4] = {0.f, 0.f, 0.f, 0.f};  // per pick tile: this lane's chunk sums
+    float wsum[NT];  // per pick tile: this lane's chunk sums
+#pragma unroll
+    for (int t = 0; t < NT; t++) wsum[t] = 0.f;
 #pragma unroll
     for (int rt = 0; rt < 2; rt++)
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
+        for (int t = 0; t < NT; t++) {
             float a[4], o[4];
 #pragma unroll
             for (int j = 0; j < 4; j++) a[j] = silu_f(acc[rt][t][j]) * acc[rt + 2][t][j];
@@ -785,7 +921,7 @@ __global__ void __launch_bounds__(64 * NWB, 2) moe_gate_up_big_kernel(const MoeT
                 split8(v, hi, lo, sum);
                 wsum[t] += sum;
                 const int pr = 16 * t + n;
-                if (pr < np) {
+                if (pr < np && mine) {
                     const size_t p = p0 + pr;
                     const int u = wu + 16 * rt + 4 * g;  // the chunk's first unit
                     *(uint4*)(ah + p * I + u) = hi;
@@ -796,19 +932,74 @@ __global__ void __launch_bounds__(64 * NWB, 2) moe_gate_up_big_kernel(const MoeT
     // group sums: a 64-unit group is waves 2 k and 2 k + 1; per wave, the even lanes g = 0, 2 of
     // pick n hold its chunk sums
 #pragma unroll
-    for (int t = 0; t < 4; t++) {
+    for (int t = 0; t < NT; t++) {
         const float s2 = wsum[t] + __shfl_xor(wsum[t], 32, WAVE);
-        if (g == 0) red[wave][16 * t + n] = s2;
+        if (g == 0) sm.red[wave][16 * t + n] = s2;
     }
     __syncthreads();
     if (tid < (UB / 64) * PBB) {
         const int k = tid / PBB, pr = tid % PBB;
-        if (pr < np) as[(size_t)(p0 + pr) * (I / 64) + (u0 / 64) + k] = red[2 * k][pr] + red[2 * k + 1][pr];
+        if (pr < np && u0 + 64 * k < I) as[(size_t)(p0 + pr) * (I / 64) + (u0 / 64) + k] = sm.red[2 * k][pr] + sm.red[2 * k + 1][pr];
     }
 }
 
-// Down for big tiles: output rows [256 ob, 256 ob + 256) x one tile of <= 64 picks; ypick[src][o] =
+__global__ void __launch_bounds__(64 * NWB, 2) moe_gate_up_big_kernel(const MoeTile* __restrict__ tiles,
+                                                              const int* __restrict__ ntiles,
+                                                              const int* __restrict__ ptok,
+                                                              const uint16_t* __restrict__ xh,
+                                                              const uint16_t* __restrict__ xl,
+                                                              const float* __restrict__ xs, int D, int I,
+                                                              ExpertOffsets off, uint16_t* __restrict__ ah,
+                                                              uint16_t* __restrict__ al, float* __restrict__ as) {
+    __shared__ BigSmem sm;
+    const MoeTile tl = tiles[blockIdx.y];
+    if ((int)blockIdx.y >= *ntiles) return;
+    const int p0 = tl.p0, np = tl.p1 - tl.p0;
+    const unsigned char* base = (const unsigned char*)tl.base;
+    switch ((np + 15) / 16) {
+        case 1: big_gate_up<1>(sm, base, off, p0, np, ptok, xs, xh, xl, D, I, ah, al, as); break;
+        case 2: big_gate_up<2>(sm, base, off, p0, np, ptok, xs, xh, xl, D, I, ah, al, as); break;
+        case 3: big_gate_up<3>(sm, base, off, p0, np, ptok, xs, xh, xl, D, I, ah, al, as); break;
+        default: big_gate_up<4>(sm, base, off, p0, np, ptok, xs, xh, xl, D, I, ah, al, as);
+    }
+}
+
+// Down for big tiles: output rows [OB ob, OB ob + OB) x one tile of <= 64 picks; ypick[src][o] =
 // wts[src] * (dn_o . act), as moe_down_kernel.
+template <int NT>
+__device__ __forceinline__ void big_down(BigSmem& sm, const unsigned char* base, const ExpertOffsets& off, int p0, int np,
+                                         const int* __restrict__ psrc, const float* __restrict__ wts,
+                                         const float* __restrict__ as, const uint16_t* __restrict__ ah, const uint16_t* __restrict__ al, int D, int I,
+                                         float* __restrict__ ypick) {
+    const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, n = lane % 16, g = lane / 16;
+    const int wo = blockIdx.x * OB + 64 * wave;
+    // D is a multiple of 128: the last workgroup's upper waves repeat its last rows, unstored
+    const int qrow[RTB] = {min(wo, D - 16), min(wo + 16, D - 16), min(wo + 32, D - 16), min(wo + 48, D - 16)};
+    f32x4 acc[RTB][4];
+    const int G = I / 64;
+    int src[NT];  // the lane's picks, wanted only at the end
+#pragma unroll
+    for (int t = 0; t < NT; t++) src[t] = psrc[p0 + min(16 * t + n, np - 1)];
+    auto row_of = [&](int pk) { return p0 + min(pk, np - 1); };
+    auto sc_row = [&](int r) { return min((int)blockIdx.x * OB + r / 32 * 32, D - 32) + r % 32; };
+    auto gs_of = [&](int pk, int k) { return as[(size_t)row_of(pk) * G + k]; };
+    big_block<NT>(sm, row_of, sc_row, gs_of, base + off.dn_q, base + off.dn_s, base + off.dn_m, qrow, I, ah, al, G, acc);
+    float w[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t++) w[t] = wts[src[t]];
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        const int pr = 16 * t + n;
+        if (pr >= np) continue;
+#pragma unroll
+        for (int rt = 0; rt < RTB; rt++) {
+            if (wo + 16 * rt >= D) break;
+            const f32x4 v = acc[rt][t] * w[t];
+            *(f32x4*)(ypick + (size_t)src[t] * D + wo + 16 * rt + 4 * g) = v;
+        }
+    }
+}
+
 __global__ void __launch_bounds__(64 * NWB, 2) moe_down_big_kernel(const MoeTile* __restrict__ tiles,
                                                            const int* __restrict__ ntiles, const int* __restrict__ psrc,
                                                            const float* __restrict__ wts,
@@ -817,39 +1008,15 @@ __global__ void __launch_bounds__(64 * NWB, 2) moe_down_big_kernel(const MoeTile
                                                            const float* __restrict__ as, int D, int I,
                                                            ExpertOffsets off, float* __restrict__ ypick) {
     __shared__ BigSmem sm;
-    __shared__ __attribute__((aligned(1024))) unsigned char act0[kActBytes];
-    __shared__ __attribute__((aligned(1024))) unsigned char act1[kActBytes];
-    __shared__ long long xrow8[PBB];
-    const int ob = blockIdx.x, tile = blockIdx.y;
-    const MoeTile tl = tiles[tile];
-    if (tile >= *ntiles) return;
-    const int G = I / 64, o0 = ob * UB;
+    const MoeTile tl = tiles[blockIdx.y];
+    if ((int)blockIdx.y >= *ntiles) return;
     const int p0 = tl.p0, np = tl.p1 - tl.p0;
     const unsigned char* base = (const unsigned char*)tl.base;
-    const int tid = threadIdx.x, wave = tid / WAVE, lane = tid % WAVE, n = lane % 16, g = lane / 16;
-    if (tid < PBB) xrow8[tid] = (long long)(p0 + min(tid, np - 1)) * I;
-    stage_sc_packed(sm.sc, (const uint16_t*)(base + off.dn_s), (const uint16_t*)(base + off.dn_m), o0, UB, G);
-    for (int i = tid; i < PBB * G; i += blockDim.x) {
-        const int pr = i / G, c = i % G;
-        sm.gs[pr * (G + 1) + c] = as[(size_t)(p0 + min(pr, np - 1)) * G + c];
-    }
-    __syncthreads();
-    const int wo = o0 + 32 * wave;
-    const long long qrow[2] = {wo, wo + 16};
-    const int srow[2] = {32 * wave, 32 * wave + 16};
-    f32x4 acc[2][4];
-    big_block<2>(base + off.dn_q, qrow, srow, I, ah, al, xrow8, sm.sc, sm.gs, G, act0, act1, acc);
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-        const int pr = 16 * t + n;
-        if (pr >= np) continue;
-        const int src = psrc[p0 + pr];
-        const float w = wts[src];
-#pragma unroll
-        for (int rt = 0; rt < 2; rt++) {
-            const f32x4 v = acc[rt][t];
-            *(float4*)(ypick + (size_t)src * D + wo + 16 * rt + 4 * g) = float4{w * v[0], w * v[1], w * v[2], w * v[3]};
-        }
+    switch ((np + 15) / 16) {
+        case 1: big_down<1>(sm, base, off, p0, np, psrc, wts, as, ah, al, D, I, ypick); break;
+        case 2: big_down<2>(sm, base, off, p0, np, psrc, wts, as, ah, al, D, I, ypick); break;
+        case 3: big_down<3>(sm, base, off, p0, np, psrc, wts, as, ah, al, D, I, ypick); break;
+        default: big_down<4>(sm, base, off, p0, np, psrc, wts, as, ah, al, D, I, ypick);
     }
 }
 
@@ -916,7 +1083,8 @@ static bool big_tiles_enabled() {
 
 // Workspace plan of aegist_moe_experts.
 struct MoePlan {
-    size_t xh, xl, xs, ah, al, as, yp, eoff, ptok, psrc, tiles1, tiles2, tiles3, meta, total;
+    size_t xh, xl, xs, ah, al, as, yp, cnt, eoff, ptok, psrc, tiles1, tiles2, tiles3, meta, total;
+    int per, nb;           // grouping: picks per block, blocks (at most 64: each reads all the blocks' counts)
     int max1, max2, max3;  // tile-list capacities: <= 16 picks (one per expert), 17..32, 33..64
 };
 static size_t al256(size_t x) { return (x + 255) / 256 * 256; }
@@ -926,7 +1094,9 @@ static MoePlan moe_plan(int T, int K, int D, int I, int E) {
     p.max1 = (int)std::min<size_t>(N, (size_t)E);
     // an expert with c picks has floor(c / PB) + [c % PB > 16] <= c / 17 large blocks
     p.max2 = (int)(N / 17);
-    p.max3 = (int)(N / 16);  // ceil(c / 64) <= c / 16 for every c > 32
+    p.max3 = (int)(N / PBB + std::min<size_t>(N, (size_t)E));  // sum of ceil(c / 64)
+    p.per = (int)std::max<size_t>(1024, (N + 63) / 64);
+    p.nb = (int)((N + p.per - 1) / p.per);
     size_t o = 0;
     auto take = [&](size_t bytes) {
         const size_t at = o;
@@ -940,6 +1110,7 @@ static MoePlan moe_plan(int T, int K, int D, int I, int E) {
     p.al = take(N * I * 2);
     p.as = take(N * (I / 64) * 4);
     p.yp = take(N * D * 4);
+    p.cnt = take((size_t)p.nb * E * 4);
     p.eoff = take((size_t)(E + 1) * 4);
     p.ptok = take(N * 4);
     p.psrc = take(N * 4);
@@ -1033,17 +1204,29 @@ int aegist_moe_experts(const float* h, const unsigned long long* eptr, const int
         moe_combine_kernel<<<dim3(T, (D + 255) / 256), 256, 0, st>>>(x, yp, idx, E, ysh, h, wg, D, K);
         return after_launch("moe_combine");
     }
-    // experts with more than 32 picks take the big-tile kernels where the shapes allow, once the
-    // batch is large enough for such experts to be common (16 picks per expert on average)
-    const bool big = (long long)N >= 16LL * E && D % UB == 0 && I % UB == 0 && D / 64 <= 32 && I / 64 <= 32 &&
-                     big_tiles_enabled();
-    moe_group_kernel<<<1, 1024, 0, st>>>(idx, N, K, E, eptr, eoff, ptok, psrc, tiles1, tiles2, tiles3, big ? 1 : 0,
-                                         meta);
-    int rc = after_launch("moe_group");
-    if (rc) return rc;
+    // the prefill tiles wherever the shapes allow (they address activation rows through 32-bit byte
+    // offsets): against the tiles of <= 32 picks 223 -> 173 us at 80 tokens (640 picks of 256 experts),
+    // 240 -> 177 at 200, 320 -> 199 at 512, 418 -> 243 at 1000
+    const bool big = D % 128 == 0 && I % 128 == 0 && D / 64 <= 32 && I / 64 <= 32 &&
+                     (long long)T * D * 2 < (1LL << 32) && (long long)N * I * 2 < (1LL << 32) && big_tiles_enabled();
+    int* cnt = (int*)(w + p.cnt);
     const long long nq = (long long)T * (D / 8);
-    moe_xprep_kernel<<<(unsigned)((nq + 255) / 256), 256, 0, st>>>(h, T, D, xh, xl, xs);
-    if ((rc = after_launch("moe_xprep"))) return rc;
+    moe_count_kernel<<<p.nb + (unsigned)((nq + 255) / 256), 256, 0, st>>>(idx, N, E, p.per, p.nb, cnt, h, T, D, xh, xl, xs);
+    int rc = after_launch("moe_count");
+    if (rc) return rc;
+    moe_place_kernel<<<p.nb, 1024, 0, st>>>(idx, N, K, E, p.per, p.nb, cnt, eptr, eoff, ptok, psrc, tiles1, tiles2, tiles3,
+                                            big ? 1 : 0, meta);
+    if ((rc = after_launch("moe_place"))) return rc;
+    if (big) {
+        moe_gate_up_big_kernel<<<dim3((I + UB - 1) / UB, p.max3), 64 * NWB, 0, st>>>(tiles3, meta + 3, ptok, xh, xl, xs, D, I, off, ah,
+                                                                   al, as);
+        if ((rc = after_launch("moe_gate_up_big"))) return rc;
+        moe_down_big_kernel<<<dim3((D + OB - 1) / OB, p.max3), 64 * NWB, 0, st>>>(tiles3, meta + 3, psrc, wts, ah, al, as, D,
+                                                                                  I, off, yp);
+        if ((rc = after_launch("moe_down_big"))) return rc;
+        moe_combine_kernel<<<dim3(T, (D + 255) / 256), 256, 0, st>>>(x, yp, idx, E, ysh, h, wg, D, K);
+        return after_launch("moe_combine");
+    }
     // Picks with an out-of-range expert id are dropped: no tile covers them and the combine
     // skips their rows, so nothing has to be cleared.
     const size_t lds_gu = (size_t)(2 * RB + PB) * (D / 64) * 8, lds_dn = (size_t)(RB + PB) * (I / 64) * 8;
@@ -1057,22 +1240,12 @@ int aegist_moe_experts(const float* h, const unsigned long long* eptr, const int
                                                                          ah, al, as);
         if ((rc = after_launch("moe_gate_up"))) return rc;
     }
-    if (big) {
-        moe_gate_up_big_kernel<<<dim3(I / UB, p.max3), 64 * NWB, 0, st>>>(tiles3, meta + 3, ptok, xh, xl, xs, D, I, off, ah,
-                                                                   al, as);
-        if ((rc = after_launch("moe_gate_up_big"))) return rc;
-    }
     moe_down_kernel<1><<<dim3(D / RB, p.max1), 256, lds_dn, st>>>(tiles1, meta, psrc, wts, ah, al, as, D, I, off, yp);
     if ((rc = after_launch("moe_down"))) return rc;
     if (p.max2 > 0) {
         moe_down_kernel<2><<<dim3(D / RB, p.max2), 256, lds_dn, st>>>(tiles2, meta + 2, psrc, wts, ah, al, as, D, I,
                                                                       off, yp);
         if ((rc = after_launch("moe_down"))) return rc;
-    }
-    if (big) {
-        moe_down_big_kernel<<<dim3(D / UB, p.max3), 64 * NWB, 0, st>>>(tiles3, meta + 3, psrc, wts, ah, al, as, D, I, off,
-                                                                yp);
-        if ((rc = after_launch("moe_down_big"))) return rc;
     }
     moe_combine_kernel<<<dim3(T, (D + 255) / 256), 256, 0, st>>>(x, yp, idx, E, ysh, h, wg, D, K);
     return after_launch("moe_combine");

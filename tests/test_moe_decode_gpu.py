@@ -47,3 +47,23 @@ def test_router_rounds_take_the_lowest_of_equals(dev, T, E, K):
     idx, _ = ops.router_topk(h.to(dev), W.to(dev), K)
     ref = torch.sort(-(h.double() @ W.double().t()), dim=-1, stable=True).indices[:, :K]
     assert torch.equal(idx.cpu().long(), ref)
+
+
+@pytest.mark.parametrize("T,D,I,E,K,hot", [(600, 384, 128, 8, 2, 8), (700, 128, 384, 300, 2, 300), (90, 640, 256, 20, 8, 20),
+                                           (130, 2048, 128, 8, 4, 5), (33, 256, 2048, 4, 4, 4), (9000, 256, 128, 64, 8, 64),
+                                           (65, 1024, 512, 16, 16, 16)])
+def test_moe_prefill_tiles_match_oracle(dev, T, D, I, E, K, hot):
+    """The prefill tiles (csrc/moe.hip) at 1 to 64 picks a tile, row lengths whose groups are no multiple of
+    8 (6, 10, 2), outputs and units that end inside a workgroup, and a grouping of more than 64 blocks."""
+    print(f"moe prefill T={T} D={D} I={I} E={E} K={K}", flush=True)
+    g = torch.Generator().manual_seed(T + D + I)
+    rows, h = _experts(E, D, I, T + E), torch.randn(T, D, generator=g)
+    idx = torch.stack([torch.randperm(hot, generator=g)[:K] for _ in range(T)]).int()
+    idx[::7, 0] = -1 if K > 1 else idx[::7, 0]
+    wts = torch.rand(T, K, generator=g)
+    x, hd, rd = torch.zeros(T, D, device=dev), h.to(dev), rows.to(dev)
+    ops.moe_experts(hd, rd, idx.to(dev), wts.to(dev), x, I)
+    torch.cuda.synchronize()
+    err = rel_err(x, R.moe_experts(h, rows, idx.long(), wts, D, I))
+    print(f"  rel err {err:.2e}", flush=True)
+    assert err < 5e-5
