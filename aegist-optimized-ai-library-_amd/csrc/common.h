@@ -91,6 +91,21 @@ __device__ __forceinline__ float pair_sum32(float x) {
     return __uint_as_float(a[0]) + __uint_as_float(a[1]);
 }
 
+// Sum over the wave by DPP adds (row shifts with zero fill, then row broadcasts) instead of LDS
+// permutes, whose six round trips a latency-bound chain would wait for; the total is the last lane's.
+__device__ __forceinline__ float wave_sum_dpp(float v) {
+#define AEG_DPP_ADD(CTRL, ROWS) \
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xF, true))
+    AEG_DPP_ADD(0x111, 0xF);  // row_shr:1
+    AEG_DPP_ADD(0x112, 0xF);
+    AEG_DPP_ADD(0x114, 0xF);
+    AEG_DPP_ADD(0x118, 0xF);
+    AEG_DPP_ADD(0x142, 0xA);  // row_bcast:15 to rows 1 and 3
+    AEG_DPP_ADD(0x143, 0xC);  // row_bcast:31 to rows 2 and 3
+#undef AEG_DPP_ADD
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), WAVE - 1));
+}
+
 // Orders LDS traffic between the lanes of one wave (no workgroup barrier needed for
 // wave-private buffers): stops compiler code motion and waits for outstanding LDS ops.
 __device__ __forceinline__ void wave_sync() {
