@@ -120,13 +120,9 @@ int alloc(Stack* s, void** p, size_t bytes) {
 
 // Y[M, N] (row-major, leading dim ldy) = A[M, K] (bf16 row-major) . W[N, K]^T (bf16 row-major)
 //                                          + beta * Y,   beta in {0, 1}
-// Decode-sized M (<= 64 rows) goes to the weight-streaming kernels (one pass over W), larger M
-// to the tiled MFMA GEMM; shapes the GEMM does not take (K not a multiple of its k step) to the
-// streaming kernels' row-group form.
+// The kernel is picked by size (proj.hip).
 int gemm(Stack*, const uint16_t* A, const uint16_t* W, float* Y, int M, int N, int K, int ldy, float beta,
          hipStream_t stream) {
-    if (M > 64 && gemm_bf16_fits(A, K, W, K, M, N, K))
-        return launch_gemm_bf16(A, K, W, K, Y, ldy, M, N, K, beta != 0.f, stream);
     if (K % 16 == 0)
         return launch_proj(A, AEGIST_BF16, K, W, AEGIST_BF16, nullptr, Y, ldy, M, N, K, beta != 0.f, stream);
     return fail(AEGIST_ERR_SHAPE, "stack: projection K must be a multiple of 16");
@@ -145,27 +141,12 @@ int out_proj(Stack* s, const uint16_t* A, const uint16_t* W, float* x, int M, in
     return gemm(s, A, W, x, M, N, K, N, 1.f, stream);
 }
 
-// The input projections of one layer (up to four weights sharing A): one grouped launch at
-// decode sizes, one GEMM each otherwise.
-int gemm_group(Stack* s, const uint16_t* A, int n, const uint16_t* const* W, float* const* Y, const int* N,
+// The input projections of one layer (up to four weights sharing A), in one launch where the kernel
+// of that size takes several weights.
+int gemm_group(Stack*, const uint16_t* A, int n, const uint16_t* const* W, float* const* Y, const int* N,
                const long long* ldy, int M, int K, hipStream_t stream) {
-    if (M <= 64 && K % 16 == 0)
-        return launch_proj_multi(A, AEGIST_BF16, K, AEGIST_BF16, n, (const void* const*)W, nullptr, Y, ldy, N, M, K, 0,
-                                 stream);
-    // up to three weights in one tiled-GEMM launch (stacked along N): the narrow ones (the
-    // DeltaNet b / a rows, 32 each) then ride in the last column tile of a wide one instead of
-    // taking a whole launch of mostly idle 256-column tiles each
-    bool one = n <= 3;
-    for (int i = 0; i < n && one; i++) one = gemm_bf16_fits(A, K, W[i], K, M, N[i], K) && (i == n - 1 || N[i] % 8 == 0);
-    if (one) {
-        const long long ldw[3] = {K, K, K};
-        return launch_gemm_bf16_multi(A, K, n, W, ldw, Y, ldy, N, M, K, 0, stream);
-    }
-    for (int i = 0; i < n; i++) {
-        int rc = gemm(s, A, W[i], Y[i], M, N[i], K, (int)ldy[i], 0.f, stream);
-        if (rc) return rc;
-    }
-    return 0;
+    if (K % 16) return fail(AEGIST_ERR_SHAPE, "stack: projection K must be a multiple of 16");
+    return launch_proj_multi(A, AEGIST_BF16, K, AEGIST_BF16, n, (const void* const*)W, nullptr, Y, ldy, N, M, K, 0, stream);
 }
 
 #define RC(x)                  \
@@ -189,7 +170,8 @@ int delta_layer(Stack* s, const AegistLayerWeights& w, int sl, float* x, int B, 
     // prefill in whole 256-token tiles: the qkv projection's GEMM applies the short convolution
     // and SiLU in its epilogue (the raw projection never reaches HBM; s->proj holds the tiles'
     // edge rows instead)
-    const bool conv_fused = T > 1 && conv_gemm_enabled() && gemm_conv_fits(s->hb, dm, w.w_qkv, dm, w.conv_w, B, T, C, dm);
+    const bool conv_fits = T > 1 && gemm_conv_fits(s->hb, dm, w.w_qkv, dm, w.conv_w, B, T, C, dm);
+    const bool conv_fused = conv_fits && conv_gemm_enabled();
     if (conv_fused) {
         RC(launch_gemm_bf16_conv(s->hb, dm, w.w_qkv, dm, w.conv_w, conv, s->y, C, s->proj, B, T, C, dm, st));
         const uint16_t* W[3] = {w.w_z, w.w_b, w.w_a};
@@ -205,7 +187,9 @@ int delta_layer(Stack* s, const AegistLayerWeights& w, int sl, float* x, int B, 
         if (rows <= 64) {
             RC(gemm_group(s, s->hb, 4, W, Y, N, ldy, rows, dm, st));
         } else {
-            RC(gemm_group(s, s->hb, 1, W, Y, N, ldy, rows, dm, st));
+            // (with the fusion switched off: the same tiles, so that both ways give the same bits)
+            if (conv_fits) RC(launch_gemm_bf16(s->hb, dm, w.w_qkv, dm, s->proj, C, rows, C, dm, 0, st));
+            else RC(gemm_group(s, s->hb, 1, W, Y, N, ldy, rows, dm, st));
             RC(gemm_group(s, s->hb, 3, W + 1, Y + 1, N + 1, ldy + 1, rows, dm, st));
         }
     }
