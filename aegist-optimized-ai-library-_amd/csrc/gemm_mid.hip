@@ -13,7 +13,7 @@
 // one LDS-only barrier per step. 16-byte slots of a staged row are XOR-swizzled by the row.
 //
 // Measured against the kernels that served these sizes before (same box, us per launch):
-//   int8 W, fp32 X   300 x 8192 x 2048: 117 -> 36   300 x 2048 x 4096: 221 -> 25   1024 x 8192 x 2048: 119 -> 63
+//   int8 W, fp32 X   300 x 8192 x 2048: 117 -> 34   300 x 2048 x 4096: 221 -> 25   1024 x 8192 x 2048: 119 -> 63
 //   bf16 W, bf16 X    64 x 2048 x 4096: 21 -> 9.6    300 x 2048 x 4096: 83 -> 25     300 x 8192 x 2048: 47 -> 33
 // Prefetching four steps instead of two, or accumulating in fewer, larger tiles at small M, gained
 // nothing: a step costs 0.1 to 0.2 us even in the smallest tile (the barrier, the LDS round trip and
@@ -288,19 +288,20 @@ __global__ void __launch_bounds__(64 * NWN * KG) gemm_mid_kernel(const MidArgs g
 }
 
 // One form of the kernel and its cost: us of one 64-k step of a round of workgroups (one per CU), the
-// median over a sweep of M 20 .. 1500 and N x K 512 .. 8192 x 2048 and 2048 x 4096 on one card; the
-// estimate ceil(tiles / 256) x steps x cost picked the fastest form or one within 10% of it at 50 of
-// the 56 swept sizes (at worst 20% slower, between neighbouring tile sizes).
+// median over a sweep of M 20 .. 1500 and N x K 512 .. 8192 x 2048 and 2048 x 4096 on one card (`base`: the
+// part that does not grow with the rounds, for the form without K groups, whose workgroups share a
+// CU); the estimate base + ceil(tiles / 256) x cost picked the fastest form or one within 10% of it
+// at 52 of the 56 swept sizes (at worst 15% slower, between neighbouring tile sizes).
 struct MidForm {
     int rt, mt, nwn, kg;
-    float cost;
+    float cost, base = 0.f;
 };
 // fp32 X: staging and splitting X is the larger part of a step
 constexpr MidForm kFormsF32[] = {{1, 2, 1, 8, 0.156f}, {1, 2, 2, 8, 0.18f}, {2, 2, 2, 8, 0.265f}, {2, 2, 4, 4, 0.375f},
-                                 {2, 4, 4, 2, 0.60f},  {2, 4, 8, 1, 1.10f}, {4, 4, 8, 1, 1.70f}};
+                                 {2, 2, 4, 1, 0.28f, 0.15f}, {2, 4, 4, 2, 0.60f}, {2, 4, 8, 1, 1.10f}, {4, 4, 8, 1, 1.70f}};
 constexpr MidForm kFormsBf16[] = {{1, 2, 1, 8, 0.100f}, {1, 2, 2, 8, 0.157f}, {1, 4, 2, 4, 0.205f}, {1, 4, 4, 2, 0.312f},
                                   {2, 4, 4, 2, 0.548f}, {2, 8, 4, 1, 0.90f},  {2, 8, 8, 1, 1.21f}};
-constexpr int kForms = 7;
+constexpr int kNF32 = 8, kNBf16 = 7, kForms = 8;  // entries of the two tables; codes of the sized forms
 // Up to 16 rows (one 16-row tile of X), after the sized forms; chosen by rows of W and K, see small_form
 constexpr MidForm kFormsSmall[] = {{1, 1, 1, 8, 0.f}, {1, 1, 1, 4, 0.f}, {1, 1, 2, 4, 0.f}, {2, 1, 2, 4, 0.f}};
 constexpr int kSmall = 4;
@@ -346,14 +347,14 @@ int run_mid(int form, const MidArgs& ga, hipStream_t st) {
     constexpr bool f32 = std::is_same<TX, float>::value;
 #define AEG_MID(I)                                                                                              \
     case I: {                                                                                                   \
-        constexpr MidForm f = f32 ? kFormsF32[I] : kFormsBf16[I];                                               \
+        constexpr MidForm f = f32 ? kFormsF32[I] : kFormsBf16[I < kNBf16 ? I : 0];                              \
         return launch_mid<TW, TX, f.rt, f.mt, f.nwn, f.kg, 2>(ga, st);                                          \
     }
 #define AEG_MID_SMALL(I)                                                                                        \
     case kForms + I: return launch_mid<TW, TX, kFormsSmall[I].rt, 1, kFormsSmall[I].nwn, kFormsSmall[I].kg, 2>(ga, st);
     switch (form) {
         AEG_MID_SMALL(0) AEG_MID_SMALL(1) AEG_MID_SMALL(2) AEG_MID_SMALL(3)
-        AEG_MID(0) AEG_MID(1) AEG_MID(2) AEG_MID(3) AEG_MID(4) AEG_MID(5) AEG_MID(6)
+        AEG_MID(0) AEG_MID(1) AEG_MID(2) AEG_MID(3) AEG_MID(4) AEG_MID(5) AEG_MID(6) AEG_MID(7)
     }
 #undef AEG_MID
 #undef AEG_MID_SMALL
@@ -385,9 +386,9 @@ int gemm_mid_form(int x_dtype, int nseg, const int* N, int M, int K, bool tile25
     const MidForm* forms = x_dtype == AEGIST_F32 ? kFormsF32 : kFormsBf16;
     int best = -1;
     float least = tile256 ? ((t256 + 255) / 256) * (x_dtype == AEGIST_F32 ? kTile256F32 : kTile256Bf16) : 3.4e38f;
-    for (int i = 0; i < kForms; i++) {
+    for (int i = 0; i < (x_dtype == AEGIST_F32 ? kNF32 : kNBf16); i++) {
         const long long t = mid_tiles(forms[i], ga);
-        const float est = ((t + 255) / 256) * forms[i].cost;
+        const float est = forms[i].base + ((t + 255) / 256) * forms[i].cost;
         if (est <= least) {
             least = est;
             best = i;
