@@ -1300,6 +1300,12 @@ __device__ __forceinline__ bf16x8 vt_operand_sw(const uint16_t* vt, int ks, int 
     return bf16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
 }
 
+// Depth of the K and V fragment rings of the kernel below. The K ring runs through both halves of a
+// 64-key tile, so the second half's first operands are read under the first half's products instead
+// of after them (B = 4, T = 2000: 234 -> 230 us; B = 1, T = 2000: 83 -> 79.5 us, with the launch
+// that makes the fp16 copy). Deeper rings (4 to 8 for either) only cost registers: 232 to 235 us.
+constexpr int KR = 3, VR = 4;
+
 template <typename Tout>
 __global__ void __launch_bounds__(64 * PW2, 1) attn_prefill_w32f_kernel(const float* __restrict__ q, Strides3 qs,
                                                                         const uint16_t* __restrict__ kf,
@@ -1471,32 +1477,33 @@ __global__ void __launch_bounds__(64 * PW2, 1) attn_prefill_w32f_kernel(const fl
                 const int row = 16 * nb + n;
                 return (const half8*)&Kt[row * HD + sw_slot(4 * ks + g, row, KSW) * 8];
             };
+            // one ring of fragment pairs over both halves' 16 steps, KR - 1 steps ahead
+            half8 kb[KR][2];
+            auto fetch = [&](int s) __attribute__((always_inline)) {
     #pragma unroll
-            for (int h = 0; h < 2; h++) {
-                half8 kb[3][2];
+                for (int i = 0; i < 2; i++) kb[s % KR][i] = *kaddr(2 * (s / 8) + i, s % 8);
+            };
     #pragma unroll
-                for (int i = 0; i < 2; i++) {
-                    kb[0][i] = *kaddr(2 * h + i, 0);
-                    kb[1][i] = *kaddr(2 * h + i, 1);
+            for (int s = 0; s < KR - 1; s++) fetch(s);
     #pragma unroll
-                    for (int qt = 0; qt < 2; qt++) sc[qt][2 * h + i] = f32x4{0.f, 0.f, 0.f, 0.f};
-                }
-    #pragma unroll
-                for (int ks = 0; ks < 8; ks++) {
+            for (int s = 0; s < 16; s++) {
+                const int h = s / 8, ks = s % 8;
+                if (ks == 0) {
     #pragma unroll
                     for (int i = 0; i < 2; i++)
     #pragma unroll
-                        for (int qt = 0; qt < 2; qt++)
-                            sc[qt][2 * h + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kb[ks % 3][i], qf[qt][ks],
-                                                                                     sc[qt][2 * h + i], 0, 0, 0);
-                    if (ks + 2 < 8) {
-    #pragma unroll
-                        for (int i = 0; i < 2; i++) kb[(ks + 2) % 3][i] = *kaddr(2 * h + i, ks + 2);
-                    }
-                    if (h == 1 && ks < 4) exp_piece(ks >> 1, ks & 1);
-                    __builtin_amdgcn_sched_barrier(0);
+                        for (int qt = 0; qt < 2; qt++) sc[qt][2 * h + i] = f32x4{0.f, 0.f, 0.f, 0.f};
                 }
-                if (h == 0) {
+                if (s + KR - 1 < 16) fetch(s + KR - 1);
+    #pragma unroll
+                for (int i = 0; i < 2; i++)
+    #pragma unroll
+                    for (int qt = 0; qt < 2; qt++)
+                        sc[qt][2 * h + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kb[s % KR][i], qf[qt][ks],
+                                                                                 sc[qt][2 * h + i], 0, 0, 0);
+                if (h == 1 && ks < 4) exp_piece(ks >> 1, ks & 1);
+                __builtin_amdgcn_sched_barrier(0);
+                if (s == 7) {
                     mask(key0, 0, masked);
                     begin_tile();
                 }
@@ -1522,23 +1529,23 @@ __global__ void __launch_bounds__(64 * PW2, 1) attn_prefill_w32f_kernel(const fl
         __syncthreads();  // K0 free for K(2)
 
         auto pv = [&](const uint16_t* Vt, auto side) {
-            bf16x8 vb[4][2];
+            bf16x8 vb[VR][2];
     #pragma unroll
-            for (int d = 0; d < 3; d++) {
+            for (int d = 0; d < VR - 1; d++) {
                 vb[d][0] = vt_operand_sw(Vt, 0, d, lane);
                 vb[d][1] = vt_operand_sw(Vt, 1, d, lane);
             }
     #pragma unroll
             for (int db = 0; db < 16; db++) {
-                if (db + 3 < 16) {
-                    vb[(db + 3) & 3][0] = vt_operand_sw(Vt, 0, db + 3, lane);
-                    vb[(db + 3) & 3][1] = vt_operand_sw(Vt, 1, db + 3, lane);
+                if (db + VR - 1 < 16) {
+                    vb[(db + VR - 1) % VR][0] = vt_operand_sw(Vt, 0, db + VR - 1, lane);
+                    vb[(db + VR - 1) % VR][1] = vt_operand_sw(Vt, 1, db + VR - 1, lane);
                 }
     #pragma unroll
                 for (int ks = 0; ks < 2; ks++)
     #pragma unroll
                     for (int qt = 0; qt < 2; qt++)
-                        oacc[qt][db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, vb[db & 3][ks]),
+                        oacc[qt][db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, vb[db % VR][ks]),
                                                                               pcur[qt][ks], oacc[qt][db], 0, 0, 0);
                 side(db);
                 __builtin_amdgcn_sched_barrier(0);
