@@ -17,6 +17,9 @@
 
 namespace aegist {
 int launch_znorm_bf16(const float* x, const uint16_t* w, uint16_t* out, int rows, int D, float eps, hipStream_t st);
+bool gemv_norm_fits(const float* x, const uint16_t* nw, int M, int K);
+int launch_gemv_norm(const float* x, const uint16_t* nw, float eps, int nseg, const uint16_t* const* W, float* const* Y,
+                     const long long* ldy, const int* N, int M, int K, hipStream_t st);
 int launch_znorm_bf16_acc(float* x, const float* part, int nks, const uint16_t* w, uint16_t* out, int rows, int D,
                           float eps, hipStream_t st);
 int launch_proj_splitk(const uint16_t* X, long long ldx, const uint16_t* W, float* part, int nks, int M, int N, int K,
@@ -132,8 +135,11 @@ int gemm(Stack*, const uint16_t* A, const uint16_t* W, float* Y, int M, int N, i
 // partial sums the next layer's ZNorm (or the end of the forward) adds into x in a fixed order:
 // the d_model = 2048 rows of W alone give only 64 workgroups, a quarter of the GPU.
 constexpr int kOutSplits = 4;
-int out_proj(Stack* s, const uint16_t* A, const uint16_t* W, float* x, int M, int N, int K, hipStream_t stream) {
-    if (M <= 16 && K % 256 == 0 && K / 256 >= kOutSplits && N % 1024 == 0 && N <= 8192) {
+// Rows that are normed inside the input projections (`direct`, one or two) add into x instead: there
+// each row of W is one wave's, and the next launch reads x alone.
+int out_proj(Stack* s, bool direct, const uint16_t* A, const uint16_t* W, float* x, int M, int N, int K,
+             hipStream_t stream) {
+    if (!direct && M <= 16 && K % 256 == 0 && K / 256 >= kOutSplits && N % 1024 == 0 && N <= 8192) {
         int rc = launch_proj_splitk(A, K, W, s->part, kOutSplits, M, N, K, stream);
         if (!rc) s->pend = kOutSplits;
         return rc;
@@ -142,11 +148,14 @@ int out_proj(Stack* s, const uint16_t* A, const uint16_t* W, float* x, int M, in
 }
 
 // The input projections of one layer (up to four weights sharing A), in one launch where the kernel
-// of that size takes several weights.
-int gemm_group(Stack*, const uint16_t* A, int n, const uint16_t* const* W, float* const* Y, const int* N,
-               const long long* ldy, int M, int K, hipStream_t stream) {
+// of that size takes several weights. nx: the residual, whose norm runs inside the projections; null:
+// the normed rows are in s->hb.
+int gemm_group(Stack* s, const float* nx, const uint16_t* norm, int n, const uint16_t* const* W, float* const* Y,
+               const int* N, const long long* ldy, int M, int K, hipStream_t stream) {
     if (K % 16) return fail(AEGIST_ERR_SHAPE, "stack: projection K must be a multiple of 16");
-    return launch_proj_multi(A, AEGIST_BF16, K, AEGIST_BF16, n, (const void* const*)W, nullptr, Y, ldy, N, M, K, 0, stream);
+    if (nx) return launch_gemv_norm(nx, norm, s->cfg.eps, n, W, Y, ldy, N, M, K, stream);
+    return launch_proj_multi(s->hb, AEGIST_BF16, K, AEGIST_BF16, n, (const void* const*)W, nullptr, Y, ldy, N, M, K, 0,
+                             stream);
 }
 
 #define RC(x)                  \
@@ -161,7 +170,8 @@ bool conv_gemm_enabled() {
     return !(e && e[0] == '0');
 }
 
-int delta_layer(Stack* s, const AegistLayerWeights& w, int sl, float* x, int B, int T, hipStream_t st) {
+int delta_layer(Stack* s, const AegistLayerWeights& w, int sl, float* x, const float* nx, int B, int T,
+                hipStream_t st) {
     const AegistStackConfig& c = s->cfg;
     const int rows = B * T, C = s->C(), HV = c.hv, HK = c.hk, dm = c.d_model;
     const size_t mb = (size_t)c.max_batch;
@@ -178,19 +188,19 @@ int delta_layer(Stack* s, const AegistLayerWeights& w, int sl, float* x, int B, 
         float* Y[3] = {s->z, s->ba, s->ba + HV};
         const int N[3] = {HV * D, HV, HV};
         const long long ldy[3] = {HV * D, 2 * HV, 2 * HV};
-        RC(gemm_group(s, s->hb, 3, W, Y, N, ldy, rows, dm, st));
+        RC(gemm_group(s, nx, w.norm1, 3, W, Y, N, ldy, rows, dm, st));
     } else {
         const uint16_t* W[4] = {w.w_qkv, w.w_z, w.w_b, w.w_a};
         float* Y[4] = {s->proj, s->z, s->ba, s->ba + HV};
         const int N[4] = {C, HV * D, HV, HV};
         const long long ldy[4] = {C, HV * D, 2 * HV, 2 * HV};
         if (rows <= 64) {
-            RC(gemm_group(s, s->hb, 4, W, Y, N, ldy, rows, dm, st));
+            RC(gemm_group(s, nx, w.norm1, 4, W, Y, N, ldy, rows, dm, st));
         } else {
             // (with the fusion switched off: the same tiles, so that both ways give the same bits)
             if (conv_fits) RC(launch_gemm_bf16(s->hb, dm, w.w_qkv, dm, s->proj, C, rows, C, dm, 0, st));
-            else RC(gemm_group(s, s->hb, 1, W, Y, N, ldy, rows, dm, st));
-            RC(gemm_group(s, s->hb, 3, W + 1, Y + 1, N + 1, ldy + 1, rows, dm, st));
+            else RC(gemm_group(s, nx, w.norm1, 1, W, Y, N, ldy, rows, dm, st));
+            RC(gemm_group(s, nx, w.norm1, 3, W + 1, Y + 1, N + 1, ldy + 1, rows, dm, st));
         }
     }
     const float qscale = 1.f / sqrtf((float)D);
@@ -199,7 +209,7 @@ int delta_layer(Stack* s, const AegistLayerWeights& w, int sl, float* x, int B, 
         // one launch (hybrid.py:401-419)
         RC(launch_delta_decode_stack(s->proj, w.conv_w, conv, s->ba, w.a_log, w.dt_bias, s->z, w.gnorm_w, c.eps, rec,
                                      s->ob, B, HK, HV, qscale, 1e-6f, st));
-        return out_proj(s, s->ob, w.w_out, x, rows, dm, HV * D, st);
+        return out_proj(s, nx != nullptr, s->ob, w.w_out, x, rows, dm, HV * D, st);
     }
     RC(launch_gates_from_proj(s->ba, w.a_log, w.dt_bias, s->g, s->beta, rows, HV, st));
     {
@@ -217,10 +227,11 @@ int delta_layer(Stack* s, const AegistLayerWeights& w, int sl, float* x, int B, 
                                 qscale, 1e-6f, s->ws, s->ws_bytes, st));
     }
     RC(launch_gated_norm_bf16(s->o, s->z, w.gnorm_w, s->ob, rows * HV, D, c.eps, st));
-    return out_proj(s, s->ob, w.w_out, x, rows, dm, HV * D, st);
+    return out_proj(s, nx != nullptr, s->ob, w.w_out, x, rows, dm, HV * D, st);
 }
 
-int attn_layer(Stack* s, const AegistLayerWeights& w, int sl, float* x, int B, int T, hipStream_t st) {
+int attn_layer(Stack* s, const AegistLayerWeights& w, int sl, float* x, const float* nx, int B, int T,
+               hipStream_t st) {
     const AegistStackConfig& c = s->cfg;
     const int rows = B * T, H = c.n_heads, KV = c.n_kv, HD = c.head_dim, dm = c.d_model;
     const size_t mb = (size_t)c.max_batch, cap = (size_t)c.max_context;
@@ -233,13 +244,13 @@ int attn_layer(Stack* s, const AegistLayerWeights& w, int sl, float* x, int B, i
         float* Y[3] = {s->proj, kp, vp};
         const int N[3] = {2 * H * HD, KV * HD, KV * HD};
         const long long ldy[3] = {2 * H * HD, KV * HD, KV * HD};
-        RC(gemm_group(s, s->hb, 3, W, Y, N, ldy, rows, dm, st));
+        RC(gemm_group(s, nx, w.norm1, 3, W, Y, N, ldy, rows, dm, st));
     }
     if (T == 1 && c.rotary_dim == 64) {
         // decode: ZNorm, RoPE and the cache append inside the split launch
         RC(stack_attn_decode_fused(s->proj, kp, vp, w.q_norm, w.k_norm, kc, vc, s->ob, B, H, KV, s->length, (int)cap,
                                    c.eps, c.rope_theta, s->ws, s->ws_bytes, st));
-        return out_proj(s, s->ob, w.w_o, x, rows, dm, H * HD, st);
+        return out_proj(s, nx != nullptr, s->ob, w.w_o, x, rows, dm, H * HD, st);
     }
     RC(launch_attn_prep(s->proj, kp, vp, AEGIST_F32, w.q_norm, w.k_norm, s->y, kc, vc, B, T, H, KV, HD, c.rotary_dim,
                         s->length, (int)cap, c.eps, c.rope_theta, st));
@@ -256,7 +267,7 @@ int attn_layer(Stack* s, const AegistLayerWeights& w, int sl, float* x, int B, i
                               s->ws_bytes, st, s->ob, &wrote_bf16));
         if (!wrote_bf16) RC(launch_cast_bf16(s->o, s->ob, (size_t)rows * H * HD, st));
     }
-    return out_proj(s, s->ob, w.w_o, x, rows, dm, H * HD, st);
+    return out_proj(s, nx != nullptr, s->ob, w.w_o, x, rows, dm, H * HD, st);
 }
 
 }  // namespace
@@ -493,15 +504,17 @@ int aegist_stack_forward(void* handle, float* x, int B, int T, void* stream) {
     s->pend = 0;
     for (int l = 0; l < c.n_layers; l++) {
         const AegistLayerWeights& w = s->w[l];
+        // one or two rows: the norm runs inside the input projections (gemv.hip)
+        const float* nx = !s->pend && gemv_norm_fits(x, w.norm1, rows, c.d_model) ? x : nullptr;
         if (s->pend) {
             const int p = s->pend;
             s->pend = 0;
             RC(launch_znorm_bf16_acc(x, s->part, p, w.norm1, s->hb, rows, c.d_model, c.eps, st));
-        } else {
+        } else if (!nx) {
             RC(launch_znorm_bf16(x, w.norm1, s->hb, rows, c.d_model, c.eps, st));
         }
-        if (c.layer_is_attn[l]) RC(attn_layer(s, w, s->slot[l], x, B, T, st));
-        else RC(delta_layer(s, w, s->slot[l], x, B, T, st));
+        if (c.layer_is_attn[l]) RC(attn_layer(s, w, s->slot[l], x, nx, B, T, st));
+        else RC(delta_layer(s, w, s->slot[l], x, nx, B, T, st));
     }
     if (s->pend) {
         const int p = s->pend;

@@ -59,6 +59,7 @@ def test_mid_batch_segments_and_strides(dev, w8, xf):
 
 @pytest.mark.parametrize("w8,xf", [(True, True), (False, False), (False, True), (True, False)])
 @pytest.mark.parametrize("M,N,K", [(1, 1, 16), (1, 5, 48), (2, 515, 1040), (1, 1030, 2064), (2, 2049, 512), (1, 4099, 528),
+                                   (1, 7, 1552), (2, 1029, 3088), (1, 4097, 4112), (2, 3, 8192),
                                    (2, 8200, 32), (1, 8192, 2048), (3, 33, 16), (5, 100, 1040), (16, 2048, 2064),
                                    (7, 6150, 64), (16, 8192, 512), (11, 9000, 256), (9, 16500, 80)])
 def test_small_batch_matches_exact(dev, M, N, K, w8, xf):
