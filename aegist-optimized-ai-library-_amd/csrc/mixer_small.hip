@@ -23,10 +23,54 @@ __global__ void __launch_bounds__(256) znorm_kernel(const float* __restrict__ x,
     for (int i = threadIdx.x; i < D; i += 256) orow[i] = (xr[i] * inv) * (1.f + bf2f(w[i]));
 }
 
+// The same for rows of up to 8192 in 16-byte pieces (D % 4 == 0, aligned rows): a thread's NV pieces and
+// their weights are requested together and stay in registers, one round trip and one barrier instead
+// of a load per value and pass. Latency-bound; us for 300 rows of 2048 6.1 -> 4.4, one row 4.0 -> 2.2.
+template <int NV>
+__global__ void __launch_bounds__(256) znorm_vec_kernel(const float* __restrict__ x, const uint16_t* __restrict__ w,
+                                                        float* __restrict__ out, int D, float eps) {
+    __shared__ float red[4];
+    const float* xr = x + (size_t)blockIdx.x * D;
+    float4 v[NV];
+    uint2 wp[NV];
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const int k = 4 * ((int)threadIdx.x + 256 * i), kk = k < D ? k : 0;
+        v[i] = *(const float4*)(xr + kk);
+        wp[i] = *(const uint2*)(w + kk);
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const float q = v[i].x * v[i].x + v[i].y * v[i].y + v[i].z * v[i].z + v[i].w * v[i].w;
+        ss += 4 * ((int)threadIdx.x + 256 * i) < D ? q : 0.f;
+    }
+    ss = wave_sum_dpp(ss);
+    if (threadIdx.x % WAVE == 0) red[threadIdx.x / WAVE] = ss;
+    __syncthreads();
+    const float inv = rsqrtf((red[0] + red[1] + red[2] + red[3]) / (float)D + eps);
+    float* orow = out + (size_t)blockIdx.x * D;
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const int k = 4 * ((int)threadIdx.x + 256 * i);
+        if (k >= D) break;
+        *(float4*)(orow + k) =
+            float4{(v[i].x * inv) * (1.f + bf_lo(wp[i].x)), (v[i].y * inv) * (1.f + bf_hi(wp[i].x)),
+                   (v[i].z * inv) * (1.f + bf_lo(wp[i].y)), (v[i].w * inv) * (1.f + bf_hi(wp[i].y))};
+    }
+}
+
 extern "C" int aegist_znorm(const float* x, const uint16_t* w, float* out, int rows, int D, float eps, void* stream) {
     AEG_REQUIRE(rows >= 0 && D > 0, "znorm: rows >= 0 and D > 0 required");
     if (rows == 0) return 0;
-    znorm_kernel<<<rows, 256, 0, AEG_STREAM(stream)>>>(x, w, out, D, eps);
+    hipStream_t st = AEG_STREAM(stream);
+    const bool vec = D % 4 == 0 && D <= 8192 && (uintptr_t)x % 16 == 0 && (uintptr_t)out % 16 == 0 &&
+                     (uintptr_t)w % 8 == 0;
+    if (!vec) znorm_kernel<<<rows, 256, 0, st>>>(x, w, out, D, eps);
+    else if (D <= 1024) znorm_vec_kernel<1><<<rows, 256, 0, st>>>(x, w, out, D, eps);
+    else if (D <= 2048) znorm_vec_kernel<2><<<rows, 256, 0, st>>>(x, w, out, D, eps);
+    else if (D <= 4096) znorm_vec_kernel<4><<<rows, 256, 0, st>>>(x, w, out, D, eps);
+    else znorm_vec_kernel<8><<<rows, 256, 0, st>>>(x, w, out, D, eps);
     return after_launch("znorm");
 }
 
@@ -421,10 +465,43 @@ __global__ void __launch_bounds__(256) l2norm_heads_kernel(float* __restrict__ y
     for (int i = lane; i < dk; i += WAVE) p[i] = (p[i] * r) * s;
 }
 
+// Sum over each half of the wave (32 lanes); every lane gets its half's.
+__device__ __forceinline__ float half_sum_dpp(float v) {
+#define AEG_DPP_ADD(CTRL, ROWS) \
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xF, true))
+    AEG_DPP_ADD(0x111, 0xF);  // row_shr:1
+    AEG_DPP_ADD(0x112, 0xF);
+    AEG_DPP_ADD(0x114, 0xF);
+    AEG_DPP_ADD(0x118, 0xF);
+    AEG_DPP_ADD(0x142, 0xA);  // row_bcast:15 to rows 1 and 3
+#undef AEG_DPP_ADD
+    const float lo = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 31));
+    const float hi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+    return threadIdx.x % WAVE < 32 ? lo : hi;
+}
+
+// The same for heads of up to 128 in 16-byte pieces: half a wave per (row, head), one load per lane.
+// Latency-bound; 300 rows of 32 heads 5.1 -> 4.1 us.
+__global__ void __launch_bounds__(256) l2norm_heads_vec_kernel(float* __restrict__ y, int items, int C, int nq, int dk,
+                                                               float qscale, float eps) {
+    const int item = blockIdx.x * 8 + threadIdx.x / 32, k = 4 * (threadIdx.x % 32);
+    const bool ok = item < items && k < dk;
+    const int it = item < items ? item : items - 1, t = it / (2 * nq), hh = it % (2 * nq);
+    float* p = y + (size_t)t * C + (size_t)hh * dk + (k < dk ? k : 0);
+    const float4 a = *(const float4*)p;
+    const float ss = half_sum_dpp(ok ? a.x * a.x + a.y * a.y + a.z * a.z + a.w * a.w : 0.f);
+    const float r = rsqrtf(ss + eps), s = hh < nq ? qscale : 1.f;
+    if (ok) *(float4*)p = float4{(a.x * r) * s, (a.y * r) * s, (a.z * r) * s, (a.w * r) * s};
+}
+
 extern "C" int aegist_l2norm_heads(float* y, int T, int C, int nq, int dk, float qscale, float eps, void* stream) {
     AEG_REQUIRE(T >= 0 && nq > 0 && dk > 0 && 2 * nq * dk <= C, "l2norm_heads: bad shape");
     if (T == 0) return 0;
     int items = T * 2 * nq;
+    if (dk % 4 == 0 && dk <= 128 && C % 4 == 0 && (uintptr_t)y % 16 == 0) {
+        l2norm_heads_vec_kernel<<<(items + 7) / 8, 256, 0, AEG_STREAM(stream)>>>(y, items, C, nq, dk, qscale, eps);
+        return after_launch("l2norm_heads");
+    }
     l2norm_heads_kernel<<<(items + 3) / 4, 256, 0, AEG_STREAM(stream)>>>(y, T, C, nq, dk, qscale, eps);
     return after_launch("l2norm_heads");
 }
@@ -449,11 +526,35 @@ __global__ void __launch_bounds__(256) gated_norm_kernel(const float* __restrict
     }
 }
 
+// The same for heads of up to 128 in 16-byte pieces: half a wave per (row, head), o, z and w requested
+// together. 300 rows of 32 heads 6.0 -> 5.5 us.
+__global__ void __launch_bounds__(256) gated_norm_vec_kernel(const float* __restrict__ o, const float* __restrict__ z,
+                                                             const uint16_t* __restrict__ w, float* __restrict__ out,
+                                                             int rows, int DV, float eps) {
+    const int item = blockIdx.x * 8 + threadIdx.x / 32, k = 4 * (threadIdx.x % 32);
+    const bool ok = item < rows && k < DV;
+    const int kk = k < DV ? k : 0;
+    const size_t at = (size_t)(item < rows ? item : rows - 1) * DV + kk;
+    const float4 a = *(const float4*)(o + at), zz = *(const float4*)(z + at);
+    const uint2 wp = *(const uint2*)(w + kk);
+    const float ss = half_sum_dpp(ok ? a.x * a.x + a.y * a.y + a.z * a.z + a.w * a.w : 0.f);
+    const float r = rsqrtf(ss / (float)DV + eps);
+    auto gate = [](float v) { return v / (1.f + expf(-v)); };
+    if (ok)
+        *(float4*)(out + at) = float4{bf_lo(wp.x) * (a.x * r) * gate(zz.x), bf_hi(wp.x) * (a.y * r) * gate(zz.y),
+                                      bf_lo(wp.y) * (a.z * r) * gate(zz.z), bf_hi(wp.y) * (a.w * r) * gate(zz.w)};
+}
+
 extern "C" int aegist_gated_norm(const float* o, const float* z, const uint16_t* w, float* out, int T, int HV, int DV,
                                  float eps, void* stream) {
     AEG_REQUIRE(T >= 0 && HV > 0 && DV > 0, "gated_norm: bad shape");
     int rows = T * HV;
     if (rows == 0) return 0;
+    if (DV % 4 == 0 && DV <= 128 && (uintptr_t)o % 16 == 0 && (uintptr_t)z % 16 == 0 && (uintptr_t)out % 16 == 0 &&
+        (uintptr_t)w % 8 == 0) {
+        gated_norm_vec_kernel<<<(rows + 7) / 8, 256, 0, AEG_STREAM(stream)>>>(o, z, w, out, rows, DV, eps);
+        return after_launch("gated_norm");
+    }
     gated_norm_kernel<<<(rows + 3) / 4, 256, 0, AEG_STREAM(stream)>>>(o, z, w, out, rows, DV, eps);
     return after_launch("gated_norm");
 }

@@ -1,6 +1,7 @@
-"""The gates' and the embedding's wide-load kernels (csrc/mixer_small.hip) at the edges of their forms:
+"""The wide-load kernels of the small ops (csrc/mixer_small.hip) at the edges of their forms: gates with
 one token a wave below 64 tokens, four from there on, heads in groups of four, rows in pieces of 512
-values; widths that are no multiple of eight take the narrow kernels."""
+values; norms whose row or head ends inside a thread's pieces; widths that are no multiple of eight or
+four take the narrow kernels."""
 import pytest
 import torch
 
@@ -39,3 +40,39 @@ def test_embed_matches_rows(dev, n, D):
     ids[0] = 49
     out = ops.embed(table.to(dev), ids.to(dev)).cpu()
     assert torch.equal(out, table[ids.long()].float())
+
+
+# norms of n values: fp32 squares, sums and one rsqrt, a sum of at most 34 levels (8 x 4 values a thread, the
+# wave's 6 and the block's 3, or 2 a lane and 6): (34 + 8) 2^-24 of the result, 2^-18 with room for the last
+# products' and the sigmoid's roundings
+REL = 2 ** -18
+
+
+@pytest.mark.parametrize("rows", [1, 5])
+@pytest.mark.parametrize("D", [4, 7, 1020, 1024, 1028, 2048, 4100, 8192, 8196])
+def test_znorm_matches_exact(dev, rows, D):
+    g_ = torch.Generator().manual_seed(rows + D)
+    x, w = torch.randn(rows, D, generator=g_), (torch.randn(D, generator=g_) * 0.1).bfloat16()
+    ref = x.double() * (x.double().square().mean(-1, keepdim=True) + 1e-6).rsqrt() * (1 + w.double())
+    got = ops.engine_znorm(x.to(dev), w.to(dev)).cpu().double()
+    assert ((got - ref).abs() <= REL * ref.abs()).all()
+
+
+@pytest.mark.parametrize("T", [1, 3, 9])
+@pytest.mark.parametrize("nq,dk", [(1, 4), (3, 60), (16, 128), (2, 30), (1, 132)])
+def test_head_norms_match_exact(dev, T, nq, dk):
+    g_ = torch.Generator().manual_seed(T + nq + dk)
+    y = torch.randn(T, 3 * nq * dk, generator=g_)
+    ref = y.double().clone()
+    hd = ref[:, :2 * nq * dk].view(T, 2 * nq, dk)
+    hd *= (hd.square().sum(-1, keepdim=True) + 1e-6).rsqrt()
+    hd[:, :nq] *= dk ** -0.5
+    yd = y.to(dev)
+    ops.engine_l2norm_heads(yd, nq, dk, dk ** -0.5)
+    assert ((yd.cpu().double() - ref).abs() <= REL * ref.abs()).all()
+    o, z = (torch.randn(T, nq, dk, generator=g_) for _ in range(2))
+    w = torch.randn(dk, generator=g_).bfloat16()
+    od, zd = o.double(), z.double()
+    ref = w.double() * od * (od.square().mean(-1, keepdim=True) + 1e-6).rsqrt() * torch.nn.functional.silu(zd)
+    got = ops.engine_gated_norm(o.to(dev), z.to(dev), w.to(dev)).cpu().double()
+    assert ((got - ref).abs() <= REL * ref.abs()).all()
