@@ -502,8 +502,12 @@ def moe_forward(h, x, router_w, experts, I: int, K: int, shared=None, shared_gat
     ysh = None
     if shared is not None:
         (wgt, sg), (wup, su), (wdn, sd) = shared
-        if wgt.dtype == wup.dtype and (sg is None) == (su is None):  # one launch for both
-            g, u = linear_multi(h, [wgt, wup], None if sg is None else [sg, su])
+        # one launch for both; operands that linear() refuses go there to be refused
+        scaled = sg is not None and su is not None and all(
+            sc.dtype == torch.bfloat16 and sc.numel() == w.shape[0] and sc.is_contiguous()
+            for sc, w in ((sg, wgt), (su, wup)))
+        if wgt.dtype == wup.dtype and (scaled or (sg is None and su is None)):
+            g, u = linear_multi(h, [wgt, wup], [sg, su] if scaled else None)
         else:
             g, u = linear(h, wgt, sg), linear(h, wup, su)
         ysh = linear(silu_mul(g, u), wdn, sd)

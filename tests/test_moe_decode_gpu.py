@@ -67,3 +67,18 @@ def test_moe_prefill_tiles_match_oracle(dev, T, D, I, E, K, hot):
     err = rel_err(x, R.moe_experts(h, rows, idx.long(), wts, D, I))
     print(f"  rel err {err:.2e}", flush=True)
     assert err < 5e-5
+
+
+@pytest.mark.parametrize("bad", ["dtype", "size", "stride"])
+def test_moe_forward_refuses_bad_shared_scales(dev, bad):
+    """The shared expert's gate and up projections go in one launch, under the checks of each alone."""
+    D, I = 512, 512
+    g = torch.Generator().manual_seed(2)
+    w = torch.randint(-127, 128, (I, D), generator=g, dtype=torch.int8).to(dev)
+    good = torch.ones(I, dtype=torch.bfloat16, device=dev)
+    sc = {"dtype": good.float(), "size": good.repeat(2), "stride": good.repeat(2)[::2]}[bad]
+    h, x = torch.randn(2, D, generator=g).to(dev), torch.zeros(2, D, device=dev)
+    router = torch.randn(8, D, generator=g).bfloat16().to(dev)
+    with pytest.raises(ops.AegistError):
+        ops.moe_forward(h, x, router, _experts(8, D, I, 3).to(dev), I, 2, shared=((w, good), (w, sc), (w, good)),
+                        shared_gate=torch.zeros(D, dtype=torch.bfloat16, device=dev))
