@@ -127,7 +127,8 @@ __global__ void __launch_bounds__(NV ? WAVE * GN_WAVES : 256) gemv_kernel(const 
         }
         __builtin_amdgcn_sched_barrier(0);
     }
-    // this wave's pieces: every KS-th from k0; pieces past a row's end repeat its first values against zeros
+    // this wave's pieces: every KS-th from k0; pieces past a row's end repeat its first values, taken as zeros
+    const bool ragged = K % (KS * PIECE) != 0;
     const int np = ((K + PIECE - 1) / PIECE + KS - 1) / KS, k0 = (wave % KS) * PIECE + V * lane;
     auto off = [&](int p) { return p * (KS * PIECE) + k0 < K ? p * (KS * PIECE) + k0 : 0; };
     const TW* wrow[R];
@@ -204,7 +205,9 @@ __global__ void __launch_bounds__(NV ? WAVE * GN_WAVES : 256) gemv_kernel(const 
 #pragma unroll
             for (int r = 0; r < R; r++) {
                 float f[V];
-                GvW<TW>::unpack(q[d][r], f);
+                u4v w = q[d][r];
+                if (ragged) w = in ? w : u4v{0, 0, 0, 0};  // (0 x Inf of the repeated values is no 0)
+                GvW<TW>::unpack(w, f);
 #pragma unroll
                 for (int m = 0; m < MX; m++)
 #pragma unroll

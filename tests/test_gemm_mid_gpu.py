@@ -83,3 +83,14 @@ def test_small_batch_segments_and_strides(dev, M, w8, xf):
     for (_, w, s), o in zip(ws, outs):
         _check(o, None, x, w, s, K)
         assert (o.as_strided((M, 3), (o.stride(0), 1), o.shape[1]) == 7).all()
+
+
+@pytest.mark.parametrize("M", [1, 2])
+@pytest.mark.parametrize("K", [48, 1552, 2064])
+def test_one_infinite_weight_is_one_infinite_output(dev, M, K):
+    """The loads past a row's end repeat its first values, which must not turn Inf into NaN."""
+    x, w, _ = _operands(M, 9, K, False, True, K, dev)
+    w[3, 0] = float("inf")
+    y = ops.linear(x, w)
+    assert torch.isinf(y[:, 3]).all() and torch.equal(y[:, 3] > 0, x[:, 0] > 0)
+    assert torch.isfinite(y[:, :3]).all() and torch.isfinite(y[:, 4:]).all()
