@@ -382,9 +382,9 @@ def linear_multi(x, weights, scales=None, outs=None):
             raise AegistError("shape", -1, "weight shape does not match x")
     if outs is None:
         outs = [torch.empty(M, w.shape[0], dtype=torch.float32, device=x.device) for w in weights]
-    Wa = (C.c_void_p * n)(*[w.data_ptr() for w in weights])
-    Sa = None if scales is None else (C.c_void_p * n)(*[None if sc is None else sc.data_ptr() for sc in scales])
-    Ya = (C.c_void_p * n)(*[o.data_ptr() for o in outs])
+    Wa = (C.c_void_p * n)(*[_p(w) for w in weights])
+    Sa = None if scales is None else (C.c_void_p * n)(*[_p(sc) for sc in scales])
+    Ya = (C.c_void_p * n)(*[_p(o) for o in outs])
     La = (C.c_longlong * n)(*[o.stride(0) for o in outs])
     Na = (C.c_int * n)(*[w.shape[0] for w in weights])
     call("aegist_linear_multi", _p(x2), _dt(x2), x2.stride(0), wdt, n, C.cast(Wa, C.c_void_p),
