@@ -24,6 +24,7 @@
 // (c3,c7) with one and-or each, so the activations are stored in the same order within every
 // 8-value chunk: x'[8q + 2j] = x[8q + j], x'[8q + 2j + 1] = x[8q + j + 4].
 #include "common.h"
+#include "moe_tiles.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -240,7 +241,8 @@ __global__ void __launch_bounds__(1024) moe_place_kernel(const int* __restrict__
         if (tid < E) {
             eoff[tid] = off;
             const unsigned long long base = c > 0 ? eptr[tid] : 0ull;
-            for (int j = 0; j < n3; j++) tiles3[off3 + j] = MoeTile{base, off + c3 * j / n3, off + c3 * (j + 1) / n3};
+            for (int j = 0; j < n3; j++)
+                tiles3[off3 + j] = MoeTile{base, off + tile_begin(c3, j, n3), off + tile_begin(c3, j + 1, n3)};
             for (int j = 0; j < big; j++)
                 tiles2[off2 + j] = MoeTile{base, off + c3 + j * PB, off + c3 + min(cr, (j + 1) * PB)};
             if (small) tiles1[off1] = MoeTile{base, off + c - rem, off + c};

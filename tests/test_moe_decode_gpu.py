@@ -82,3 +82,14 @@ def test_moe_forward_refuses_bad_shared_scales(dev, bad):
     with pytest.raises(ops.AegistError):
         ops.moe_forward(h, x, router, _experts(8, D, I, 3).to(dev), I, 2, shared=((w, good), (w, sc), (w, good)),
                         shared_gate=torch.zeros(D, dtype=torch.bfloat16, device=dev))
+
+
+def test_more_picks_of_one_expert_than_tile_products_fit_32_bits(dev):
+    """400000 picks of one expert: its tiles' boundaries must not be formed by products of two counts."""
+    T, D, I = 400_000, 128, 128
+    g = torch.Generator().manual_seed(5)
+    rows, h = _experts(1, D, I, 5), torch.randn(T, D, generator=g)
+    idx, wts = torch.zeros(T, 1, dtype=torch.int32), torch.rand(T, 1, generator=g)
+    x = torch.zeros(T, D, device=dev)
+    ops.moe_experts(h.to(dev), rows.to(dev), idx.to(dev), wts.to(dev), x, I)
+    assert rel_err(x, R.moe_experts(h, rows, idx.long(), wts, D, I)) < 5e-5
