@@ -30,7 +30,9 @@ typedef int int4v __attribute__((ext_vector_type(4)));
 
 constexpr int MKS = 64;                             // k per step
 constexpr int kMidBufWord3 = 0x00020000;            // buffer resource word 3 on gfx9: 32-bit data, no swizzle
-constexpr int kMidOob = 0x7ffffff0;                 // past every operand (< 2^31 - 16 bytes): loads return 0
+// past every operand (< 2^31 - 16 bytes): loads return 0. Offsets are unsigned, since a second load lies 16
+// bytes past it
+constexpr uint32_t kMidOob = 0x7ffffff0u;
 
 constexpr int MID_SEG = 4;
 struct MidSeg {
@@ -46,7 +48,11 @@ struct MidArgs {
     int nseg, ldx, M, K, accumulate, tiles_m, ntiles, per_xcd;
 };
 
-__device__ __forceinline__ int4v buf16(__amdgpu_buffer_rsrc_t rs, int off) {
+// offset of the 16 bytes that follow those at `off`
+__device__ constexpr uint32_t next16(uint32_t off) { return off + 16; }
+static_assert(next16(kMidOob) > kMidOob, "the load after an out-of-range one is out of range too");
+
+__device__ __forceinline__ int4v buf16(__amdgpu_buffer_rsrc_t rs, uint32_t off) {
     return __builtin_bit_cast(int4v, __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0));
 }
 
@@ -59,7 +65,7 @@ template <> struct MidW<int8_t> {
     static __device__ __forceinline__ int slot(int h, int g) { return 2 * g + h; }
     // k0: first k of the step; rows end at K (a multiple of 16)
     __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rs, int row, int k0, int g, int K) {
-        r = buf16(rs, k0 + 16 * g < K ? row + k0 + 16 * g : kMidOob);
+        r = buf16(rs, k0 + 16 * g < K ? (uint32_t)(row + k0 + 16 * g) : kMidOob);
     }
     __device__ __forceinline__ bf16x8 frag(int h) const {
         // int8 -> fp32 is exact and keeps 8 significant bits, so its top half is the exact bf16
@@ -82,7 +88,7 @@ template <> struct MidW<uint16_t> {
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             const int k = k0 + 32 * h + 8 * g;
-            r[h] = buf16(rs, k < K ? (row + k) * 2 : kMidOob);
+            r[h] = buf16(rs, k < K ? (uint32_t)(row + k) * 2 : kMidOob);
         }
     }
     __device__ __forceinline__ bf16x8 frag(int h) const { return __builtin_bit_cast(bf16x8, r[h]); }
@@ -93,9 +99,9 @@ template <typename TX> struct MidX;
 template <> struct MidX<float> {
     static constexpr int kParts = 2;
     int4v r[2];
-    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rs, int off) {
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rs, uint32_t off) {
         r[0] = buf16(rs, off);
-        r[1] = buf16(rs, off + 16);
+        r[1] = buf16(rs, next16(off));
     }
     // x = hi + lo, hi = x truncated to bf16, lo = the rounded remainder: |x - hi - lo| <= 2^-16 |x|
     __device__ __forceinline__ void store(unsigned char* dst, int part) const {
@@ -117,7 +123,7 @@ template <> struct MidX<float> {
 template <> struct MidX<uint16_t> {
     static constexpr int kParts = 1;
     int4v r;
-    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rs, int off) { r = buf16(rs, off); }
+    __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rs, uint32_t off) { r = buf16(rs, off); }
     __device__ __forceinline__ void store(unsigned char* dst, int) const { *(int4v*)dst = r; }
 };
 
@@ -170,7 +176,7 @@ __global__ void __launch_bounds__(64 * NWN * KG) gemm_mid_kernel(const MidArgs g
         const int k0 = (kg + KG * t) * MKS;
         const bool ok = k0 + xs8 < K;
 #pragma unroll
-        for (int i = 0; i < SL; i++) xr[set][i].load(xrs, ok ? (xbase[i] + k0) * (int)sizeof(TX) : kMidOob);
+        for (int i = 0; i < SL; i++) xr[set][i].load(xrs, ok ? (uint32_t)(xbase[i] + k0) * (uint32_t)sizeof(TX) : kMidOob);
     };
     auto load_w = [&](int slot, int t) {
 #pragma unroll
