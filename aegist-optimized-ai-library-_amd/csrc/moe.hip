@@ -161,7 +161,7 @@ __global__ void __launch_bounds__(256) router_topk_kernel(const float* __restric
 // counts up, scans them over the experts and places its block's picks. (One workgroup doing all of it
 // took 32 us for 16384 picks, twice through LDS atomics; 8 us each in blocks of 1024, the activation
 // split's 8 us included.)
-// An expert's positions are cut into tiles: in big mode all into ceil(c / 64) balanced ones (tiles3,
+// An expert's positions are cut into tiles: with a `cap` all into ceil(c / cap) balanced ones (tiles3,
 // meta[3] of them), else into blocks of 17..32 (tiles2, meta[2]) and a last one of <= 16 (tiles1,
 // meta[0]). meta[1] = dropped picks. The order of positions inside an expert is unspecified (atomics);
 // no result depends on it (every pick's sums run in the same order whatever tile it lands in with whom).
@@ -214,7 +214,7 @@ __global__ void __launch_bounds__(1024) moe_place_kernel(const int* __restrict__
                                                          int* __restrict__ eoff, int* __restrict__ ptok,
                                                          int* __restrict__ psrc, MoeTile* __restrict__ tiles1,
                                                          MoeTile* __restrict__ tiles2, MoeTile* __restrict__ tiles3,
-                                                         int big3, int* __restrict__ meta) {
+                                                         int cap, int* __restrict__ meta) {
     __shared__ int cur[MAX_E], wsum[16];
     const int tid = threadIdx.x, b = blockIdx.x;
     int c = 0, mine = 0;  // the expert's picks; those of the blocks before this one
@@ -230,7 +230,7 @@ __global__ void __launch_bounds__(1024) moe_place_kernel(const int* __restrict__
     const int off = block_excl_scan(c, wsum, &tot_c);
     if (tid < E) cur[tid] = off + mine;
     if (b == 0) {
-        const int n3 = big3 ? (c + PBB - 1) / PBB : 0;
+        const int n3 = cap ? (c + cap - 1) / cap : 0;
         const int c3 = n3 > 0 ? c : 0, cr = c - c3, rem = cr % PB;
         const int small = rem > 0 && rem <= 16 ? 1 : 0;      // the last block, if it is small
         const int big = cr / PB + (rem > 16 ? 1 : 0);        // full blocks and a large last block
@@ -638,6 +638,7 @@ constexpr int NWB = 8;         // waves per big workgroup (one workgroup per CU)
 constexpr int RTB = 4;         // row tiles per wave
 constexpr int UB = 32 * NWB;   // units per gate / up workgroup
 constexpr int OB = 64 * NWB;   // output rows per down workgroup
+static_assert(2 * UB == kMoeRows && OB == kMoeRows, "moe_tile_picks counts workgroups of this many rows");
 
 // Scales and group sums lie group-major: a lane's 4 rows of scales are one 8-byte read, the picks' sums
 // 16 consecutive words, and every offset is a constant.
@@ -1087,7 +1088,8 @@ static bool big_tiles_enabled() {
 struct MoePlan {
     size_t xh, xl, xs, ah, al, as, yp, cnt, eoff, ptok, psrc, tiles1, tiles2, tiles3, meta, total;
     int per, nb;           // grouping: picks per block, blocks (at most 64: each reads all the blocks' counts)
-    int max1, max2, max3;  // tile-list capacities: <= 16 picks (one per expert), 17..32, 33..64
+    int cap;               // picks per prefill tile, 0: the tiles of <= 32 picks
+    int max1, max2, max3;  // tile-list capacities: <= 16 picks (one per expert), 17..32, prefill tiles
 };
 static size_t al256(size_t x) { return (x + 255) / 256 * 256; }
 static MoePlan moe_plan(int T, int K, int D, int I, int E) {
@@ -1096,7 +1098,11 @@ static MoePlan moe_plan(int T, int K, int D, int I, int E) {
     p.max1 = (int)std::min<size_t>(N, (size_t)E);
     // an expert with c picks has floor(c / PB) + [c % PB > 16] <= c / 17 large blocks
     p.max2 = (int)(N / 17);
-    p.max3 = (int)(N / PBB + std::min<size_t>(N, (size_t)E));  // sum of ceil(c / 64)
+    // the prefill tiles' rows are whole pairs of groups up to 2048, addressed through 32-bit byte offsets
+    const bool fits = D % 128 == 0 && I % 128 == 0 && D / 64 <= 32 && I / 64 <= 32 && (size_t)T * D * 2 < (1ull << 32) &&
+                      N * I * 2 < (1ull << 32);
+    p.cap = fits ? moe_tile_picks(T, K, E, D, I) : 0;
+    p.max3 = p.cap ? (int)(N / p.cap + std::min<size_t>(N, (size_t)E)) : 0;  // sum of ceil(c / cap)
     p.per = (int)std::max<size_t>(1024, (N + 63) / 64);
     p.nb = (int)((N + p.per - 1) / p.per);
     size_t o = 0;
@@ -1206,20 +1212,16 @@ int aegist_moe_experts(const float* h, const unsigned long long* eptr, const int
         moe_combine_kernel<<<dim3(T, (D + 255) / 256), 256, 0, st>>>(x, yp, idx, E, ysh, h, wg, D, K);
         return after_launch("moe_combine");
     }
-    // the prefill tiles wherever the shapes allow (they address activation rows through 32-bit byte
-    // offsets): against the tiles of <= 32 picks 223 -> 173 us at 80 tokens (640 picks of 256 experts),
-    // 240 -> 177 at 200, 320 -> 199 at 512, 418 -> 243 at 1000
-    const bool big = D % 128 == 0 && I % 128 == 0 && D / 64 <= 32 && I / 64 <= 32 &&
-                     (long long)T * D * 2 < (1LL << 32) && (long long)N * I * 2 < (1LL << 32) && big_tiles_enabled();
+    const int cap = big_tiles_enabled() ? p.cap : 0;
     int* cnt = (int*)(w + p.cnt);
     const long long nq = (long long)T * (D / 8);
     moe_count_kernel<<<p.nb + (unsigned)((nq + 255) / 256), 256, 0, st>>>(idx, N, E, p.per, p.nb, cnt, h, T, D, xh, xl, xs);
     int rc = after_launch("moe_count");
     if (rc) return rc;
     moe_place_kernel<<<p.nb, 1024, 0, st>>>(idx, N, K, E, p.per, p.nb, cnt, eptr, eoff, ptok, psrc, tiles1, tiles2, tiles3,
-                                            big ? 1 : 0, meta);
+                                            cap, meta);
     if ((rc = after_launch("moe_place"))) return rc;
-    if (big) {
+    if (cap) {
         moe_gate_up_big_kernel<<<dim3((I + UB - 1) / UB, p.max3), 64 * NWB, 0, st>>>(tiles3, meta + 3, ptok, xh, xl, xs, D, I, off, ah,
                                                                    al, as);
         if ((rc = after_launch("moe_gate_up_big"))) return rc;

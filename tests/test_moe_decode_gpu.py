@@ -93,3 +93,22 @@ def test_more_picks_of_one_expert_than_tile_products_fit_32_bits(dev):
     x = torch.zeros(T, D, device=dev)
     ops.moe_experts(h.to(dev), rows.to(dev), idx.to(dev), wts.to(dev), x, I)
     assert rel_err(x, R.moe_experts(h, rows, idx.long(), wts, D, I)) < 5e-5
+
+
+@pytest.mark.parametrize("T,D,I,E,K", [(70, 384, 256, 256, 8), (96, 256, 256, 8, 2), (128, 384, 256, 8, 2), (2048, 256, 256, 4, 2),
+                                       (5000, 256, 256, 8, 2), (9000, 256, 256, 8, 2), (1, 256, 768, 64, 8), (9, 512, 512, 8, 2),
+                                       (100, 256, 192, 8, 4)])
+def test_moe_tile_sizes_match_oracle(dev, T, D, I, E, K):
+    """Every size of tile the rule picks (test_moe_tiles.py has it for these batches): prefill tiles of up to
+    64 with 1 to 8 picks, 64-row workgroups at 17 to 32 picks, prefill tiles of up to 16, 32, 48 and 64;
+    64-row workgroups for one token and few experts, and for units that are no multiple of 128."""
+    print(f"moe tiles T={T} D={D} I={I} E={E} K={K}", flush=True)
+    g = torch.Generator().manual_seed(T + D + I)
+    rows, h = _experts(E, D, I, T + E), torch.randn(T, D, generator=g)
+    idx = torch.topk(torch.rand(T, E, generator=g), K, -1).indices.int()
+    wts = torch.rand(T, K, generator=g)
+    x = torch.zeros(T, D, device=dev)
+    ops.moe_experts(h.to(dev), rows.to(dev), idx.to(dev), wts.to(dev), x, I)
+    err = rel_err(x, R.moe_experts(h, rows, idx.long(), wts, D, I))
+    print(f"  rel err {err:.2e}", flush=True)
+    assert err < 5e-5

@@ -1,4 +1,4 @@
-"""The cut of an expert's picks into tiles (csrc/moe_tiles.h), compiled for the CPU: the arithmetic at the
+"""The cut of a batch's picks into tiles (csrc/moe_tiles.h), compiled for the CPU: the rule, and the arithmetic at the
 largest batches, where a GPU run would need every pick's buffers."""
 import ctypes
 import subprocess
@@ -9,6 +9,7 @@ from conftest import PKG
 
 SRC = """#include "moe_tiles.h"
 extern "C" int tile_begin(int c, int j, int n) { return aegist::tile_begin(c, j, n); }
+extern "C" int tile_picks(int T, int K, int E, int D, int I) { return aegist::moe_tile_picks(T, K, E, D, I); }
 """
 
 
@@ -29,3 +30,41 @@ def test_tiles_cover_the_picks_in_order(tiles, c):
     for j in js:
         a, b = tiles.tile_begin(c, j, n), tiles.tile_begin(c, j + 1, n)
         assert c // n <= b - a <= min(64, c // n + 1), (j, a, b)
+
+
+@pytest.mark.parametrize("T,K,E,I,picks", [
+    # too few workgroups of 256 units: few experts, one token's picks at widths the decode kernel does not take
+    (9, 2, 8, 512, 0), (32, 2, 8, 512, 0), (1, 8, 256, 768, 0), (4, 8, 256, 256, 0), (1, 2, 8, 1408, 0), (16, 4, 16, 128, 0),
+    # the second round of workgroups nearly empty; padded units
+    (16, 8, 256, 768, 0), (24, 8, 128, 768, 0), (64, 8, 256, 1408, 0),
+    # experts of 17 to 32 picks, few workgroups
+    (192, 2, 16, 768, 0), (96, 4, 16, 256, 0),
+    # full rounds
+    (65, 8, 256, 512, 64), (96, 8, 256, 512, 64), (128, 8, 256, 512, 64), (512, 8, 256, 512, 64), (1000, 8, 256, 512, 64),
+    (2048, 8, 256, 512, 64), (64, 8, 256, 256, 64), (128, 8, 256, 768, 64),
+    # experts past 16 picks that leave room for smaller tiles
+    (128, 2, 8, 512, 16), (512, 2, 8, 1408, 32), (400_000, 1, 1, 128, 64), (2048, 2, 4, 256, 32)])
+def test_tile_rule(tiles, T, K, E, I, picks):
+    assert tiles.tile_picks(T, K, E, 2048, I) == picks
+
+
+def test_tile_rule_takes_any_batch(tiles):
+    for E in (1, 2, 5, 16, 255, 1024):
+        for K in (1, 2, 8, 16):
+            for T in (1, 2, 17, 333, 70_000, 2 ** 30 // K - 1):
+                for I in (128, 640, 2048):
+                    assert tiles.tile_picks(T, K, E, 640, I) in (0, 16, 32, 48, 64)
+
+
+def test_tile_rule_counts_the_longer_rows_workgroups(tiles):
+    """Wide experts of a narrow model: the down projection's few outputs decide."""
+    assert tiles.tile_picks(24, 4, 32, 256, 2048) == 0 and tiles.tile_picks(96, 8, 256, 512, 2048) == 64
+
+
+# the batches of test_moe_decode_gpu.py's sizes of tiles
+@pytest.mark.parametrize("T,D,I,E,K,picks", [(70, 384, 256, 256, 8, 64), (96, 256, 256, 8, 2, 0), (128, 384, 256, 8, 2, 16),
+                                             (1024, 256, 256, 4, 2, 16), (2048, 256, 256, 4, 2, 32),
+                                             (5000, 256, 256, 8, 2, 48), (9000, 256, 256, 8, 2, 64),
+                                             (1, 256, 768, 64, 8, 0), (9, 512, 512, 8, 2, 0)])
+def test_tile_rule_of_the_gpu_test(tiles, T, D, I, E, K, picks):
+    assert tiles.tile_picks(T, K, E, D, I) == picks
