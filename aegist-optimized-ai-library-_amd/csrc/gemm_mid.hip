@@ -127,8 +127,26 @@ template <> struct MidX<uint16_t> {
     __device__ __forceinline__ void store(unsigned char* dst, int) const { *(int4v*)dst = r; }
 };
 
-template <typename TW, typename TX, int RT, int MT, int NWN, int KG, int PD>
+// With exact bf16 X what is left of an output's error is the fp32 sums' and grows with the root of the number
+// of products added one after the other. So they are short chains where they were before these tiles (kShort: up
+// to 64 rows, and int8 weights): kSets sets of accumulators take the step's 32-k halves (and, of four, the
+// steps) in turn, K / (KG kSets) products each; the forms of few K groups that int8 weights take at the largest
+// batches add theirs up every kFlush steps. 2-norm error, one set and now: bf16 16 rows of 8192 x 2048 1.31e-7,
+// 0.98e-7, of 2048 x 4096 1.37e-7, 1.06e-7, 64 of 12352 x 2048 1.86e-7, 0.98e-7; int8 W, bf16 X, 600 rows of
+// 4096 x 8192 2.79e-7, 1.0e-7. It costs 0 to 6% at up to 64 rows, up to 14% at 300 of int8 12352 x 2048. (Past 64 rows
+// bf16 W is in the place of full-K chains. fp32 X: its split's 2^-17 is 40 times as much; one set.)
+template <typename TW, typename TX, int RT, int MT, int KG, bool kShort>
+struct MidSums {
+    static constexpr bool kBf16X = MidX<TX>::kParts == 1, kI8 = sizeof(TW) == 1;
+    static constexpr int kFlush = kBf16X && kI8 && KG <= 2 ? 4 : 0;
+    static constexpr int kSets = !kBf16X || !kShort || kFlush || KG == 1 ? 1 : KG == 2 && RT * MT <= 4 ? 4 : 2;
+};
+
+template <typename TW, typename TX, int RT, int MT, int NWN, int KG, int PD, bool kShort>
 __global__ void __launch_bounds__(64 * NWN * KG) gemm_mid_kernel(const MidArgs ga) {
+    using Sums = MidSums<TW, TX, RT, MT, KG, kShort>;
+    constexpr int kSets = Sums::kSets, kFlush = Sums::kFlush;
+    static_assert(kFlush % PD == 0 && kSets <= 2 * PD, "sums are flushed between rounds of PD steps");
     constexpr int BM = 16 * MT, BN = 16 * RT * NWN, TPG = 64 * NWN, SL = BM * 8 / TPG;
     static_assert(SL >= 1 && SL * TPG == BM * 8, "the X stage must split evenly over the group's threads");
     constexpr int kPart = BM * MKS * 2;                       // bytes of one part (hi or lo) of an X stage
@@ -187,11 +205,15 @@ __global__ void __launch_bounds__(64 * NWN * KG) gemm_mid_kernel(const MidArgs g
         for (int i = 0; i < SL; i++) xr[set][i].store(buf + (t & 1) * kStage + xdst[i], kPart);
     };
 
-    f32x4 acc[RT][MT];
+    f32x4 part[kSets][RT][MT], acc[RT][MT];
 #pragma unroll
     for (int rt = 0; rt < RT; rt++)
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++) acc[rt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int mt = 0; mt < MT; mt++) {
+#pragma unroll
+            for (int u = 0; u < kSets; u++) part[u][rt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+            acc[rt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
 
     // the row scales of the lane's 4 RT outputs, requested before the stream
     const bool fin = kg == 0;
@@ -219,6 +241,7 @@ __global__ void __launch_bounds__(64 * NWN * KG) gemm_mid_kernel(const MidArgs g
         const unsigned char* cur = buf + (slot & 1) * kStage;  // PD is even: slot and t agree
 #pragma unroll
         for (int ks = 0; ks < 2; ks++) {
+            f32x4(&sum)[RT][MT] = part[(2 * slot + ks) % kSets];
             bf16x8 a[RT];
 #pragma unroll
             for (int rt = 0; rt < RT; rt++) a[rt] = wr[slot][rt].frag(ks);
@@ -230,12 +253,12 @@ __global__ void __launch_bounds__(64 * NWN * KG) gemm_mid_kernel(const MidArgs g
                 const bf16x8 bh = *(const bf16x8*)p;
 #pragma unroll
                 for (int rt = 0; rt < RT; rt++)
-                    acc[rt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rt], bh, acc[rt][mt], 0, 0, 0);
+                    sum[rt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rt], bh, sum[rt][mt], 0, 0, 0);
                 if constexpr (MidX<TX>::kParts == 2) {
                     const bf16x8 bl = *(const bf16x8*)(p + kPart);
 #pragma unroll
                     for (int rt = 0; rt < RT; rt++)
-                        acc[rt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rt], bl, acc[rt][mt], 0, 0, 0);
+                        sum[rt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rt], bl, sum[rt][mt], 0, 0, 0);
                 }
             }
         }
@@ -245,7 +268,27 @@ __global__ void __launch_bounds__(64 * NWN * KG) gemm_mid_kernel(const MidArgs g
     for (int t = 0; t < nt; t += PD) {
 #pragma unroll
         for (int d = 0; d < PD; d++) step(t + d, d);
+        if constexpr (kFlush > 0) {
+            if ((t + PD) % kFlush == 0) {
+#pragma unroll
+                for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+                    for (int mt = 0; mt < MT; mt++) {
+                        acc[rt][mt] += part[0][rt][mt];
+                        part[0][rt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    }
+            }
+        }
     }
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+        for (int mt = 0; mt < MT; mt++) {
+            if constexpr (kSets == 4) acc[rt][mt] = (part[0][rt][mt] + part[1][rt][mt]) + (part[2][rt][mt] + part[3][rt][mt]);
+            else if constexpr (kSets == 2) acc[rt][mt] = part[0][rt][mt] + part[1][rt][mt];
+            else if constexpr (kFlush > 0) acc[rt][mt] += part[0][rt][mt];
+            else acc[rt][mt] = part[0][rt][mt];
+        }
 
     if constexpr (KG > 1) {
         // the K groups' partial tiles, added in group order
@@ -344,7 +387,12 @@ int launch_mid(MidArgs ga, hipStream_t st) {
     }
     ga.ntiles = ga.tiles_m * t;
     ga.per_xcd = (ga.ntiles + 7) / 8;
-    gemm_mid_kernel<TW, TX, RT, MT, NWN, KG, PD><<<8 * ga.per_xcd, 64 * NWN * KG, 0, st>>>(ga);
+    // (one instance where both would be the same)
+    constexpr bool both = MidSums<TW, TX, RT, MT, KG, true>::kSets > 1 && sizeof(TW) == 2 && MT > 1;
+    if (both && ga.M > 64)
+        gemm_mid_kernel<TW, TX, RT, MT, NWN, KG, PD, !both><<<8 * ga.per_xcd, 64 * NWN * KG, 0, st>>>(ga);
+    else
+        gemm_mid_kernel<TW, TX, RT, MT, NWN, KG, PD, true><<<8 * ga.per_xcd, 64 * NWN * KG, 0, st>>>(ga);
     return after_launch("gemm_mid");
 }
 
