@@ -420,9 +420,11 @@ int run_mid(int form, const MidArgs& ga, hipStream_t st) {
 namespace aegist {
 
 // The form this file's kernel would take the product in, or -1 if the 256 x 256 tiles of gemm.hip are
-// estimated faster (`tile256`: they could take it, as one launch of all weights). Every operand is
-// below 2^31 - 16 bytes (the caller splits larger ones), K % 16 == 0, rows 16-byte aligned.
-int gemm_mid_form(int x_dtype, int nseg, const int* N, int M, int K, bool tile256) {
+// estimated faster (`tile256`: they could take it; `stacked`: as one launch of all weights, else one after the
+// other, each in rounds of its own: bf16 8192, 4096, 32 and 32 rows x 2048 at 1024 rows of X take
+// 176 us that way and 85 here). Every operand is below 2^31 - 16 bytes (the caller splits larger ones),
+// K % 16 == 0, rows 16-byte aligned.
+int gemm_mid_form(int x_dtype, int nseg, const int* N, int M, int K, bool tile256, bool stacked) {
     if (M <= 16) {
         long long rows = 0;
         for (int i = 0; i < nseg; i++) rows += N[i];
@@ -431,15 +433,18 @@ int gemm_mid_form(int x_dtype, int nseg, const int* N, int M, int K, bool tile25
     MidArgs ga{};
     ga.nseg = nseg;
     ga.M = M;
-    long long t256 = 0;
+    const long long tm = (M + 255) / 256;
+    auto rounds256 = [&](long long n) { return ((n + 255) / 256 * tm + 255) / 256; };
+    long long rows = 0, r256 = 0;
     for (int i = 0; i < nseg; i++) {
         ga.seg[i].N = N[i];
-        t256 += N[i];
+        rows += N[i];
+        r256 += rounds256(N[i]);
     }
-    t256 = (t256 + 255) / 256 * ((M + 255) / 256);
+    if (stacked) r256 = rounds256(rows);
     const MidForm* forms = x_dtype == AEGIST_F32 ? kFormsF32 : kFormsBf16;
     int best = -1;
-    float least = tile256 ? ((t256 + 255) / 256) * (x_dtype == AEGIST_F32 ? kTile256F32 : kTile256Bf16) : 3.4e38f;
+    float least = tile256 ? r256 * (x_dtype == AEGIST_F32 ? kTile256F32 : kTile256Bf16) : 3.4e38f;
     for (int i = 0; i < (x_dtype == AEGIST_F32 ? kNF32 : kNBf16); i++) {
         const long long t = mid_tiles(forms[i], ga);
         const float est = forms[i].base + ((t + 255) / 256) * forms[i].cost;

@@ -28,7 +28,7 @@ int launch_gemm_bf16(const uint16_t* X, long long ldx, const uint16_t* W, long l
 int launch_gemm_bf16_multi(const uint16_t* X, long long ldx, int nseg, const uint16_t* const* W, const long long* ldw,
                            float* const* Y, const long long* ldy, const int* N, int M, int K, int accumulate,
                            hipStream_t st);
-int gemm_mid_form(int x_dtype, int nseg, const int* N, int M, int K, bool tile256);
+int gemm_mid_form(int x_dtype, int nseg, const int* N, int M, int K, bool tile256, bool stacked);
 int launch_gemv(const void* X, int x_dtype, long long ldx, int w_dtype, int nseg, const void* const* W,
                 const uint16_t* const* scale, float* const* Y, const long long* ldy, const int* N, int M, int K,
                 int accumulate, hipStream_t st);
@@ -256,7 +256,7 @@ int run_proj(const void* X, int xd, long long ldx, int wd, const ProjSegs& segs,
         launch_stream<2, 2>((const uint16_t*)X, ldx, segs, M, K, accumulate, st);
         return after_launch("proj_stream");
     }
-    const int form = gemm_mid_form(xd, segs.n, N, M, K, tile256);
+    const int form = gemm_mid_form(xd, segs.n, N, M, K, tile256, !i8 && stack8);
     if (form >= 0)
         return launch_gemm_mid(form, X, xd, ldx, wd, segs.n, W, scale, Y, ldy, N, M, K, accumulate, st);
     if (i8) {
