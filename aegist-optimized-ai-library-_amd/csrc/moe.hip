@@ -154,16 +154,15 @@ __global__ void __launch_bounds__(256) router_topk_kernel(const float* __restric
 }
 
 // ---------------------------------------------------------------------------------------------
-// Grouping: picks i = t K + k with expert idx[i]; out of range experts are dropped and counted.
-// eoff[E + 1]: exclusive prefix of the counts; ptok / psrc: token and pick index of each grouped
-// position. Two launches, each over blocks of `per` picks: moe_count_kernel counts the block's picks per
+// Grouping: picks i = t K + k with expert idx[i]; out of range experts are dropped. ptok / psrc: token and
+// pick index of each grouped position. Two launches, each over blocks of `per` picks: moe_count_kernel counts the block's picks per
 // expert in LDS (its other workgroups split the activations), moe_place_kernel adds the blocks'
 // counts up, scans them over the experts and places its block's picks. (One workgroup doing all of it
 // took 32 us for 16384 picks, twice through LDS atomics; 8 us each in blocks of 1024, the activation
 // split's 8 us included.)
 // An expert's positions are cut into tiles: with a `cap` all into ceil(c / cap) balanced ones (tiles3,
-// meta[3] of them), else into blocks of 17..32 (tiles2, meta[2]) and a last one of <= 16 (tiles1,
-// meta[0]). meta[1] = dropped picks. The order of positions inside an expert is unspecified (atomics);
+// meta[2] of them), else into blocks of 17..32 (tiles2, meta[1]) and a last one of <= 16 (tiles1,
+// meta[0]). The order of positions inside an expert is unspecified (atomics);
 // no result depends on it (every pick's sums run in the same order whatever tile it lands in with whom).
 __device__ __forceinline__ int block_excl_scan(int v, int* wsum, int* total) {
     const int lane = threadIdx.x % WAVE, w = threadIdx.x / WAVE, nw = blockDim.x / WAVE;
@@ -211,10 +210,10 @@ __global__ void __launch_bounds__(256) moe_count_kernel(const int* __restrict__ 
 __global__ void __launch_bounds__(1024) moe_place_kernel(const int* __restrict__ idx, int N, int K, int E, int per, int nb,
                                                          const int* __restrict__ cnt,
                                                          const unsigned long long* __restrict__ eptr,
-                                                         int* __restrict__ eoff, int* __restrict__ ptok,
-                                                         int* __restrict__ psrc, MoeTile* __restrict__ tiles1,
-                                                         MoeTile* __restrict__ tiles2, MoeTile* __restrict__ tiles3,
-                                                         int cap, int* __restrict__ meta) {
+                                                         int* __restrict__ ptok, int* __restrict__ psrc,
+                                                         MoeTile* __restrict__ tiles1, MoeTile* __restrict__ tiles2,
+                                                         MoeTile* __restrict__ tiles3, int cap,
+                                                         int* __restrict__ meta) {
     __shared__ int cur[MAX_E], wsum[16];
     const int tid = threadIdx.x, b = blockIdx.x;
     int c = 0, mine = 0;  // the expert's picks; those of the blocks before this one
@@ -226,8 +225,8 @@ __global__ void __launch_bounds__(1024) moe_place_kernel(const int* __restrict__
             c += v;
         }
     }
-    int tot_c;
-    const int off = block_excl_scan(c, wsum, &tot_c);
+    int total;
+    const int off = block_excl_scan(c, wsum, &total);
     if (tid < E) cur[tid] = off + mine;
     if (b == 0) {
         const int n3 = cap ? (c + cap - 1) / cap : 0;
@@ -239,7 +238,6 @@ __global__ void __launch_bounds__(1024) moe_place_kernel(const int* __restrict__
         const int off2 = block_excl_scan(big, wsum, &tot_2);
         const int off3 = block_excl_scan(n3, wsum, &tot_3);
         if (tid < E) {
-            eoff[tid] = off;
             const unsigned long long base = c > 0 ? eptr[tid] : 0ull;
             for (int j = 0; j < n3; j++)
                 tiles3[off3 + j] = MoeTile{base, off + tile_begin(c3, j, n3), off + tile_begin(c3, j + 1, n3)};
@@ -248,11 +246,9 @@ __global__ void __launch_bounds__(1024) moe_place_kernel(const int* __restrict__
             if (small) tiles1[off1] = MoeTile{base, off + c - rem, off + c};
         }
         if (tid == 0) {
-            eoff[E] = tot_c;
             meta[0] = tot_1;
-            meta[1] = N - tot_c;
-            meta[2] = tot_2;
-            meta[3] = tot_3;
+            meta[1] = tot_2;
+            meta[2] = tot_3;
         }
     }
     __syncthreads();
@@ -1086,7 +1082,7 @@ static bool big_tiles_enabled() {
 
 // Workspace plan of aegist_moe_experts.
 struct MoePlan {
-    size_t xh, xl, xs, ah, al, as, yp, cnt, eoff, ptok, psrc, tiles1, tiles2, tiles3, meta, total;
+    size_t xh, xl, xs, ah, al, as, yp, cnt, ptok, psrc, tiles1, tiles2, tiles3, meta, total;
     int per, nb;           // grouping: picks per block, blocks (at most 64: each reads all the blocks' counts)
     int cap;               // picks per prefill tile, 0: the tiles of <= 32 picks
     int max1, max2, max3;  // tile-list capacities: <= 16 picks (one per expert), 17..32, prefill tiles
@@ -1119,7 +1115,6 @@ static MoePlan moe_plan(int T, int K, int D, int I, int E) {
     p.as = take(N * (I / 64) * 4);
     p.yp = take(N * D * 4);
     p.cnt = take((size_t)p.nb * E * 4);
-    p.eoff = take((size_t)(E + 1) * 4);
     p.ptok = take(N * 4);
     p.psrc = take(N * 4);
     p.tiles1 = take((size_t)p.max1 * sizeof(MoeTile));
@@ -1189,7 +1184,6 @@ int aegist_moe_experts(const float* h, const unsigned long long* eptr, const int
     hipStream_t st = AEG_STREAM(stream);
     const ExpertOffsets off = expert_offsets(D, I);
     const int N = T * K;
-    int* eoff = (int*)(w + p.eoff);
     int* ptok = (int*)(w + p.ptok);
     int* psrc = (int*)(w + p.psrc);
     MoeTile* tiles1 = (MoeTile*)(w + p.tiles1);
@@ -1218,14 +1212,13 @@ int aegist_moe_experts(const float* h, const unsigned long long* eptr, const int
     moe_count_kernel<<<p.nb + (unsigned)((nq + 255) / 256), 256, 0, st>>>(idx, N, E, p.per, p.nb, cnt, h, T, D, xh, xl, xs);
     int rc = after_launch("moe_count");
     if (rc) return rc;
-    moe_place_kernel<<<p.nb, 1024, 0, st>>>(idx, N, K, E, p.per, p.nb, cnt, eptr, eoff, ptok, psrc, tiles1, tiles2, tiles3,
-                                            cap, meta);
+    moe_place_kernel<<<p.nb, 1024, 0, st>>>(idx, N, K, E, p.per, p.nb, cnt, eptr, ptok, psrc, tiles1, tiles2, tiles3, cap, meta);
     if ((rc = after_launch("moe_place"))) return rc;
     if (cap) {
-        moe_gate_up_big_kernel<<<dim3((I + UB - 1) / UB, p.max3), 64 * NWB, 0, st>>>(tiles3, meta + 3, ptok, xh, xl, xs, D, I, off, ah,
+        moe_gate_up_big_kernel<<<dim3((I + UB - 1) / UB, p.max3), 64 * NWB, 0, st>>>(tiles3, meta + 2, ptok, xh, xl, xs, D, I, off, ah,
                                                                    al, as);
         if ((rc = after_launch("moe_gate_up_big"))) return rc;
-        moe_down_big_kernel<<<dim3((D + OB - 1) / OB, p.max3), 64 * NWB, 0, st>>>(tiles3, meta + 3, psrc, wts, ah, al, as, D,
+        moe_down_big_kernel<<<dim3((D + OB - 1) / OB, p.max3), 64 * NWB, 0, st>>>(tiles3, meta + 2, psrc, wts, ah, al, as, D,
                                                                                   I, off, yp);
         if ((rc = after_launch("moe_down_big"))) return rc;
         moe_combine_kernel<<<dim3(T, (D + 255) / 256), 256, 0, st>>>(x, yp, idx, E, ysh, h, wg, D, K);
@@ -1240,14 +1233,14 @@ int aegist_moe_experts(const float* h, const unsigned long long* eptr, const int
                                                                      as);
     if ((rc = after_launch("moe_gate_up"))) return rc;
     if (p.max2 > 0) {
-        moe_gate_up_kernel<2><<<dim3(I / RB, p.max2), 256, lds_gu, st>>>(tiles2, meta + 2, ptok, xh, xl, xs, D, I, off,
+        moe_gate_up_kernel<2><<<dim3(I / RB, p.max2), 256, lds_gu, st>>>(tiles2, meta + 1, ptok, xh, xl, xs, D, I, off,
                                                                          ah, al, as);
         if ((rc = after_launch("moe_gate_up"))) return rc;
     }
     moe_down_kernel<1><<<dim3(D / RB, p.max1), 256, lds_dn, st>>>(tiles1, meta, psrc, wts, ah, al, as, D, I, off, yp);
     if ((rc = after_launch("moe_down"))) return rc;
     if (p.max2 > 0) {
-        moe_down_kernel<2><<<dim3(D / RB, p.max2), 256, lds_dn, st>>>(tiles2, meta + 2, psrc, wts, ah, al, as, D, I,
+        moe_down_kernel<2><<<dim3(D / RB, p.max2), 256, lds_dn, st>>>(tiles2, meta + 1, psrc, wts, ah, al, as, D, I,
                                                                       off, yp);
         if ((rc = after_launch("moe_down"))) return rc;
     }

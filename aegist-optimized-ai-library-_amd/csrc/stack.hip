@@ -48,12 +48,8 @@ int stack_attn_prefill(const float* qn, const uint16_t* kc, const uint16_t* vc, 
                        int H, int KV, int T, int pos, int cap, float scale, void* ws, size_t ws_bytes, hipStream_t st,
                        uint16_t* out_bf16, bool* wrote_bf16);
 size_t prefill_f16_bytes(int B, int KV, int rows);
-bool gemm_bf16_fits(const void* X, long long ldx, const void* W, long long ldw, int M, int N, int K);
 int launch_gemm_bf16(const uint16_t* X, long long ldx, const uint16_t* W, long long ldw, float* Y, long long ldy, int M,
                      int N, int K, int accumulate, hipStream_t st);
-int launch_gemm_bf16_multi(const uint16_t* X, long long ldx, int nseg, const uint16_t* const* W, const long long* ldw,
-                           float* const* Y, const long long* ldy, const int* N, int M, int K, int accumulate,
-                           hipStream_t st);
 bool gemm_conv_fits(const void* X, long long ldx, const void* W, long long ldw, const void* conv_w, int B, int T, int N,
                     int K);
 int launch_gemm_bf16_conv(const uint16_t* X, long long ldx, const uint16_t* W, long long ldw, const uint16_t* conv_w,
