@@ -1099,6 +1099,8 @@ static MoePlan moe_plan(int T, int K, int D, int I, int E) {
                       N * I * 2 < (1ull << 32);
     p.cap = fits ? moe_tile_picks(T, K, E, D, I) : 0;
     p.max3 = p.cap ? (int)(N / p.cap + std::min<size_t>(N, (size_t)E)) : 0;  // sum of ceil(c / cap)
+    // room for the smallest tiles whatever this batch takes: a workspace for more tokens serves fewer
+    const size_t room3 = N / 16 + std::min<size_t>(N, (size_t)E);
     p.per = (int)std::max<size_t>(1024, (N + 63) / 64);
     p.nb = (int)((N + p.per - 1) / p.per);
     size_t o = 0;
@@ -1119,7 +1121,7 @@ static MoePlan moe_plan(int T, int K, int D, int I, int E) {
     p.psrc = take(N * 4);
     p.tiles1 = take((size_t)p.max1 * sizeof(MoeTile));
     p.tiles2 = take((size_t)std::max(p.max2, 1) * sizeof(MoeTile));
-    p.tiles3 = take((size_t)std::max(p.max3, 1) * sizeof(MoeTile));
+    p.tiles3 = take(room3 * sizeof(MoeTile));
     p.meta = take(16);
     p.total = o;
     return p;

@@ -68,3 +68,15 @@ def test_tile_rule_counts_the_longer_rows_workgroups(tiles):
                                              (1, 256, 768, 64, 8, 0), (9, 512, 512, 8, 2, 0)])
 def test_tile_rule_of_the_gpu_test(tiles, T, D, I, E, K, picks):
     assert tiles.tile_picks(T, K, E, D, I) == picks
+
+
+@pytest.mark.parametrize("K,D,I,E", [(8, 2048, 512, 256), (2, 512, 1408, 8), (1, 128, 128, 1), (4, 256, 256, 16), (8, 64, 192, 64)])
+def test_workspace_of_more_tokens_serves_fewer(K, D, I, E):
+    """The workspace is asked for once, for up to T tokens: its size may not fall with T, whatever tiles a
+    smaller batch takes."""
+    from aegist_mixer._lib import lib
+    size = lib().aegist_moe_workspace_bytes
+    ts = sorted({*range(1, 3000), *range(3000, 1_000_000, 997), *(int(2 ** 32 / (2 * n)) + d for n in (D, K * I) for d in (-1, 0, 1))})
+    sizes = [size(t, K, D, I, E) for t in ts]
+    for t, a, b in zip(ts, sizes, sizes[1:]):
+        assert a <= b, (t, a, b)
