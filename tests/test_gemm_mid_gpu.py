@@ -1,4 +1,4 @@
-"""GPU parity of the middling-batch projections (17 rows and more, csrc/gemm_mid.hip) against fp64 dot
+"""GPU parity of the projections of one row and more (csrc/gemv.hip, csrc/gemm_mid.hip) against fp64 dot
 products of the exact operands, at the edges of their tiles (16 to 128 rows of X, 16 to 256 of W, 64 k
 split over 1 to 8 wave groups). bf16 products are exact and summed in fp32: every output is within
 K 2^-24 sum |x w s| of the exact one; fp32 X enters as bf16 hi + lo, within another 2^-16 sum |x w s|."""

@@ -54,7 +54,8 @@ def test_router_rounds_take_the_lowest_of_equals(dev, T, E, K):
                                            (65, 1024, 512, 16, 16, 16)])
 def test_moe_prefill_tiles_match_oracle(dev, T, D, I, E, K, hot):
     """The prefill tiles (csrc/moe.hip) at 1 to 64 picks a tile, row lengths whose groups are no multiple of
-    8 (6, 10, 2), outputs and units that end inside a workgroup, and a grouping of more than 64 blocks."""
+    8 (6, 10, 2), outputs and units that end inside a workgroup, and a grouping of more than 64 blocks; the
+    700 tokens of 300 narrow experts take the 64-row workgroups of up to 16 picks."""
     print(f"moe prefill T={T} D={D} I={I} E={E} K={K}", flush=True)
     g = torch.Generator().manual_seed(T + D + I)
     rows, h = _experts(E, D, I, T + E), torch.randn(T, D, generator=g)

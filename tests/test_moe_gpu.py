@@ -107,10 +107,9 @@ def _run_experts(dev, T, D, I, E, K, seed, x0=None, shared=False, eptr_perm=None
 @pytest.mark.parametrize("T,E,K", [(1, 256, 8), (16, 256, 8), (4, 8, 8), (300, 16, 8), (200, 16, 8), (130, 8, 4),
                                    (512, 64, 8), (100, 24, 8)])
 def test_moe_experts(dev, T, E, K):
-    """Decode and prefill batches: in batches of 16 or more picks per expert on average, experts
-    with more than 32 picks take balanced tiles of up to 64 (300 x 8 / 16: 150 each = 3 x 50;
-    200 x 8 / 16: 2 x 50; 130 x 4 / 8: 65 = 33 + 32; 512 x 8 / 64: ~64 each, one or two tiles;
-    100 x 8 / 24: ~33 each, so some experts stay on the <= 32-pick tiles)."""
+    """Decode batches (1 x 8 / 256, 16 x 8 / 256), few experts past them on 64-row workgroups (4 x 8 / 8), and
+    prefill tiles, balanced, of up to 32 picks (300 x 8 / 16: 150 each = 5 x 30), 16 (200 x 8 / 16, 130 x 4 / 8,
+    100 x 8 / 24) and 48 (512 x 8 / 64: ~64 each, two tiles)."""
     print(f"moe experts T={T} E={E} K={K}", flush=True)
     got, ref = _run_experts(dev, T, 2048, 512, E, K, seed=T * 7 + E)
     err = rel_err(got, ref)
