@@ -24,7 +24,7 @@ HIPCC_FLAGS = [
     "-std=c++17",
     "-fPIC",
     # packed fp32 VALU ops are kept out of every code object (they have shown silent
-    # wrong results on this GPU pool)
+    # wrong results on MI355X)
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-result",
 ]

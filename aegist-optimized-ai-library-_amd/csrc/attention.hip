@@ -1302,8 +1302,9 @@ __device__ __forceinline__ bf16x8 vt_operand_sw(const uint16_t* vt, int ks, int 
 
 // Depth of the K and V fragment rings of the kernel below. The K ring runs through both halves of a
 // 64-key tile, so the second half's first operands are read under the first half's products instead
-// of after them (B = 4, T = 2000: 234 -> 230 us; B = 1, T = 2000: 83 -> 79.5 us, with the launch
-// that makes the fp16 copy). Deeper rings (4 to 8 for either) only cost registers: 232 to 235 us.
+// of after them (whole call with the launch that makes the fp16 copy, B = 4, T = 2000: 217.4 -> 214.4 us, traced
+// 239 with 8 of the copy; B = 1, T = 2000: 83 -> 79.5 us). Deeper rings (4 to 8 for either) only cost
+// registers: 1 to 2% more.
 constexpr int KR = 3, VR = 4;
 
 template <typename Tout>

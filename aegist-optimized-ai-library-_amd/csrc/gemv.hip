@@ -7,10 +7,10 @@
 // run on the VALU in fp32 (x and w exactly, no hi / lo parts), which at one or two rows costs less than
 // the MFMA forms' conversion, LDS and barrier steps; the R rows of a wave are summed over the lanes by
 // halving exchanges. R, the waves a row is split over and the pieces in flight: see gemv_launch.
-// Measured against the MFMA row-tile kernel this replaces (us, weights from HBM, one row): bf16 W, fp32 X
-// 32768 x 2048 36.3 -> 23.4 (5.7 TB/s), 256 x 2048 6.3 -> 3.0; int8 W, fp32 X 2048 x 4096 8.4 -> 4.9,
-// 4096 x 2048 5.6 -> 5.3, 512 x 2048 5.6 -> 3.7, 8192 x 2048 7.1 (alike); bf16 both 9216 x 2048
-// 11.3 -> 8.8, 2048 x 4096 7.5 -> 5.8.
+// Measured against the MFMA row-tile kernel this replaces (us per launch in a graph, weights from HBM, one row): bf16
+// W, fp32 X 32768 x 2048 36.3 -> 22.0 (6.1 TB/s; 20.9 to 21.8 traced), 256 x 2048 6.3 -> 3.4; int8 W, fp32 X
+// 2048 x 4096 8.4 -> 4.9, 4096 x 2048 5.6 -> 4.8, 512 x 2048 5.6 -> 3.3, 8192 x 2048 7.1 -> 6.6; bf16 both 9216 x 2048
+// 11.3 -> 9.2, 2048 x 4096 7.5 -> 6.0. (A/B figures further down are of other cards: up to 10% off these.)
 #include "common.h"
 
 #include <type_traits>
@@ -96,7 +96,7 @@ __device__ __forceinline__ void gv_x(const uint16_t* p, float (&f)[V]) {
 // norms the rows for itself, into LDS: x and the norm weight are requested ahead of the wave's first
 // weights, so the norm runs while those are on their way from HBM. That costs 12 KB of L2 reads per 8
 // rows and takes out a launch that only moved 12 KB (4.0 to 4.4 us of a decode layer's chain; a 4-layer
-// stack's 16-token generation 2827 -> 2696 us, 2430 with KS).
+// stack's 16-token generation 2827 -> 2696 us, 2430 to 2470 with KS).
 template <typename TW, typename TX, int R, int MX, int PD, int NV = 0, int KS = 1>
 __global__ void __launch_bounds__(NV ? WAVE * GN_WAVES : 256) gemv_kernel(const GemvArgs ga) {
     constexpr int V = GvW<TW>::kVals, PIECE = V * WAVE, WAVES = NV ? GN_WAVES : 4;
@@ -327,8 +327,8 @@ bool gemv_norm_fits(const float* x, const uint16_t* nw, int M, int K) {
 
 template <int MX>
 static int gemv_norm_run(const GemvArgs& ga, hipStream_t st) {
-    // 8 rows per workgroup (two groups of four waves); measured on a generation of 16 tokens of a 4-layer
-    // stack at one / two rows: 2430 / 2655 us, with 16 rows (R = 2 over whole rows) 2515 / 2718, with
+    // 8 rows per workgroup (two groups of four waves); measured on one card on a generation of 16 tokens of a
+    // 4-layer stack at one / two rows: 2430 / 2655 us, with 16 rows (R = 2 over whole rows) 2515 / 2718, with
     // 4 rows and 4 waves 2436 / 2664, with 4 rows and 8 waves 2504 / 2802, with 16 waves 2585 / 2824
     if (ga.K <= 2048) return launch_gv<uint16_t, uint16_t, 4, MX, 1, 1, 4>(ga, st);
     if (ga.K <= 4096) return launch_gv<uint16_t, uint16_t, 4, MX, 2, 2, 4>(ga, st);

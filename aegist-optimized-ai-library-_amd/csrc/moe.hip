@@ -626,8 +626,8 @@ __global__ void __launch_bounds__(256, 2) moe_down_kernel(const MoeTile* __restr
 //     applied by one mixed-precision FMA per value with the fp16 scale as it stands;
 //   - column tiles without picks: NT = 1 .. 4 by the tile's count.
 // The codes stay two groups ahead over an LDS-only barrier per pair of groups.
-// Measured, batch 2048 (gate / up + down, profiled): 331 + 205 us before, 265 + 175 us now; with neither
-// codes, activations nor LDS reads in the loop the whole op still takes 380 of its 415 us: the products
+// Measured, batch 2048 of 256 experts (gate / up + down, traced): 331 + 205 us before, 259 + 179 us now (over the
+// benchmark's ring of layers, whose scales and mins are all alike, 230 + 159); with neither codes, activations nor LDS reads in the loop the whole op still takes 380 of its 415 us: the products
 // and the vector work of the two waves of a SIMD overlap poorly (28% and 25% busy), and a workgroup's
 // start is 8 us of its 40 (down) to 100 (gate / up).
 constexpr int NWB = 8;         // waves per big workgroup (one workgroup per CU)

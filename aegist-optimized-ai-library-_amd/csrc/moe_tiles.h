@@ -24,12 +24,12 @@ constexpr int kMoeCus = 256;   // such workgroups on the chip at once (one per C
 // Picks per prefill tile of moe.hip for T tokens with K of E experts each (D x I): 16, 32, 48 or 64, or 0
 // for the tiles of at most 32 picks on 64-row workgroups. A prefill tile reads and converts its codes
 // once for all its picks, but its workgroups are large and walk all of a row's groups one after the other
-// (45 to 75 us a round at D = 2048): they pay where they fill the chip. What fills it is counted for
+// (60 to 80 us a round of both projections at D = 2048): they pay where they fill the chip. What fills it is counted for
 // experts that are drawn alike. Measured (us, 64-row workgroups, then prefill tiles of 64; D x I):
 //   few experts, 2048 x 512, 9 tokens with 2 of 8 39.7, 68.7; other widths at decode batches, 2048 x 768, 1
 //   token with 8 of 256 34.7, 70.0; 16 tokens 129, 148; 1536 x 768, 4 tokens with 2 of 8 34.4, 66.1
 //   2048 x 512, 128 tokens with 8 of 256 231, 182, 2048 tokens 698, 418; 1024 x 256, 64 tokens 88.3, 66.9
-// Over 1437 batches of 1 to 2048 tokens, 4 to 512 experts, D 512 to 2048, I 128 to 1536 the rule's choice is
+// Over 1428 batches of 1 to 2048 tokens, 4 to 512 experts, D 512 to 2048, I 128 to 1536 the rule's choice is
 // 1.2% above the fastest of the five on average (I up to 2 D; experts three and more times as wide as a model
 // of 512 or less have too few rows in the down projection for any of them: 1.03 to 1.3 of the time
 // that 128-row workgroups took).
@@ -56,7 +56,7 @@ inline int moe_tile_picks(int T, int K, int E, int D, int I) {
     // 2048 x 768: 66 us, prefill tiles 86)
     if (mean >= 20 && mean <= 28 && workgroups(64) < kMoeCus / 2) return 0;
     // the smallest tiles that the chip takes in one round (2048 x 1408, 2 of 8 experts, 512 tokens: 32 picks
-    // 108 us, 64 143); past that the least code traffic
+    // 111 us, 64 143); past that the least code traffic
     for (int cap = 16; cap < 64; cap += 16)
         if (workgroups(cap) <= kMoeCus) return cap;
     return 64;

@@ -8,9 +8,10 @@
 // This file picks the kernel by size and holds the weight stream of decode batches. One or two rows
 // run in gemv.hip, the rest up to a few thousand in gemm_mid.hip, the largest in gemm.hip.
 //
-// int8 and bf16 weights are exact in bf16. An fp32 X is split into bf16 hi + lo
-// (x = hi + lo + O(2^-17 |x|)) and both halves go through the MFMA, so the result matches an
-// fp32 dot product to ~1e-5 relative; a bf16 X needs only the hi half.
+// int8 and bf16 weights are exact in bf16. From three rows on an fp32 X is split into bf16 hi + lo (hi
+// truncated, lo rounded: x = hi + lo to 2^-16 |x|) and both parts go through the MFMA, so the result matches
+// an fp32 dot product to ~1e-5 relative; a bf16 X needs only the hi part. One and two rows are fp32
+// products on the VALU.
 #include "common.h"
 
 #include <algorithm>
@@ -66,7 +67,7 @@ struct ProjSegs {
 // ---------------------------------------------------------------------------------------------
 // Decode-size bf16 projections (M <= 16) with W staged through LDS. Lanes that hold (row, run)
 // fragments straight from global memory read 16 rows x 64 or 128 bytes per instruction, and the
-// DRAM side serves that at ~half the rate of contiguous reads (same box: a read-only kernel
+// DRAM side serves that at ~half the rate of contiguous reads (same card: a read-only kernel
 // with that pattern 51% of HBM on 50 MB, 1 KB-contiguous reads 67%). Here every load
 // instruction is a direct global -> LDS copy of 1 KB of one pair of W rows (512 bytes each) and
 // the MFMA A operands are read back from LDS. Per workgroup: 16 NW rows of W (16 per wave, so

@@ -240,9 +240,8 @@ int aegist_attention_core(const float* q, const uint16_t* kc, const uint16_t* vc
  * (HybridBlock.forward, aegist/hybrid.py:812-843; HybridEngine::forward_chunk / mixer,
  * aegist_rs/src/hybrid.rs:760-861). The stack owns every layer's recurrent state, conv state
  * and bf16 KV cache (HybridCache, hybrid.py:171-260; engine buffers hybrid.rs:607-629); all
- * sequences of a batch share one length. Projections: bf16 operands, fp32 accumulation; up to
- * 64 rows on this library's weight-streaming kernel (aegist_linear), more on its tiled MFMA
- * GEMM; every op runs on this library's kernels. Weights are caller-owned bf16,
+ * sequences of a batch share one length. Projections: bf16 operands, fp32 accumulation, on the
+ * kernel of their size as in aegist_linear_multi; every op runs on this library's kernels. Weights are caller-owned bf16,
  * row-major [out, in] as torch nn.Linear stores them.
  * ------------------------------------------------------------------------------------- */
 #define AEGIST_MAX_LAYERS 64
@@ -358,12 +357,9 @@ int aegist_gemv_bf16(const float* x, const uint16_t* W, float* y, int N, int K, 
 int aegist_gemm_i8(const float* X, const int8_t* W, const uint16_t* scale, float* Y, int M, int N, int K,
                    int accumulate, void* stream);
 /* Strided form of the three above: X dtype AEGIST_F32 | AEGIST_BF16 (row stride ldx elements),
- * W dtype AEGIST_I8 | AEGIST_BF16, scale NULL = 1, Y fp32 with row stride ldy. 17..64 rows of
- * bf16 X against one bf16 weight of under 6144 rows (K % 256 == 0, N % 4 == 0, no scale) split
- * K when the calling thread has bound a workspace (aegist_bind_workspace) of at least
- * splits * M * N * 4 bytes (splits <= 256 * 32 / N, at most K / 256): fp32 partials, added in
- * slice order by a second launch (deterministic; the same result to fp32 rounding as the
- * unsplit kernel, which runs otherwise). */
+ * W dtype AEGIST_I8 | AEGIST_BF16, scale NULL = 1, Y fp32 with row stride ldy. K % 16 == 0, rows of
+ * X and W 16-byte aligned. Deterministic, needs no workspace and uses none that is bound; operands
+ * of 2 GiB and more are cut into blocks of rows, a launch each. */
 int aegist_linear(const void* X, int x_dtype, long long ldx, const void* W, int w_dtype, const uint16_t* scale,
                   float* Y, long long ldy, int M, int N, int K, int accumulate, void* stream);
 /* Grouped form: n (1..4) weight matrices W[i] [N[i], K] of one dtype that share the input X
