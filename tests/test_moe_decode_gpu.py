@@ -97,7 +97,7 @@ def test_more_picks_of_one_expert_than_tile_products_fit_32_bits(dev):
 
 
 @pytest.mark.parametrize("T,D,I,E,K", [(70, 384, 256, 256, 8), (96, 256, 256, 8, 2), (128, 384, 256, 8, 2), (2048, 256, 256, 4, 2),
-                                       (5000, 256, 256, 8, 2), (9000, 256, 256, 8, 2), (1, 256, 768, 64, 8), (9, 512, 512, 8, 2),
+                                       (5000, 256, 256, 8, 2), (8000, 256, 256, 8, 2), (1, 256, 768, 64, 8), (9, 512, 512, 8, 2),
                                        (100, 256, 192, 8, 4)])
 def test_moe_tile_sizes_match_oracle(dev, T, D, I, E, K):
     """Every size of tile the rule picks (test_moe_tiles.py has it for these batches): prefill tiles of up to

@@ -64,7 +64,7 @@ def test_tile_rule_counts_the_longer_rows_workgroups(tiles):
 # the batches of test_moe_decode_gpu.py's sizes of tiles
 @pytest.mark.parametrize("T,D,I,E,K,picks", [(70, 384, 256, 256, 8, 64), (96, 256, 256, 8, 2, 0), (128, 384, 256, 8, 2, 16),
                                              (1024, 256, 256, 4, 2, 16), (2048, 256, 256, 4, 2, 32),
-                                             (5000, 256, 256, 8, 2, 48), (9000, 256, 256, 8, 2, 64),
+                                             (5000, 256, 256, 8, 2, 48), (8000, 256, 256, 8, 2, 64),
                                              (1, 256, 768, 64, 8, 0), (9, 512, 512, 8, 2, 0)])
 def test_tile_rule_of_the_gpu_test(tiles, T, D, I, E, K, picks):
     assert tiles.tile_picks(T, K, E, D, I) == picks
@@ -80,3 +80,8 @@ def test_workspace_of_more_tokens_serves_fewer(K, D, I, E):
     sizes = [size(t, K, D, I, E) for t in ts]
     for t, a, b in zip(ts, sizes, sizes[1:]):
         assert a <= b, (t, a, b)
+
+
+def test_tile_rule_does_not_open_a_round_for_a_few_workgroups(tiles):
+    """272 workgroups of 64 picks are two rounds of 256, which 48 picks fill better."""
+    assert tiles.tile_picks(2048, 2, 8, 896, 896) == 48
