@@ -3,16 +3,16 @@
 // o = S^T q (hybrid.py:318-324 looped; the engine's delta_scan, hybrid.cu:240-300).
 //
 // The columns of S evolve independently (column j only needs k, q, v_j), so the work is split
-// by column block: one wave64 per (sequence, value head, 8-column block) holds 128 x 8 of
-// the state in VGPRs (16 rows x 1 column per lane) for the whole sequence. B = 1 with 32
-// value heads gives 512 waves instead of the 32 workgroups of a head-per-block scan.
+// by column block: one wave64 per (sequence, value head, block of 8 or 16 columns) holds 128 x 8 or
+// 128 x 16 of the state in VGPRs (16 or 32 rows x 1 column per lane) for the whole sequence. B = 1 with 32
+// value heads gives 512 or 256 waves instead of the 32 workgroups of a head-per-block scan.
 //
 // Latency-bound: one wave's chain per token. Both column sums are taken over the old state (S^T k and
 // S^T q), so the output does not wait for the update: o = e^g S^T q + (k . q) delta. Everything that
 // does not depend on the state runs a token ahead, beside the sums: the norms (DPP sums instead of
 // LDS permutes), q and k staged in the wave's own LDS (no workgroup barrier, which also waited for the
-// prefetch of the next token's inputs), the loads two tokens ahead. 37 tokens, 32 heads, batch 1: 44 -> 30 us
-// (in the layer stack 36), 256 tokens 305 -> 213.
+// prefetch of the next token's inputs), the loads two tokens ahead. In the layer stack 37 tokens, 32 heads, batch 1:
+// 44 -> 36 us.
 #include "common.h"
 
 using namespace aegist;
@@ -20,20 +20,19 @@ using namespace aegist;
 namespace {
 
 constexpr int D = 128;
-constexpr int CB = 8;                 // columns per workgroup (one wave)
-constexpr int RPL = D * CB / WAVE;     // state rows per lane
 
 struct SeqArgs {
     long long sb_qk, st_qk, sh_qk, sb_v, st_v, sh_v, sb_o, st_o, sh_o;
     long long sb_g, st_g;  // g / beta strides by sequence and token (value head contiguous)
 };
 
-template <typename Tin, typename Tout>
+template <typename Tin, typename Tout, int CB>  // CB: columns per workgroup (one wave), 8 or 16
 __global__ void __launch_bounds__(64) delta_recurrent_kernel(const Tin* __restrict__ q, const Tin* __restrict__ k,
                                                              const Tin* __restrict__ v, const float* __restrict__ g,
                                                              const float* __restrict__ beta, float* __restrict__ state,
                                                              Tout* __restrict__ out, SeqArgs a, int T, int HK, int HV,
                                                              int normalize, float qscale, float eps) {
+    constexpr int RPL = D * CB / WAVE;  // state rows per lane
     __shared__ __attribute__((aligned(16))) float sk[2][D], sq[2][D];  // wave-private, two tokens
     const int cb = blockIdx.x, hv = blockIdx.y, b = blockIdx.z, lane = threadIdx.x;
     const int c = lane % CB, rg = lane / CB;  // column within block, row group (RPL rows)
@@ -113,8 +112,10 @@ __global__ void __launch_bounds__(64) delta_recurrent_kernel(const Tin* __restri
             pq[r & 1] = fmaf(s[r], qr[r], pq[r & 1]);
         }
         float SK = pk[0] + pk[1], SQ = pq[0] + pq[1];
-        SK += lane_xor<8>(SK);
-        SQ += lane_xor<8>(SQ);
+        if constexpr (CB == 8) {
+            SK += lane_xor<8>(SK);
+            SQ += lane_xor<8>(SQ);
+        }
         SK = pair_sum32(pair_sum16(SK));
         SQ = pair_sum32(pair_sum16(SQ));
         const float delta = (cv - cd * SK) * cbt;
@@ -128,12 +129,24 @@ __global__ void __launch_bounds__(64) delta_recurrent_kernel(const Tin* __restri
     }
 }
 
+// Blocks of 8 columns shorten a token's chain, but read and write the state in pieces of 32 bytes instead of 64
+// and stage q and k twice as often: they pay for few heads over many tokens. Measured (fp32, us, 16 and 8
+// columns): 32 heads 1 token 6.0, 7.4; 12 18.1, 18.5; 16 22.6, 21.9; 63 66, 61; 64 heads 24 32.8, 34.8; 63 69, 65;
+// 128 heads 37 49.0, 48.8; 63 73.7, 72.2; 256 heads 63 83, 102; 2048 heads 1 token 65.8, 132. (The first form, 16 columns
+// with two barriers a token, took 6.2, 20.9, 25.8, 78; 38, 82; 55, 86; 89 and 65.5 us.)
+constexpr bool narrow_columns(long long heads, int T) { return heads <= 128 && 2LL * T >= heads; }
+static_assert(!narrow_columns(64 * 32, 1) && !narrow_columns(32, 1) && narrow_columns(32, 37) && !narrow_columns(256, 200),
+              "a step of many heads takes 16 columns");
+
 template <typename Tin, typename Tout>
 int launch2(const void* q, const void* k, const void* v, const float* g, const float* beta, float* state, void* out,
             const SeqArgs& a, int B, int T, int HK, int HV, int normalize, float qscale, float eps, hipStream_t st) {
-    dim3 grid(D / CB, HV, B);
-    delta_recurrent_kernel<Tin, Tout><<<grid, 64, 0, st>>>((const Tin*)q, (const Tin*)k, (const Tin*)v, g, beta, state,
-                                                           (Tout*)out, a, T, HK, HV, normalize, qscale, eps);
+    if (narrow_columns((long long)B * HV, T))
+        delta_recurrent_kernel<Tin, Tout, 8><<<dim3(D / 8, HV, B), 64, 0, st>>>(
+            (const Tin*)q, (const Tin*)k, (const Tin*)v, g, beta, state, (Tout*)out, a, T, HK, HV, normalize, qscale, eps);
+    else
+        delta_recurrent_kernel<Tin, Tout, 16><<<dim3(D / 16, HV, B), 64, 0, st>>>(
+            (const Tin*)q, (const Tin*)k, (const Tin*)v, g, beta, state, (Tout*)out, a, T, HK, HV, normalize, qscale, eps);
     return after_launch("delta_recurrent");
 }
 
@@ -199,10 +212,8 @@ extern "C" int aegist_delta_scan_ws(const float* y, const float* gb, float* stat
     // g and beta are interleaved per token in gb: present them through the strided kernel
     // by pointing g at gb and beta at gb + HV with a token stride of 2*HV.
     SeqArgs a{0, C, D, 0, C, D, 0, (long long)HV * D, D, 0, 2 * HV};
-    dim3 grid(D / CB, HV, 1);
-    delta_recurrent_kernel<float, float><<<grid, 64, 0, st>>>(y, y + (size_t)HK * D, y + (size_t)2 * HK * D, gb,
-                                                              gb + HV, state, o, a, T, HK, HV, 0, 1.f, 0.f);
-    return after_launch("delta_scan");
+    return launch2<float, float>(y, y + (size_t)HK * D, y + (size_t)2 * HK * D, gb, gb + HV, state, o, a, 1, T, HK, HV, 0,
+                                 1.f, 0.f, st);
 }
 
 // The reference signature (no workspace argument): T >= 64 takes the workspace bound to this

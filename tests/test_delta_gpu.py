@@ -122,6 +122,21 @@ def test_recurrent_with_state_and_fp32(dev, T):
     assert rel_err(o, o_ref) < DELTA_TOL and rel_err(S, S_ref) < DELTA_TOL
 
 
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,HK,HV,T", [(1, 2, 4, 1), (1, 2, 4, 2), (1, 4, 32, 15), (1, 4, 32, 16), (2, 4, 32, 31), (2, 4, 32, 32),
+                                       (16, 8, 8, 63), (16, 8, 8, 64), (43, 3, 3, 70), (64, 2, 4, 1)])
+def test_recurrent_column_blocks(dev, B, HK, HV, T, dt):
+    """Both widths of the column blocks, on the two sides of the line between them (half as many tokens as
+    heads, up to 128 heads): 8 columns from there on."""
+    q, k, v, g, beta = (x.to(dt) if x.dtype == torch.bfloat16 else x for x in seq_inputs(B, HK, HV, T, seed=B + T))
+    S0 = torch.randn(B, HV, D, D, generator=_gen(3)) * 0.02
+    o_ref, S_ref = oracle_seq(q, k, v, g, beta, S0.clone(), chunked=False)
+    S = S0.to(dev)
+    o = ops.delta_rule_recurrent(q.to(dev), k.to(dev), v.to(dev), g.to(dev), beta.to(dev), S, normalize=True,
+                                 qscale=D ** -0.5)
+    assert rel_err(o, o_ref) < DELTA_TOL and rel_err(S, S_ref) < DELTA_TOL
+
+
 def test_delta_rule_step_mirror(dev):
     B, H = 3, 4
     g_ = _gen(7)
