@@ -313,7 +313,7 @@ __global__ void __launch_bounds__(256) delta_gates_kernel(const float* __restric
 // The same for D a multiple of 8 and 16-byte aligned rows: one wave per MT tokens and 4 outputs (beta's
 // and g's in separate waves), 16 bytes of weights and 32 of h per lane and piece of 512 values, the
 // sums over the lanes by halving exchanges. The wave-per-output form above read h once per output and
-// 2 bytes of weights per lane and load: 300 tokens x 2048 x 64 outputs 23.8 us, here 10.3; fp32
+// 2 bytes of weights per lane and load: 300 tokens x 2048 x 64 outputs 18.4 to 23.8 us, here 8.0; fp32
 // products as there.
 template <int MT>
 __global__ void __launch_bounds__(256) delta_gates_vec_kernel(const float* __restrict__ h, const uint16_t* __restrict__ wb,
@@ -381,10 +381,16 @@ extern "C" int aegist_delta_gates(const float* h, const uint16_t* wb, const uint
     AEG_REQUIRE(T >= 0 && D > 0 && HV > 0, "delta_gates: bad shape");
     if (T == 0) return 0;
     if (D % 8 == 0 && (uintptr_t)h % 16 == 0 && (uintptr_t)wb % 16 == 0 && (uintptr_t)wa % 16 == 0) {
-        // four tokens per wave once that leaves enough waves
+        // two tokens per wave once that leaves enough waves. Measured (us, one, two and four tokens a wave; the
+        // wave-per-output form): 2048 x 64 outputs 64 tokens 5.4, 6.7, 11.3; 7.8; 200 tokens (3200 waves of one)
+        // 7.4, 6.8, 10.7; 13.5; 1024 18.2, 14.4, 15.9; 92; 8192 x 64 outputs 160 (2560) 13.6, 12.3, 22.1; 80;
+        // 512 x 16 outputs 700 (2800) 4.7, 5.3, 7.1; 7.5; four for many of short rows: 512 x 96 outputs 1024 14.1, 12.0, 10.8
         const long long per = 2 * ((HV + 3) / 4);
-        if (T >= 64)
+        if (T * per >= 24576 && D <= 512)
             delta_gates_vec_kernel<4><<<(unsigned)(((T + 3) / 4 * per + 3) / 4), 256, 0, AEG_STREAM(stream)>>>(
+                h, wb, wa, a_log, dt_bias, gb, T, D, HV);
+        else if (T * per >= 3072)
+            delta_gates_vec_kernel<2><<<(unsigned)(((T + 1) / 2 * per + 3) / 4), 256, 0, AEG_STREAM(stream)>>>(
                 h, wb, wa, a_log, dt_bias, gb, T, D, HV);
         else
             delta_gates_vec_kernel<1><<<(unsigned)((T * per + 3) / 4), 256, 0, AEG_STREAM(stream)>>>(

@@ -1,6 +1,5 @@
 """The wide-load kernels of the small ops (csrc/mixer_small.hip) at the edges of their forms: gates with
-one token a wave below 64 tokens, four from there on, heads in groups of four, rows in pieces of 512
-values; norms whose row or head ends inside a thread's pieces; widths that are no multiple of eight or
+one token a wave, two from 3072 waves on, four from 24576 of short rows, heads in groups of four, rows in pieces of 512 values; norms whose row or head ends inside a thread's pieces; widths that are no multiple of eight or
 four take the narrow kernels."""
 import pytest
 import torch
@@ -10,8 +9,8 @@ from aegist_mixer import ops
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("T", [1, 3, 63, 64, 66, 129])
-@pytest.mark.parametrize("HV,D", [(1, 8), (3, 520), (6, 504), (32, 2048), (5, 12)])
+@pytest.mark.parametrize("T", [1, 3, 63, 64, 66, 129, 191, 192, 767, 769])
+@pytest.mark.parametrize("HV,D", [(1, 8), (3, 520), (6, 504), (32, 2048), (5, 12), (130, 512)])
 def test_gates_match_exact(dev, T, HV, D):
     g_ = torch.Generator().manual_seed(T * HV + D)
     h = torch.randn(T, D, generator=g_)
