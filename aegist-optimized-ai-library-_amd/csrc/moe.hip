@@ -92,6 +92,21 @@ __device__ __forceinline__ float wave_max_dpp(float v) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), WAVE - 1));
 }
 
+// The least value of the wave, in the same way.
+__device__ __forceinline__ int wave_min_dpp(int v) {
+    auto step = [](int x, auto ctrl, auto rows) {
+        return min(x, __builtin_amdgcn_update_dpp(x, x, decltype(ctrl)::value, decltype(rows)::value, 0xF, false));
+    };
+    using std::integral_constant;
+    v = step(v, integral_constant<int, 0x111>{}, integral_constant<int, 0xF>{});
+    v = step(v, integral_constant<int, 0x112>{}, integral_constant<int, 0xF>{});
+    v = step(v, integral_constant<int, 0x114>{}, integral_constant<int, 0xF>{});
+    v = step(v, integral_constant<int, 0x118>{}, integral_constant<int, 0xF>{});
+    v = step(v, integral_constant<int, 0x142>{}, integral_constant<int, 0xA>{});
+    v = step(v, integral_constant<int, 0x143>{}, integral_constant<int, 0xC>{});
+    return __builtin_amdgcn_readlane(v, WAVE - 1);
+}
+
 // ---------------------------------------------------------------------------------------------
 // Router top-K over precomputed logits [T, E] (the projection kernel computes h W^T): one wave
 // per token, lane holds the probabilities of experts lane + 64 i in registers; softmax in fp32;
@@ -124,14 +139,20 @@ __global__ void __launch_bounds__(256) router_topk_kernel(const float* __restric
     float myv = 0.f;  // lane k keeps pick k
     int mye = 0;
     for (int k = 0; k < K; k++) {
-        // the largest probability of the wave, then the lowest expert that has it (experts lane + 64 i:
-        // the first i with a holder, its lowest lane); NaN and taken entries never compare greater
+        // the largest probability of the wave, then the lowest expert that has it (experts lane + 64 i);
+        // NaN and taken entries never compare greater
         float lv = -1.f;
+        int li = 0x7fffffff, bi = 0x7fffffff;  // the lane's first holder of its largest
 #pragma unroll
-        for (int i = 0; i < NPER; i++) lv = p[i] > lv ? p[i] : lv;
+        for (int i = 0; i < NPER; i++) {
+            if (NPER > 4 && p[i] > lv) li = lane + WAVE * i;
+            lv = p[i] > lv ? p[i] : lv;
+        }
         const float bv = wave_max_dpp(lv);
-        int bi = 0x7fffffff;
-        if (bv > -1.f) {
+        if constexpr (NPER > 4) {
+            bi = wave_min_dpp(lv == bv && bv > -1.f ? li : 0x7fffffff);
+        } else if (bv > -1.f) {
+            // few registers: the first i with a holder, its lowest lane
 #pragma unroll
             for (int i = 0; i < NPER; i++) {
                 const unsigned long long m = __ballot(p[i] == bv);

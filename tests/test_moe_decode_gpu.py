@@ -37,7 +37,7 @@ def test_moe_decode_matches_oracle(dev, T, D, I, E, K, hot, bad):
     assert err < 5e-5
 
 
-@pytest.mark.parametrize("T,E,K", [(3, 16, 4), (2, 64, 8), (5, 65, 16), (4, 1000, 8), (2, 2000, 3)])
+@pytest.mark.parametrize("T,E,K", [(3, 16, 4), (2, 64, 8), (5, 65, 16), (4, 1000, 8), (2, 2000, 3), (2, 4096, 16)])
 def test_router_rounds_take_the_lowest_of_equals(dev, T, E, K):
     """Equal probabilities in lanes and registers of every distance: groups of experts share one weight
     row, so the K picks are the lowest ids of the best groups, in order."""
