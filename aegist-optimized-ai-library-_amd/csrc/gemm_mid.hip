@@ -265,8 +265,13 @@ __global__ void __launch_bounds__(64 * NWN * KG) gemm_mid_kernel(const MidArgs g
         }
         lds_barrier();
     };
-    // whole rounds of PD steps: steps past K are products of zeros
-    for (int t = 0; t < nt; t += PD) {
+    // Rounds of PD steps; steps past K are products of zeros. A step of 4 and 8 K groups is 256 and 512 k, so there
+    // an odd one out has its own code (1536 = 3 steps of 8 groups: 33 rows of 5120 x 1536 int8 12.4 -> 10.7 us);
+    // in the forms of fewer groups that copy costs more than the step (555 x 4096 x 2048 bf16 32.5, 33.3 with it)
+    constexpr bool kTail = KG >= 4;
+    static_assert(PD == 2, "the step left over is slot 0's");
+    int t = 0;
+    for (; t + (kTail ? PD : 1) <= nt; t += PD) {
 #pragma unroll
         for (int d = 0; d < PD; d++) step(t + d, d);
         if constexpr (kFlush > 0) {
@@ -280,6 +285,9 @@ __global__ void __launch_bounds__(64 * NWN * KG) gemm_mid_kernel(const MidArgs g
                     }
             }
         }
+    }
+    if constexpr (kTail) {
+        if (t < nt) step(t, 0);
     }
 #pragma unroll
     for (int rt = 0; rt < RT; rt++)

@@ -43,6 +43,16 @@ def test_mid_batch_matches_exact(dev, M, N, K, w8, xf):
     _check(out, y0, x, w, s, K)
 
 
+@pytest.mark.parametrize("w8,xf", [(True, True), (False, False), (False, True), (True, False)])
+@pytest.mark.parametrize("M,N,K", [(33, 5120, 1536), (130, 2100, 1040), (600, 4100, 1552)])
+def test_odd_steps(dev, M, N, K, w8, xf):
+    print(f"odd M={M} N={N} K={K} w8={w8} xf={xf}", flush=True)
+    x, w, s = _operands(M, N, K, w8, xf, M + N + K, dev)
+    _check(ops.linear(x, w, s), None, x, w, s, K)
+    y0 = torch.randn(M, N, generator=torch.Generator().manual_seed(1)).to(dev)
+    _check(ops.linear(x, w, s, out=y0.clone(), accumulate=True), y0, x, w, s, K)
+
+
 @pytest.mark.parametrize("w8,xf", [(True, True), (False, False)])
 def test_mid_batch_segments_and_strides(dev, w8, xf):
     """Four weights in one launch (sizes that end inside a tile), X rows inside wider rows and
