@@ -360,7 +360,8 @@ constexpr MidForm kFormsF32[] = {{1, 2, 1, 8, 0.156f}, {1, 2, 2, 8, 0.18f}, {2, 
 constexpr MidForm kFormsBf16[] = {{1, 2, 1, 8, 0.100f}, {1, 2, 2, 8, 0.157f}, {1, 4, 2, 4, 0.205f}, {1, 4, 4, 2, 0.312f},
                                   {2, 4, 4, 2, 0.548f}, {2, 8, 4, 1, 0.90f},  {2, 8, 8, 1, 1.21f}};
 constexpr int kNF32 = 8, kNBf16 = 7, kForms = 8;  // entries of the two tables; codes of the sized forms
-// Up to 16 rows (one 16-row tile of X), after the sized forms; chosen by rows of W and K, see small_form
+// 16 rows of X a tile, after the sized forms: up to 16 rows chosen by rows of W and K, see small_form; past
+// them where all tiles run in one round, see one_round_form
 constexpr MidForm kFormsSmall[] = {{1, 1, 1, 8, 0.f}, {1, 1, 1, 4, 0.f}, {1, 1, 2, 4, 0.f}, {2, 1, 2, 4, 0.f}};
 constexpr int kSmall = 4;
 
@@ -369,11 +370,13 @@ constexpr int kSmall = 4;
 //   2048 x 4096 13.4 -> 9.3, 10.3 -> 7.9   512 x 2048 8.0 -> 5.5, 6.1 -> 4.9
 // 4 K groups instead of 8 where the rows alone give the chip enough waves or K is short; wider tiles
 // (X staged for more rows) from 6144 rows of W for fp32 X, whose stage costs most, and where even
-// these are more than two workgroups per CU (bf16 W, fp32 X 32768 x 2048: 36.2 -> 33.0).
+// these are more than two workgroups per CU (bf16 W, fp32 X 32768 x 2048: 36.2 -> 33.0). Past 4096 rows, where
+// tiles of 16 rows of W open a second round, the next wider ones (3 rows of 5120 x 1536: int8 9.0 -> 6.6,
+// bf16 8.2 -> 7.3; row-tile kernel 8.7, 7.3).
 int small_form(bool f32, long long rows, int K) {
     if (rows > 16384) return kForms + 3;
-    if (f32 ? rows >= 6144 : rows > 8192) return kForms + 2;
-    if (K <= 1024 || (!f32 && rows >= 6144)) return kForms + 1;
+    if (f32 ? rows > 4096 : rows > 8192) return kForms + 2;
+    if (K <= 1024 || rows > 4096) return kForms + 1;
     return kForms;
 }
 // the 256 x 256 tiles of gemm.hip, in the same unit: int8 W with fp32 X, bf16 W with bf16 X
@@ -383,6 +386,22 @@ long long mid_tiles(const MidForm& f, const MidArgs& ga) {
     long long t = 0;
     for (int i = 0; i < ga.nseg; i++) t += (ga.seg[i].N + 16 * f.rt * f.nwn - 1) / (16 * f.rt * f.nwn);
     return t * ((ga.M + 16 * f.mt - 1) / (16 * f.mt));
+}
+
+// The 16-row form for more than 16 rows of X, or -1. A workgroup of 32 and more rows stages that much X before
+// its first product and takes most of a CU's LDS; where the chip runs all tiles of 16 rows in one round, they are
+// done sooner, and short rows of K were slower on the larger tiles than on the row-tile kernel before those.
+// Measured (us; row-tile kernel, sized form, here):
+//   int8 W, fp32 X   17 x 2048 x 512 4.8, 6.3, 4.2   64 x 2048 x 512 5.6, 6.4, 4.4   17 x 1000 x 1040 5.5, 7.9, 5.3
+//   bf16 W, bf16 X   17 x 2048 x 512 4.4, 5.0, 3.6   17 x 1000 x 1040 4.4, 6.1, 4.5   17 x 1024 x 8192 -, 15.0, 12.5
+// Over 968 sizes this form took 0.84 of the sized one's time on average, 1.08 at most. The limits on K: past them 4
+// K groups walk too long (bf16 X 33 x 2048 x 4096 10.1 sized, 12.2 here; bf16 W, fp32 X 100 x 1536 x 6144 23.6, 27.4).
+int one_round_form(bool f32, const MidArgs& ga) {
+    auto one_round = [&](int i) { return mid_tiles(kFormsSmall[i], ga) <= 256; };
+    if (one_round(0)) return kForms + (ga.K <= 1024 ? 1 : 0);
+    if ((f32 || ga.K < 1024) && one_round(2)) return kForms + 2;
+    if (f32 && ga.K <= 1024 && one_round(3)) return kForms + 3;
+    return -1;
 }
 
 template <typename TW, typename TX, int RT, int MT, int NWN, int KG, int PD>
@@ -442,6 +461,7 @@ int gemm_mid_form(int x_dtype, int nseg, const int* N, int M, int K, bool tile25
     MidArgs ga{};
     ga.nseg = nseg;
     ga.M = M;
+    ga.K = K;
     const long long tm = (M + 255) / 256;
     auto rounds256 = [&](long long n) { return ((n + 255) / 256 * tm + 255) / 256; };
     long long rows = 0, r256 = 0;
@@ -450,6 +470,8 @@ int gemm_mid_form(int x_dtype, int nseg, const int* N, int M, int K, bool tile25
         rows += N[i];
         r256 += rounds256(N[i]);
     }
+    const int one = one_round_form(x_dtype == AEGIST_F32, ga);
+    if (one >= 0) return one;
     if (stacked) r256 = rounds256(rows);
     const MidForm* forms = x_dtype == AEGIST_F32 ? kFormsF32 : kFormsBf16;
     int best = -1;
