@@ -345,18 +345,20 @@ __global__ void __launch_bounds__(64 * NWN * KG) gemm_mid_kernel(const MidArgs g
     }
 }
 
-// One form of the kernel and its cost: us of one 64-k step of a round of workgroups (one per CU), the
-// median over a sweep of M 20 .. 1500 and N x K 512 .. 8192 x 2048 and 2048 x 4096 on one card (`base`: the
-// part that does not grow with the rounds, for the form without K groups, whose workgroups share a
-// CU); the estimate base + ceil(tiles / 256) x cost picked the fastest form or one within 10% of it
-// at 52 of the 56 swept sizes (at worst 15% slower, between neighbouring tile sizes).
+// One form of the kernel and its cost: us of one 64-k step of a round of workgroups (one per CU; `base`: the
+// part that does not grow with the rounds, for the form without K groups, whose workgroups share a CU), the fastest
+// estimate base + ceil(tiles / 256) x cost is taken. Bf16 X: the median over a sweep of M 20 .. 1500 and N x K 512 ..
+// 8192 x 2048 and 2048 x 4096. fp32 X: fitted to 236 sizes of M 17 .. 2048, N x K 512 .. 12352 x 256 .. 8192
+// (int8 and bf16 W alike), where the choice is 1.5% above the fastest form on average (2.8% with a first fit to few
+// rounds, which sent 2048 x 5120 x 1536 int8 to the form without K groups: 110 us, 256 x 256 tiles 97, here 80) and 16
+// sizes are more than 5% above it, bf16 W with 420 to 1500 rows mostly (at most 1.38).
 struct MidForm {
     int rt, mt, nwn, kg;
     float cost, base = 0.f;
 };
 // fp32 X: staging and splitting X is the larger part of a step
-constexpr MidForm kFormsF32[] = {{1, 2, 1, 8, 0.156f}, {1, 2, 2, 8, 0.18f}, {2, 2, 2, 8, 0.265f}, {2, 2, 4, 4, 0.375f},
-                                 {2, 2, 4, 1, 0.28f, 0.15f}, {2, 4, 4, 2, 0.60f}, {2, 4, 8, 1, 1.10f}, {4, 4, 8, 1, 1.70f}};
+constexpr MidForm kFormsF32[] = {{1, 2, 1, 8, 0.156f}, {1, 2, 2, 8, 0.18f}, {2, 2, 2, 8, 0.265f}, {2, 2, 4, 4, 0.42f},
+                                 {2, 2, 4, 1, 0.33f, 0.15f}, {2, 4, 4, 2, 0.70f}, {2, 4, 8, 1, 1.15f}, {4, 4, 8, 1, 1.80f}};
 constexpr MidForm kFormsBf16[] = {{1, 2, 1, 8, 0.100f}, {1, 2, 2, 8, 0.157f}, {1, 4, 2, 4, 0.205f}, {1, 4, 4, 2, 0.312f},
                                   {2, 4, 4, 2, 0.548f}, {2, 8, 4, 1, 0.90f},  {2, 8, 8, 1, 1.21f}};
 constexpr int kNF32 = 8, kNBf16 = 7, kForms = 8;  // entries of the two tables; codes of the sized forms

@@ -38,3 +38,9 @@ def test_tiles_of_16_rows_where_they_run_in_one_round(x, N, M, K, code):
     larger tiles than on the kernel before those."""
     form = _form(x, N, M, K, False)
     assert form < 8 if code is None else form == code
+
+
+@pytest.mark.parametrize("M,N,K", [(2048, 5120, 1536), (2048, 5120, 2048), (1500, 4096, 1536)])
+def test_many_rounds_are_not_left_to_the_form_without_k_groups(M, N, K):
+    """Form 4 of the fp32 table: 110 us at the first size, the 256 x 256 tiles before it 97, form 6 80."""
+    assert _form(F32, (N,), M, K, False) != 4
