@@ -365,16 +365,14 @@ constexpr int kNF32 = 8, kNBf16 = 7, kForms = 8;  // entries of the two tables; 
 // 16 rows of X a tile, after the sized forms: up to 16 rows chosen by rows of W and K, see small_form; past
 // them where all tiles run in one round, see one_round_form
 constexpr MidForm kFormsSmall[] = {{1, 1, 1, 8, 0.f}, {1, 1, 1, 4, 0.f}, {1, 1, 2, 4, 0.f}, {2, 1, 2, 4, 0.f}};
-constexpr int kSmall = 4;
 
 // Measured (us, 16 rows, weights from HBM; fp32 X with int8 W, then bf16 both), row-tile kernel -> here:
 //   8192 x 2048 9.5 -> 7.6, 10.1 -> 8.8    4096 x 2048 8.4 -> 7.0, 7.0 -> 6.1
 //   2048 x 4096 13.4 -> 9.3, 10.3 -> 7.9   512 x 2048 8.0 -> 5.5, 6.1 -> 4.9
-// 4 K groups instead of 8 where the rows alone give the chip enough waves or K is short; wider tiles
-// (X staged for more rows) from 6144 rows of W for fp32 X, whose stage costs most, and where even
-// these are more than two workgroups per CU (bf16 W, fp32 X 32768 x 2048: 36.2 -> 33.0). Past 4096 rows, where
-// tiles of 16 rows of W open a second round, the next wider ones (3 rows of 5120 x 1536: int8 9.0 -> 6.6,
-// bf16 8.2 -> 7.3; row-tile kernel 8.7, 7.3).
+// 4 K groups instead of 8 where K is short and past 4096 rows of W, where tiles of 16 of them open a second
+// round: for fp32 X, whose stage costs most, with tiles of 32 (3 rows of 5120 x 1536: int8, fp32 X 9.0 -> 6.6, bf16
+// both 8.2 -> 7.3; row-tile kernel 8.7, 7.3). Tiles of 32 and 64 rows where even these are more than two
+// workgroups per CU (bf16 W, fp32 X 32768 x 2048: 36.2 -> 33.0).
 int small_form(bool f32, long long rows, int K) {
     if (rows > 16384) return kForms + 3;
     if (f32 ? rows > 4096 : rows > 8192) return kForms + 2;

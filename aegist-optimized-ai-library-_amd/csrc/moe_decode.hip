@@ -285,7 +285,9 @@ namespace aegist {
 
 // Whether the decode kernels take the batch: up to 512 picks, at most two per expert on average
 // (beyond that the MFMA tiles of moe.hip read each expert once for more picks), row lengths
-// of whole rounds of 4 chunks of 128 codes.
+// of whole rounds of 4 chunks of 128 codes. The host does not know which experts were picked: where all tokens
+// pick the same ones, an expert's picks go four to a workgroup, and the call takes about as long as for experts
+// drawn alike (2048 x 512, 8 of 256 experts, 64 tokens: 134 and 124 us; the tiles of moe.hip 61 and 204).
 bool moe_decode_fits(int T, int D, int I, int E, int K) {
     const long long N = (long long)T * K;
     return N <= kMaxPicks && N <= 2LL * E && row_fits(D) && row_fits(I);
