@@ -373,10 +373,13 @@ constexpr MidForm kFormsSmall[] = {{1, 1, 1, 8, 0.f}, {1, 1, 1, 4, 0.f}, {1, 1, 
 // round: for fp32 X, whose stage costs most, with tiles of 32 (3 rows of 5120 x 1536: int8, fp32 X 9.0 -> 6.6, bf16
 // both 8.2 -> 7.3; row-tile kernel 8.7, 7.3). Tiles of 32 and 64 rows where even these are more than two
 // workgroups per CU (bf16 W, fp32 X 32768 x 2048: 36.2 -> 33.0).
+// K is short up to 1280: 5 steps of 4 K groups against 3 of 8 (us, 8 and 4 groups, 16 x 1000 x 1040 bf16 W, fp32 X 5.4, 5.1,
+// bf16 both 4.4, 4.2; 3 x 2048 x 1024 5.3, 5.4; 16 x 1024 x 1536 5.4, 5.7)
+constexpr int kShortK = 1280;
 int small_form(bool f32, long long rows, int K) {
     if (rows > 16384) return kForms + 3;
     if (f32 ? rows > 4096 : rows > 8192) return kForms + 2;
-    if (K <= 1024 || rows > 4096) return kForms + 1;
+    if (K <= kShortK || rows > 4096) return kForms + 1;
     return kForms;
 }
 // the 256 x 256 tiles of gemm.hip, in the same unit: int8 W with fp32 X, bf16 W with bf16 X
@@ -398,7 +401,7 @@ long long mid_tiles(const MidForm& f, const MidArgs& ga) {
 // K groups walk too long (bf16 X 33 x 2048 x 4096 10.1 sized, 12.2 here; bf16 W, fp32 X 100 x 1536 x 6144 23.6, 27.4).
 int one_round_form(bool f32, const MidArgs& ga) {
     auto one_round = [&](int i) { return mid_tiles(kFormsSmall[i], ga) <= 256; };
-    if (one_round(0)) return kForms + (ga.K <= 1024 ? 1 : 0);
+    if (one_round(0)) return kForms + (ga.K <= kShortK ? 1 : 0);
     if ((f32 || ga.K < 1024) && one_round(2)) return kForms + 2;
     if (f32 && ga.K <= 1024 && one_round(3)) return kForms + 3;
     return -1;

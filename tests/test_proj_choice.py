@@ -28,9 +28,9 @@ def test_one_weight_is_a_stack_of_one():
 
 
 @pytest.mark.parametrize("x,N,M,K,code", [
-    (F32, (4096,), 16, 512, 9), (F32, (2048,), 32, 512, 9), (F32, (2048,), 32, 1040, 8), (F32, (2048,), 64, 512, 10),
+    (F32, (4096,), 16, 512, 9), (F32, (2048,), 32, 512, 9), (F32, (2048,), 32, 1280, 9), (F32, (2048,), 32, 1296, 8), (F32, (2048,), 64, 512, 10),
     (F32, (4096,), 64, 1024, 11), (F32, (4096,), 65, 1024, None), (F32, (4096,), 64, 1040, None),
-    (BF16, (1000,), 17, 1040, 8), (BF16, (2048,), 64, 512, 10), (BF16, (2048,), 64, 4096, None),
+    (BF16, (1000,), 17, 1040, 9), (BF16, (2048,), 64, 512, 10), (BF16, (2048,), 64, 4096, None),
     (BF16, (2000, 48), 32, 256, 9), (BF16, (2000, 49), 32, 256, 10),
     (F32, (5120,), 3, 1536, 10), (BF16, (5120,), 3, 1536, 9), (BF16, (4096,), 3, 1536, 8)])
 def test_tiles_of_16_rows_where_they_run_in_one_round(x, N, M, K, code):
