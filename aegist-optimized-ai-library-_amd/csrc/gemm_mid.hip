@@ -135,12 +135,13 @@ template <> struct MidX<uint16_t> {
 // batches add theirs up every kFlush steps. 2-norm error, one set and now: bf16 16 rows of 8192 x 2048 1.31e-7,
 // 0.98e-7, of 2048 x 4096 1.37e-7, 1.06e-7, 64 of 12352 x 2048 1.86e-7, 0.98e-7; int8 W, bf16 X, 600 rows of
 // 4096 x 8192 2.79e-7, 1.0e-7. It costs 0 to 6% at up to 64 rows, up to 14% at 300 of int8 12352 x 2048. (Past 64 rows
-// bf16 W is in the place of full-K chains. fp32 X: its split's 2^-17 is 40 times as much; one set.)
+// bf16 W is in the place of full-K chains, except in the form of 4 K groups on 32 rows, whose chains would be
+// longer than with the 8 before. fp32 X: its split's 2^-17 is 40 times as much; one set.)
 template <typename TW, typename TX, int RT, int MT, int KG, bool kShort>
 struct MidSums {
     static constexpr bool kBf16X = MidX<TX>::kParts == 1, kI8 = sizeof(TW) == 1;
     static constexpr int kFlush = kBf16X && kI8 && KG <= 2 ? 4 : 0;
-    static constexpr int kSets = !kBf16X || !kShort || kFlush || KG == 1 ? 1 : KG == 2 && RT * MT <= 4 ? 4 : 2;
+    static constexpr int kSets = !kBf16X || !kShort || kFlush || KG == 1 ? 1 : (KG == 2 && RT * MT <= 4) || (KG == 4 && MT == 2) ? 4 : 2;
 };
 
 template <typename TW, typename TX, int RT, int MT, int NWN, int KG, int PD, bool kShort>
@@ -359,8 +360,10 @@ struct MidForm {
 // fp32 X: staging and splitting X is the larger part of a step
 constexpr MidForm kFormsF32[] = {{1, 2, 1, 8, 0.156f}, {1, 2, 2, 8, 0.18f}, {2, 2, 2, 8, 0.265f}, {2, 2, 4, 4, 0.42f},
                                  {2, 2, 4, 1, 0.33f, 0.15f}, {2, 4, 4, 2, 0.70f}, {2, 4, 8, 1, 1.15f}, {4, 4, 8, 1, 1.80f}};
-constexpr MidForm kFormsBf16[] = {{1, 2, 1, 8, 0.100f}, {1, 2, 2, 8, 0.157f}, {1, 4, 2, 4, 0.205f}, {1, 4, 4, 2, 0.312f},
+constexpr MidForm kFormsBf16[] = {{1, 2, 1, 8, 0.100f}, {1, 2, 2, 4, 0.157f}, {1, 4, 2, 4, 0.205f}, {1, 4, 4, 2, 0.312f},
                                   {2, 4, 4, 2, 0.548f}, {2, 8, 4, 1, 0.90f},  {2, 8, 8, 1, 1.21f}};
+// (bf16 X, the second form: 8 K groups for int8 W. bf16 W is fuller with 4 of them, whose workgroups take half the
+// threads: 17 x 8192 x 2048 12.1 -> 10.8 us (row-tile kernel 11.4), 100 x 2048 x 2048 9.4 -> 9.0; int8 150 x 1024 x 8192 15.5 -> 18.0)
 constexpr int kNF32 = 8, kNBf16 = 7, kForms = 8;  // entries of the two tables; codes of the sized forms
 // 16 rows of X a tile, after the sized forms: up to 16 rows chosen by rows of W and K, see small_form; past
 // them where all tiles run in one round, see one_round_form
@@ -419,7 +422,7 @@ int launch_mid(MidArgs ga, hipStream_t st) {
     ga.ntiles = ga.tiles_m * t;
     ga.per_xcd = (ga.ntiles + 7) / 8;
     // (one instance where both would be the same)
-    constexpr bool both = MidSums<TW, TX, RT, MT, KG, true>::kSets > 1 && sizeof(TW) == 2 && MT > 1;
+    constexpr bool both = MidSums<TW, TX, RT, MT, KG, true>::kSets > 1 && sizeof(TW) == 2 && MT > 1 && !(KG == 4 && MT == 2);
     if (both && ga.M > 64)
         gemm_mid_kernel<TW, TX, RT, MT, NWN, KG, PD, !both><<<8 * ga.per_xcd, 64 * NWN * KG, 0, st>>>(ga);
     else
@@ -433,7 +436,8 @@ int run_mid(int form, const MidArgs& ga, hipStream_t st) {
 #define AEG_MID(I)                                                                                              \
     case I: {                                                                                                   \
         constexpr MidForm f = f32 ? kFormsF32[I] : kFormsBf16[I < kNBf16 ? I : 0];                              \
-        return launch_mid<TW, TX, f.rt, f.mt, f.nwn, f.kg, 2>(ga, st);                                          \
+        constexpr int kg = !f32 && I == 1 && sizeof(TW) == 1 ? 8 : f.kg;                                        \
+        return launch_mid<TW, TX, f.rt, f.mt, f.nwn, kg, 2>(ga, st);                                            \
     }
 #define AEG_MID_SMALL(I)                                                                                        \
     case kForms + I: return launch_mid<TW, TX, kFormsSmall[I].rt, 1, kFormsSmall[I].nwn, kFormsSmall[I].kg, 2>(ga, st);

@@ -46,7 +46,7 @@ def test_mid_batch_matches_exact(dev, M, N, K, w8, xf):
 @pytest.mark.parametrize("w8,xf", [(True, True), (False, False), (False, True), (True, False)])
 @pytest.mark.parametrize("M,N,K", [(17, 1, 16), (32, 2048, 512), (33, 1000, 1040), (47, 1365, 1552), (64, 2047, 976),
                                    (100, 2300, 272), (4096, 16, 1024), (4095, 17, 1040),   # 16 rows a tile, one round
-                                   (33, 5120, 1536), (130, 2100, 1040), (600, 4100, 1552)])  # sized, odd steps
+                                   (33, 5120, 1536), (24, 8190, 1552), (130, 2100, 1040), (600, 4100, 1552)])  # sized, odd steps
 def test_one_round_and_odd_steps(dev, M, N, K, w8, xf):
     print(f"round M={M} N={N} K={K} w8={w8} xf={xf}", flush=True)
     x, w, s = _operands(M, N, K, w8, xf, M + N + K, dev)
